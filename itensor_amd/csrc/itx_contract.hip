@@ -1075,82 +1075,110 @@ __global__ __launch_bounds__(64 * GM * GN) void k_gemm3(const double *__restrict
 }
 
 // Skinny contractions (N <= 32 and K <= 64 for every task, e.g. the
-// MPO-tensor stages of H*psi): HBM-bound, so one thread owns one row m of
-// a 256-row unit and accumulates its N outputs in registers (FP64 FMA)
-// while B (K x N) sits in LDS.  Same task/unit/table format as k_gemm.
+// MPO-tensor stages of H*psi): HBM-bound, on the FP64 matrix cores in every
+// form.  Same task/unit/table format as k_gemm.  A unit is 256 rows of one C
+// block; each of its four waves takes 64 rows as four 16 x 16 MFMA row
+// groups.  A lane loads the operands of its own fragment positions straight
+// from memory (16 rows x 4 k: with A contiguous along k in runs of 4, or
+// along m, a load instruction covers whole 128-byte lines) and the D^T tile
+// stores 16 consecutive m per column, the four row groups of a column back
+// to back.  No LDS and no barrier; 4 x SK_KS independent loads of A per lane
+// are in flight, three waves per SIMD.
+// ONE: every unit has one task with K <= 4 SK_KS, so the k offsets and B's
+// fragments are straight-line code (with the task and k loops around them
+// the registers allow two waves per SIMD: 104 against 84 us at chi = 1024).
+// K = N = 20 (the dense Heisenberg MPO pair), chi = 32, 255, 768, 1024: 6,
+// 7, 32 and 84 us; one thread per row with B in LDS, the form before this
+// one, was bound by its K x N LDS reads and column tests: 22, 26, 84 and
+// 115 us.  Stores past the caches make this kernel faster at chi = 1024
+// (54 us) and the next stage, which reads C back, slower by more (the chain
+// 1514 against 1495 us).
 constexpr int SK_ROWS = 256, SK_N = 32, SK_K = 64;
+constexpr int SK_KS = 5;  // k slots (of 4) loaded together: K = 20 in one chunk
+constexpr int SK_G = 4;   // 16-row groups of a wave
 
-// V4: every task's A is contiguous along k in runs of 4 starting at even
-// offsets (K a multiple of 4): a row's 8 k of a batch are two runs, read as
-// four 16-byte loads instead of eight 8-byte loads.
-template <bool V4>
-__global__ __launch_bounds__(SK_ROWS) void k_skinny(const double *__restrict__ A, const double *__restrict__ B,
-                                                    double *__restrict__ C, const GemmTask *__restrict__ tasks,
-                                                    const WorkUnit *__restrict__ units, int nunits,
-                                                    const int64_t *__restrict__ tab, double alpha, double beta) {
-  __shared__ double Bs[SK_K * SK_N];
-  const int tid = threadIdx.x;
+template <int NB, bool ONE>  // NB 16-column groups: 1 (N <= 16) or 2
+__global__ __launch_bounds__(SK_ROWS, 3) void k_skinny(const double *__restrict__ A, const double *__restrict__ B,
+                                                       double *__restrict__ C, const GemmTask *__restrict__ tasks,
+                                                       const WorkUnit *__restrict__ units, int nunits,
+                                                       const int64_t *__restrict__ tab, double alpha, double beta) {
+  using v4 = MF<double>::v4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r16 = lane & 15, q4 = lane >> 4;
   for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
     const WorkUnit wu = units[u];
-    const int m = wu.m0 + tid;
-    double acc[SK_N];
-#pragma unroll
-    for (int n = 0; n < SK_N; ++n) acc[n] = 0.0;
-    for (int t = wu.tbeg; t < wu.tend; ++t) {
-      const GemmTask tk = tasks[t];
-      const int N = tk.N, K = tk.K;
-      __syncthreads();  // the previous task's B tile is no longer read
-      for (int x = tid; x < K * N; x += SK_ROWS) {
-        const int k = x / N, n = x - k * N;
-        Bs[k * SK_N + n] = B[tk.b_off + tab[tk.tBK + k] + tab[tk.tBN + n]];
-      }
-      __syncthreads();
-      if (m < tk.M) {
-        const double *Ar = A + tk.a_off + tab[tk.tAM + m];
-        const int64_t *tAK = tab + tk.tAK;
-        for (int k0 = 0; k0 < K; k0 += 8) {
-          double av[8];  // issue 8 independent loads before using any
-          if constexpr (V4) {
-            const bool two = k0 + 4 < K;  // K % 4 == 0: one or two runs left
-            const double2 *r0 = reinterpret_cast<const double2 *>(Ar + tAK[k0]);
-            const double2 *r1 = reinterpret_cast<const double2 *>(Ar + tAK[two ? k0 + 4 : k0]);
-            const double2 x0 = r0[0], x1 = r0[1], x2 = r1[0], x3 = r1[1];
-            av[0] = x0.x;
-            av[1] = x0.y;
-            av[2] = x1.x;
-            av[3] = x1.y;
-            av[4] = two ? x2.x : 0.0;
-            av[5] = two ? x2.y : 0.0;
-            av[6] = two ? x3.x : 0.0;
-            av[7] = two ? x3.y : 0.0;
-          } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) av[j] = (k0 + j < K) ? Ar[tAK[k0 + j]] : 0.0;
-          }
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            if (k0 + j < K) {
-#pragma unroll
-              for (int n = 0; n < SK_N; ++n)
-                if (n < N) acc[n] += av[j] * Bs[(k0 + j) * SK_N + n];
-            }
-          }
-        }
-      }
-    }
     const GemmTask t0 = tasks[wu.tbeg];
-    if (m < t0.M) {
-      double *Cm = C + t0.c_off + tab[t0.tCM + m];
-      const int64_t *tCN = tab + t0.tCN;
+    const int mb = wu.m0 + 16 * SK_G * wave;
+    if (mb >= t0.M) continue;  // wave-uniform
+    int mr[SK_G];  // rows past the block repeat its last row and are not stored
 #pragma unroll
-      for (int n = 0; n < SK_N; ++n) {
-        if (n < t0.N) {
-          double v = alpha * acc[n];
-          if (beta != 0.0) v += beta * Cm[tCN[n]];
-          Cm[tCN[n]] = v;
+    for (int g = 0; g < SK_G; ++g) mr[g] = min(mb + 16 * g + r16, t0.M - 1);
+    v4 acc[NB][SK_G];
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int g = 0; g < SK_G; ++g) acc[i][g] = v4{0, 0, 0, 0};
+    // 4 SK_KS k of one task: loads from clamped positions, zeroed where k
+    // or the column is past the end, so no branch separates them
+    auto chunk = [&](const GemmTask &tk, int k0) {
+      double a[SK_KS][SK_G], b[SK_KS][NB];
+      int64_t ka[SK_KS];
+#pragma unroll
+      for (int s = 0; s < SK_KS; ++s) {
+        const int k = k0 + 4 * s + q4;
+        const bool kv = k < tk.K;
+        ka[s] = tab[tk.tAK + (kv ? k : 0)];
+        const int64_t kb = tab[tk.tBK + (kv ? k : 0)];
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+          const bool nv = 16 * i + r16 < tk.N;
+          const double x = B[tk.b_off + kb + tab[tk.tBN + (nv ? 16 * i + r16 : 0)]];
+          b[s][i] = (kv && nv) ? x : 0.0;
         }
       }
+#pragma unroll
+      for (int g = 0; g < SK_G; ++g) {
+        const double *Ar = A + tk.a_off + tab[tk.tAM + mr[g]];
+#pragma unroll
+        for (int s = 0; s < SK_KS; ++s) {
+          const double x = Ar[ka[s]];
+          a[s][g] = k0 + 4 * s + q4 < tk.K ? x : 0.0;
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < SK_KS; ++s)
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+          for (int g = 0; g < SK_G; ++g) acc[i][g] = MF<double>::mma(b[s][i], a[s][g], acc[i][g]);
+    };
+    if constexpr (ONE) {
+      if (t0.K > 0) chunk(t0, 0);
+    } else {
+      for (int t = wu.tbeg; t < wu.tend; ++t) {
+        const GemmTask tk = tasks[t];
+        for (int k0 = 0; k0 < tk.K; k0 += 4 * SK_KS) chunk(tk, k0);
+      }
     }
+    int64_t cm[SK_G];
+#pragma unroll
+    for (int g = 0; g < SK_G; ++g) cm[g] = t0.c_off + tab[t0.tCM + mr[g]];
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int n = 16 * i + MF<double>::orow(lane, r);
+        if (n >= t0.N) continue;
+        const int64_t cn = tab[t0.tCN + n];
+#pragma unroll
+        for (int g = 0; g < SK_G; ++g) {
+          if (mb + 16 * g + r16 >= t0.M) continue;
+          double *cp = C + cm[g] + cn;
+          double v = alpha * acc[i][g][r];
+          if (beta != 0.0) v += beta * (*cp);
+          *cp = v;
+        }
+      }
   }
 }
 
@@ -1806,7 +1834,7 @@ constexpr int kDgemm = 14, kDgemm2 = 15;
 constexpr int kSkinny = 5;
 static_assert(kSkinny == kSkinnyTile, "tile index of the skinny path");
 constexpr int kSmall = 10;
-constexpr int kSkinnyOcc = 4;
+constexpr int kSkinnyOcc = 3, kSkinnyQOcc = 4;
 
 // Kernel instantiation of a tile shape, operand layout and form.  All
 // kernels of the engine share one argument list (see KernelArgs).
@@ -1878,15 +1906,24 @@ const void *gemm_fn_tile(int tile, bool akc, bool bkc, bool vec) {
   }
 }
 
+// What the skinny path's variants depend on.
+struct Skinny {
+  int maxn = SK_N;    // largest N of the tasks
+  bool tiny = false;  // every task has K <= 8 and N <= 8
+  bool one = false;   // one task per C block, K <= 4 SK_KS
+};
+
 // Entry point and workgroup size of a plan's kernel.
 const void *kernel_of(int tile, int prec, bool akc, bool bkc, int *block, int vec = 0, bool split = false,
-                      bool tiny = false) {
+                      Skinny sk = Skinny{}) {
   if (tile == kSkinny) {  // HBM-bound: FP64 arithmetic in every form
     *block = SK_ROWS;
-    // tiny: every task has K <= 8 and N <= 8; vec bit 3: A in aligned k runs of 4
-    if (tiny) return reinterpret_cast<const void *>(&k_skinny_q);
-    return (vec & 8) ? reinterpret_cast<const void *>(&k_skinny<true>)
-                     : reinterpret_cast<const void *>(&k_skinny<false>);
+    if (sk.tiny) return reinterpret_cast<const void *>(&k_skinny_q);
+    if (sk.maxn <= 16)
+      return sk.one ? reinterpret_cast<const void *>(&k_skinny<1, true>)
+                    : reinterpret_cast<const void *>(&k_skinny<1, false>);
+    return sk.one ? reinterpret_cast<const void *>(&k_skinny<2, true>)
+                  : reinterpret_cast<const void *>(&k_skinny<2, false>);
   }
   if (tile == kSmall) {  // FP64 on the VALU, FP32 / BF16x3 on the matrix cores
     *block = SM_T;
@@ -2007,7 +2044,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     int64_t tAM, tCM, tBN, tCN, tAK, tBK;
     int64_t am, cm, bn, cn, ak, bk;
     bool akc, bkc, empty;
-    int vec;  // bit 0: k runs of 2 usable by both operands, bit 1: runs of 4 (bits 2, 3: below)
+    int vec;  // bit 0: k runs of 2 usable by both operands, bit 1: runs of 4 (bit 2: below)
   };
   std::vector<DimInfo> infos;
   std::vector<int64_t> ikeys;  // the dims of each entry (rA + rB per entry)
@@ -2106,9 +2143,6 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
         if (c[i].s1 % al) return false;
       return true;
     };
-    // bit 3: A alone in runs of 4 at even offsets (the skinny path reads
-    // only A from memory)
-    if (fi.akc && aligned(dm, true, 2) && runs(dk, true, K, 4, 2)) fi.vec |= 8;
     if (fi.akc && fi.bkc) {
       if (aligned(dm, true, 2) && aligned(dn, true, 2)) {
         if (runs(dk, true, K, 2, 2) && runs(dk, false, K, 2, 2)) fi.vec |= 1;
@@ -2119,7 +2153,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     }
     return ITX_OK;
   };
-  int vecbits = 15;  // AND over the tasks
+  int vecbits = 7;  // AND over the tasks
   for (int t = 0; t < ntasks; ++t) {
     const int64_t *dA = blkA + size_t(t) * rA;
     const int64_t *dB = blkB + size_t(t) * rB;
@@ -2159,8 +2193,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
       bkc = fi.bkc;
     }
     vecbits &= fi.vec;
-    if (offs[3 * size_t(t)] % 2) vecbits = 0;
-    if (offs[3 * size_t(t) + 1] % 2) vecbits &= 8;
+    if (offs[3 * size_t(t)] % 2 || offs[3 * size_t(t) + 1] % 2) vecbits = 0;
     if (offs[3 * size_t(t)] % 4 || offs[3 * size_t(t) + 1] % 4) vecbits &= ~4;
     GemmTask g{};
     g.a_off = offs[3 * size_t(t)];
@@ -2345,11 +2378,12 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     p->ntasks = int(vt.size());
     p->nunits = int(units.size());
     p->flops = flops;
-    p->grid = int(std::min<int64_t>(int64_t(units.size()), int64_t(cus) * tile_occupancy(best, prec, akc, bkc)));
-    p->vec = (akc && bkc) ? vecbits : akc ? (vecbits & 8) : 0;
-    const bool tiny = best == kSkinny && tinyq;
-    p->fn = kernel_of(best, prec, akc, bkc, &p->block, p->vec, false, tiny);
-    p->fn_scalar = kernel_of(best, prec, akc, bkc, &p->block, 0, false, tiny);
+    const int occ = best == kSkinny && tinyq ? kSkinnyQOcc : tile_occupancy(best, prec, akc, bkc);
+    p->grid = int(std::min<int64_t>(int64_t(units.size()), int64_t(cus) * occ));
+    p->vec = (akc && bkc) ? vecbits : 0;
+    const Skinny sk{maxN, tinyq, st.size() == groups.size() && maxK <= 4 * SK_KS};
+    p->fn = kernel_of(best, prec, akc, bkc, &p->block, p->vec, false, sk);
+    p->fn_scalar = kernel_of(best, prec, akc, bkc, &p->block, 0, false, sk);
     p->nred = int(red.size());
     if (p->nred) {
       p->fn_red = reinterpret_cast<const void *>(&k_reduce_tiles);
