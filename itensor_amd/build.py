@@ -24,7 +24,9 @@ CSRC = os.path.join(PKG, "csrc")
 HOST = os.path.join(PKG, "host")
 INCLUDE = os.path.join(ROOT, "include")
 
-HIP_SOURCES = ["itx_runtime.hip", "itx_contract.hip", "itx_vec.hip", "itx_eig.hip", "itx_svd.hip"]
+HIP_SOURCES = ["itx_runtime.hip", "itx_contract.hip", "itx_vec.hip", "itx_eig.hip", "itx_tridiag.hip", "itx_dc.hip", "itx_svd.hip"]
+EIG_HEADERS = [os.path.join(CSRC, "itx_eig.h"), os.path.join(CSRC, "itx_tri.h")]
+EIG_SOURCES = ("itx_eig.hip", "itx_tridiag.hip", "itx_dc.hip")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # Packed FP32 instructions are disabled for all device code (they have
 # produced wrong results on this hardware); -O3 for the kernels.
@@ -67,7 +69,7 @@ def build_libitx(force: bool = True) -> str:
     os.makedirs(LIBDIR, exist_ok=True)
     out = os.path.join(LIBDIR, "libitx.so")
     srcs = [os.path.join(CSRC, s) for s in HIP_SOURCES]
-    deps = srcs + [os.path.join(CSRC, "itx_internal.h"), os.path.join(INCLUDE, "itx.h")]
+    deps = srcs + [os.path.join(CSRC, "itx_internal.h"), *EIG_HEADERS, os.path.join(INCLUDE, "itx.h")]
     if not force and _newer(out, deps):
         return out
     # one object per source, compiled side by side, then one link
@@ -75,8 +77,12 @@ def build_libitx(force: bool = True) -> str:
     os.makedirs(objdir, exist_ok=True)
     objs = [os.path.join(objdir, os.path.basename(s) + ".o") for s in srcs]
     cflags = [f for f in HIP_FLAGS if f != "-shared"]
-    hdrs = deps[len(srcs):]
-    todo = [(s, o) for s, o in zip(srcs, objs) if force or not _newer(o, [s, *hdrs])]
+    hdrs = [os.path.join(CSRC, "itx_internal.h"), os.path.join(INCLUDE, "itx.h")]
+
+    def reads(s):  # the headers a source includes
+        return [s, *hdrs, *(EIG_HEADERS if os.path.basename(s) in EIG_SOURCES else [])]
+
+    todo = [(s, o) for s, o in zip(srcs, objs) if force or not _newer(o, reads(s))]
     with ThreadPoolExecutor(max_workers=min(len(todo), _jobs()) or 1) as ex:
         for f in [ex.submit(_run, [HIPCC, *cflags, "-c", s, "-o", o]) for s, o in todo]:
             f.result()

@@ -1,27 +1,27 @@
-// FP64 symmetric eigensolver of libitx (one workgroup per matrix).
+// FP64 symmetric eigensolver of libitx.
 //
 // Replaces dsyev('V','U') as called by diagHermitian on -M
 // (tensor/algs_impl.h:91-139, tensor/algs.cc:34-41): eigenvalues come out
 // in descending order with orthonormal eigenvectors as columns.
 //
-// Method (textbook, not LAPACK's code): Householder reduction to
-// tridiagonal form T = Q^T A Q with explicit accumulation of Q, then the
-// implicit QL iteration with Wilkinson-type shift on T (Bowdler, Martin,
-// Reinsch & Wilkinson, Numer. Math. 11 (1968) 293, "tql2"), whose plane
-// rotations are applied to Q.  The work is split the way hybrid symmetric
-// eigensolvers split it: the O(n^3) parts on the device (reduction and Q:
-// one workgroup per matrix with the matrix resident in LDS up to 128, one
-// 16-wave workgroup per matrix over global memory up to 512, one
-// cooperative launch over the whole device per larger matrix; the
-// rotations applied to Q's rows in parallel in a second launch),
-// the O(n^2) scalar QL recurrence -- a chain of dependent flops that one
-// host core runs far faster than one GPU lane -- on the host in between.
+// Matrices up to 512 rows, all of a call together: Householder reduction to
+// tridiagonal form (itx_tridiag.hip), divide and conquer on it (itx_dc.hip),
+// and the eigenvectors taken back through the reflectors, all on the device;
+// the host waits once, for the eigenvalues, while the last products run.
+// Larger ones go to rocSOLVER.  With ITX_EIG_OWN=1 those up to 2048 rows run
+// on this file's kernels instead: the same reduction over global memory with
+// Q accumulated, then the implicit QL iteration with Wilkinson-type shift
+// (Bowdler, Martin, Reinsch & Wilkinson, Numer. Math. 11 (1968) 293,
+// "tql2") on the host, whose plane rotations are applied to Q's rows on the
+// device.  The same path takes a matrix whose workgroups did not meet
+// during the reduction (see itx_tridiag.hip).
 #include <cfloat>
 #include <cmath>
 #include <cstdlib>
 #include <algorithm>
 #include <cstring>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <functional>
 #include <mutex>
@@ -33,7 +33,7 @@
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>
 
-#include "itx_internal.h"
+#include "itx_eig.h"
 
 namespace itx {
 namespace {
@@ -61,11 +61,10 @@ __device__ __forceinline__ double bsum(double v, double *red) {
   return s;
 }
 
-// Reduction and Q for n > 128: A in global memory (overwritten by the
-// reflectors), W as scratch for p, Q into the workspace.
-// One workgroup per matrix over global memory (n > 128): used when a batch
-// holds several such matrices that are cheaper side by side than one after
-// the other through the cooperative kernel.
+// Reduction and Q: A in global memory (overwritten by the reflectors), W as
+// scratch for p, Q into the workspace.  One workgroup per matrix: used when a
+// batch holds several matrices that are cheaper side by side than one after
+// the other through the cooperative kernel, and up to 512 rows.
 __global__ __launch_bounds__(ET) void k_syev(const EigTask *__restrict__ tasks, double *__restrict__ Abase,
                                              double *__restrict__ Wbase, double *__restrict__ Zbase) {
   __shared__ double d[EMAX], e[EMAX], tau_[EMAX];
@@ -166,250 +165,7 @@ __global__ __launch_bounds__(ET) void k_syev(const EigTask *__restrict__ tasks, 
   }
 }
 
-// ---- one workgroup of 16 waves per matrix, 128 < n <= 64 RA -------------
-// The matrix stays in global memory (it fits the L2); the reduction makes
-// one pass over the trailing block per Householder step.  Step k: wave 0
-// brings column k up to date with the pending rank-2 update of step k-1
-// (v', w'), forms the reflector (v, tau) from it and stores v in the
-// column; then every thread walks its part of the trailing block
-// [k+1, n)^2 -- rows lane + 64 a, columns = wave (mod 16) -- applying the
-// pending update, storing the element (column k+1 also to LDS, where wave 0
-// reads it for the next reflector) and accumulating p = S v with the
-// updated value; the 16 partial sums of each row go through LDS, and wave 0
-// forms K = tau/2 v.p and w = p - K v, the next pending update.  Each
-// element is read and written once per step and every thread has up to
-// RA x (its columns) independent loads in flight.  Q is accumulated
-// backwards with the same column ownership: a wave owns whole columns of
-// Q, so the reflections need no barrier between waves.
-constexpr int MT = 1024, MW = MT / 64;
-
-__device__ __forceinline__ double wsum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
-template <int RA, int UP, int UQ, int QG>
-__global__ __launch_bounds__(MT) void k_syev_mid(const EigTask *__restrict__ tasks, double *__restrict__ Abase,
-                                                 double *__restrict__ Zbase) {
-  constexpr int NM = 64 * RA;
-  __shared__ double ppart[MW][NM];
-  __shared__ double sv[NM], svp[NM], swp[NM];
-  __shared__ double scol[NM];  // column k+1 as the pass of step k stored it
-  __shared__ double sd[NM], se[NM], stau[NM];
-
-  const EigTask tk = tasks[blockIdx.x];
-  const int n = tk.n;
-  if (n <= 0 || n > NM) return;
-  double *__restrict__ A = Abase + tk.a_off;
-  double *__restrict__ Z = Zbase + tk.z_off;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int i = tid; i < NM; i += MT) {
-    svp[i] = 0.0;
-    swp[i] = 0.0;
-  }
-  __syncthreads();
-
-  for (int k = 0; k + 2 < n; ++k) {
-    if (wave == 0) {
-      // column k with the pending update; rows i = k + lane + 64 q
-      const double wpk = swp[k], vpk = svp[k];
-      double c[RA];
-      double sig = 0.0;
-#pragma unroll
-      for (int q = 0; q < RA; ++q) {
-        const int i = k + lane + 64 * q;
-        const double a0 = (i < n) ? (k == 0 ? A[size_t(k) * n + i] : scol[i]) : 0.0;
-        c[q] = (i < n) ? a0 - (svp[i] * wpk + swp[i] * vpk) : 0.0;
-        if (i > k + 1 && i < n) sig += c[q] * c[q];
-      }
-      sig = wsum(sig);
-      const double dk = __shfl(c[0], 0, 64), x0 = __shfl(c[0], 1, 64);
-      double tau = 0.0, alpha = x0, v0 = x0;
-      if (sig > 0.0) {
-        const double mu = sqrt(x0 * x0 + sig);
-        v0 = (x0 <= 0) ? x0 - mu : x0 + mu;
-        alpha = (x0 <= 0) ? mu : -mu;
-        tau = 2.0 / (v0 * v0 + sig);
-      }
-#pragma unroll
-      for (int q = 0; q < RA; ++q) {
-        const int i = k + lane + 64 * q;
-        if (i > k && i < n) {
-          const double vi = (tau == 0.0) ? 0.0 : ((i == k + 1) ? v0 : c[q]);
-          sv[i] = vi;
-          A[size_t(k) * n + i] = vi;
-        }
-      }
-      if (lane == 0) {
-        sd[k] = dk;
-        se[k] = alpha;
-        stau[k] = tau;
-      }
-    }
-    __syncthreads();
-    const double tau = stau[k];
-    const int r0 = k + 1;
-    double pacc[RA], vpi[RA], wpi[RA];
-#pragma unroll
-    for (int a = 0; a < RA; ++a) {
-      const int i = r0 + lane + 64 * a;
-      pacc[a] = 0.0;
-      vpi[a] = (i < n) ? svp[i] : 0.0;
-      wpi[a] = (i < n) ? swp[i] : 0.0;
-    }
-    // groups of UP columns: every load of a group is issued before its
-    // stores, so that a thread keeps UP x RA loads in flight
-    for (int j0 = r0 + wave; j0 < n; j0 += MW * UP) {
-      double x[UP][RA];
-#pragma unroll
-      for (int u = 0; u < UP; ++u) {
-        const int j = j0 + MW * u;
-#pragma unroll
-        for (int a = 0; a < RA; ++a) {
-          const int i = r0 + lane + 64 * a;
-          x[u][a] = (j < n && i < n) ? A[size_t(j) * n + i] : 0.0;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < UP; ++u) {
-        const int j = j0 + MW * u;
-        if (j < n) {
-          const double vj = sv[j], vpj = svp[j], wpj = swp[j];
-#pragma unroll
-          for (int a = 0; a < RA; ++a) {
-            const int i = r0 + lane + 64 * a;
-            if (i < n) {
-              const double y = x[u][a] - (vpi[a] * wpj + wpi[a] * vpj);
-              A[size_t(j) * n + i] = y;
-              if (j == r0) scol[i] = y;  // the next step's column, without a round trip
-              pacc[a] += y * vj;
-            }
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int a = 0; a < RA; ++a) {
-      const int i = r0 + lane + 64 * a;
-      if (i < n) ppart[wave][i] = pacc[a];
-    }
-    __syncthreads();
-    // wave 0 alone sums the partials into p, forms K and the next pending
-    // update and goes on to the next step's column: everything it reads
-    // there it wrote itself, so the step needs no further barrier (the
-    // other waves read svp / swp / sv only after the next barrier)
-    if (wave == 0) {
-      double pv[RA];
-      double sm = 0.0;
-#pragma unroll
-      for (int q = 0; q < RA; ++q) {
-        const int i = r0 + lane + 64 * q;
-        double ps = 0.0;
-        if (i < n) {
-#pragma unroll
-          for (int w = 0; w < MW; ++w) ps += ppart[w][i];
-        }
-        pv[q] = tau * ps;
-        if (i < n) sm += sv[i] * pv[q];
-      }
-      const double K = 0.5 * tau * wsum(sm);
-#pragma unroll
-      for (int q = 0; q < RA; ++q) {
-        const int i = r0 + lane + 64 * q;
-        if (i < n) {
-          swp[i] = pv[q] - K * sv[i];
-          svp[i] = sv[i];
-        }
-      }
-    }
-  }
-  // the last 2 x 2 block with the pending update
-  if (tid == 0) {
-    if (n == 1) {
-      sd[0] = A[0];
-      se[0] = 0.0;
-    } else {
-      const int k = n - 2;
-      auto upd = [&](int i, int j) { return A[size_t(j) * n + i] - (svp[i] * swp[j] + swp[i] * svp[j]); };
-      sd[k] = upd(k, k);
-      se[k] = upd(k + 1, k);
-      sd[k + 1] = upd(k + 1, k + 1);
-      se[k + 1] = 0.0;
-    }
-  }
-  for (size_t x = tid; x < size_t(n) * n; x += MT) Z[x] = ((x / n) == (x % n)) ? 1.0 : 0.0;
-  __syncthreads();
-
-  // Q = H_0 ... H_{n-3}, backwards; wave w owns the columns c = w (mod 16).
-  // QG reflectors per pass: a column is loaded once, H_kh, ..., H_kl are
-  // applied to it in registers (each reflector masked to its rows >= k+1,
-  // so a column it does not reach gets an exact zero dot), stored once.
-  for (int kh = n - 3; kh >= 0; kh -= QG) {
-    const int kl = max(kh - QG + 1, 0);
-    const int r0 = kl + 1;
-    double vg[QG][RA], tg[QG];
-#pragma unroll
-    for (int g = 0; g < QG; ++g) {
-      const int k = kh - g;
-      tg[g] = (k >= kl) ? stau[k] : 0.0;
-#pragma unroll
-      for (int a = 0; a < RA; ++a) {
-        const int i = r0 + lane + 64 * a;
-        vg[g][a] = (k >= kl && i < n && i > k) ? A[size_t(k) * n + i] : 0.0;
-      }
-    }
-    const int cstart = r0 + (((wave - r0) % MW) + MW) % MW;
-    for (int c0 = cstart; c0 < n; c0 += MW * UQ) {
-      double z[UQ][RA];
-#pragma unroll
-      for (int u = 0; u < UQ; ++u) {
-        const int c = c0 + MW * u;
-#pragma unroll
-        for (int a = 0; a < RA; ++a) {
-          const int i = r0 + lane + 64 * a;
-          z[u][a] = (c < n && i < n) ? Z[size_t(c) * n + i] : 0.0;
-        }
-      }
-#pragma unroll
-      for (int g = 0; g < QG; ++g) {
-        if (tg[g] == 0.0) continue;  // uniform
-        double sm[UQ];
-#pragma unroll
-        for (int u = 0; u < UQ; ++u) {
-          sm[u] = 0.0;
-#pragma unroll
-          for (int a = 0; a < RA; ++a) sm[u] += vg[g][a] * z[u][a];
-        }
-#pragma unroll
-        for (int u = 0; u < UQ; ++u) {
-          const double f = tg[g] * wsum(sm[u]);
-#pragma unroll
-          for (int a = 0; a < RA; ++a) z[u][a] -= f * vg[g][a];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < UQ; ++u) {
-        const int c = c0 + MW * u;
-        if (c < n) {
-#pragma unroll
-          for (int a = 0; a < RA; ++a) {
-            const int i = r0 + lane + 64 * a;
-            if (i < n) Z[size_t(c) * n + i] = z[u][a];
-          }
-        }
-      }
-    }
-  }
-  // (d, e) to the host, which runs the QL recurrence
-  double *DE = Zbase + tk.de_off;
-  for (int i = tid; i < n; i += MT) {
-    DE[i] = sd[i];
-    DE[n + i] = se[i];
-  }
-}
-
-// ---- multi-workgroup reduction for n > 128 (cooperative launch) ---------
+// ---- multi-workgroup reduction (cooperative launch) ------------ ---------
 // The same Householder reduction and backward accumulation of Q, spread
 // over the whole device: the trailing block is cut into 64 x 64 tiles that
 // the workgroups walk (persistent loop), and grid-wide barriers separate
@@ -596,234 +352,6 @@ __global__ __launch_bounds__(CT) void k_syev_coop(double *__restrict__ A, int n,
   }
 }
 
-// ---- LDS-resident reduction for n <= NMAX (<= 128) -------------------
-// The matrix lives in LDS: Householder reduction, then Q formed in place
-// from the stored reflectors (backward accumulation, the row and column of
-// each new trailing index reset to the unit vector), written out with
-// (d, e) for the host.
-constexpr int ES = 512;
-
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
-// Householder reduction of the symmetric n x n matrix S (element (r, c) at
-// S[c * LD + r], LDS or global memory) to tridiagonal form (d, e), then Q
-// formed in place in S.  ES threads; PL = rows per lane (n <= 64 PL).
-template <int PL>
-__device__ __forceinline__ void reduce_form_q(double *__restrict__ S, int LD, int n, double *d, double *e,
-                                              double *tau, double *pv, double *part) {
-  constexpr int NMAX = 64 * PL;
-  const int tid = threadIdx.x;
-  // ---- 1. Householder tridiagonalisation ----
-  // Every wave computes the reflector redundantly (lanes over rows, shuffle
-  // sums), the product p = tau S v is split over the four waves by column
-  // residue mod 4, and the rank-2 update runs waves over columns, lanes
-  // over rows: three barriers per step.
-  constexpr int NW = ES / 64;
-  const int lane = tid & 63, wv = tid >> 6;
-  for (int k = 0; k + 2 < n; ++k) {
-    const int L = n - k - 1;
-    double *col = S + k * LD + (k + 1);  // x = S(k+1:, k)
-    double xr[PL];
-    double sg = 0;
-#pragma unroll
-    for (int u = 0; u < PL; ++u) {
-      const int i = lane + 64 * u;
-      xr[u] = i < L ? col[i] : 0.0;
-      if (i >= 1) sg += xr[u] * xr[u];
-    }
-    const double sigma = wave_sum(sg);
-    const double x0 = __shfl(xr[0], 0, 64);
-    double t = 0, alpha = x0, v0 = x0;
-    if (sigma > 0) {
-      const double mu = sqrt(x0 * x0 + sigma);
-      v0 = (x0 <= 0) ? x0 - mu : x0 + mu;
-      alpha = (x0 <= 0) ? mu : -mu;
-      t = 2.0 / (v0 * v0 + sigma);
-    }
-    if (lane == 0) xr[0] = v0;  // this lane's copy of v
-    if (t == 0) {
-      if (tid == 0) {
-        e[k] = alpha;
-        tau[k] = 0;
-      }
-      continue;  // S unchanged; nothing to order
-    }
-    // partial products over columns j = wv mod NW
-    double acc[PL];
-#pragma unroll
-    for (int u = 0; u < PL; ++u) acc[u] = 0;
-    for (int j = wv; j < L; j += NW) {
-      const double vj = (j == 0) ? v0 : col[j];
-      const double *Sj = S + (k + 1 + j) * LD + (k + 1);
-#pragma unroll
-      for (int u = 0; u < PL; ++u) {
-        const int i = lane + 64 * u;
-        if (i < L) acc[u] += Sj[i] * vj;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < PL; ++u) {
-      const int i = lane + 64 * u;
-      if (i < L) part[wv * NMAX + i] = acc[u];
-    }
-    __syncthreads();
-    double pr[PL], dv = 0;
-#pragma unroll
-    for (int u = 0; u < PL; ++u) {
-      const int i = lane + 64 * u;
-      double pi = 0;
-      if (i < L) {
-#pragma unroll
-        for (int q = 0; q < NW; ++q) pi += part[q * NMAX + i];
-      }
-      pr[u] = t * pi;
-      dv += xr[u] * pr[u];
-    }
-    const double Kc = 0.5 * t * wave_sum(dv);
-#pragma unroll
-    for (int u = 0; u < PL; ++u) pr[u] -= Kc * xr[u];  // w = p - K v
-    if (wv == 0) {
-#pragma unroll
-      for (int u = 0; u < PL; ++u) {
-        const int i = lane + 64 * u;
-        if (i < L) pv[i] = pr[u];
-      }
-      if (lane == 0) {
-        col[0] = v0;  // col now holds v
-        e[k] = alpha;
-        tau[k] = t;
-      }
-    }
-    __syncthreads();
-    // S -= v w^T + w v^T
-    for (int j = wv; j < L; j += NW) {
-      const double vj = col[j], wj = pv[j];
-      double *Sj = S + (k + 1 + j) * LD + (k + 1);
-#pragma unroll
-      for (int u = 0; u < PL; ++u) {
-        const int i = lane + 64 * u;
-        if (i < L) Sj[i] -= xr[u] * wj + pr[u] * vj;
-      }
-    }
-    __syncthreads();
-  }
-  for (int i = tid; i < n; i += ES) d[i] = S[i * LD + i];
-  if (tid == 0) {
-    if (n >= 2) e[n - 2] = S[(n - 2) * LD + (n - 1)];
-    e[n - 1] = 0;
-    S[(n - 1) * LD + (n - 1)] = 1.0;
-  }
-  __syncthreads();
-
-  // ---- 2. Q = H_0 ... H_{n-3} in place (trailing block grows backwards) ----
-  // s_c = tau v^T Z(:, c) split over the waves by row residue mod 4 (lanes
-  // over columns), then Z -= v s^T with waves over columns, lanes over rows.
-  for (int k = n - 3; k >= 0; --k) {
-    const int j0 = k + 1;
-    for (int i = j0 + tid; i < n; i += ES) {
-      S[j0 * LD + i] = (i == j0) ? 1.0 : 0.0;  // column j0 (held v_{k+1})
-      S[i * LD + j0] = (i == j0) ? 1.0 : 0.0;  // row j0
-    }
-    __syncthreads();
-    const double t = tau[k];
-    if (t == 0) continue;  // block-uniform; the next step's reset is ordered by its own barrier
-    const double *v = S + k * LD + j0;  // v_k, first entry at row j0
-    const int L = n - j0;
-    double acc[PL];
-#pragma unroll
-    for (int u = 0; u < PL; ++u) acc[u] = 0;
-    for (int i = wv; i < L; i += NW) {
-      const double vi = v[i];
-#pragma unroll
-      for (int u = 0; u < PL; ++u) {
-        const int c = lane + 64 * u;
-        if (c < L) acc[u] += vi * S[(j0 + c) * LD + j0 + i];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < PL; ++u) {
-      const int c = lane + 64 * u;
-      if (c < L) part[wv * NMAX + c] = acc[u];
-    }
-    __syncthreads();
-    double vr[PL];
-#pragma unroll
-    for (int u = 0; u < PL; ++u) {
-      const int i = lane + 64 * u;
-      vr[u] = i < L ? v[i] : 0.0;
-    }
-    for (int c = wv; c < L; c += NW) {
-      double sc = 0;
-#pragma unroll
-      for (int q = 0; q < NW; ++q) sc += part[q * NMAX + c];
-      sc *= t;
-      double *Tc = S + (j0 + c) * LD + j0;
-#pragma unroll
-      for (int u = 0; u < PL; ++u) {
-        const int i = lane + 64 * u;
-        if (i < L) Tc[i] -= sc * vr[u];
-      }
-    }
-    __syncthreads();
-  }
-  for (int i = tid; i < n; i += ES) {
-    S[i] = (i == 0) ? 1.0 : 0.0;       // column 0
-    S[i * LD] = (i == 0) ? 1.0 : 0.0;  // row 0
-  }
-  __syncthreads();
-
-}
-
-template <int NMAX>
-__global__ __launch_bounds__(ES) void k_syev_lds(const EigTask *__restrict__ tasks, const double *__restrict__ Abase,
-                                                 double *__restrict__ Zbase) {
-  constexpr int LD = NMAX + 1;
-  __shared__ double S[NMAX * LD];
-  __shared__ double d[NMAX], e[NMAX], tau[NMAX], pv[NMAX];
-  __shared__ double part[(ES / 64) * NMAX];
-
-  const EigTask tk = tasks[blockIdx.x];
-  const int n = tk.n;
-  const int tid = threadIdx.x;
-  const double *__restrict__ A = Abase + tk.a_off;
-  if (n <= 0 || n > NMAX) return;  // the host sorts matrices into size classes
-  // staged through registers, eight loads in flight per thread
-  for (int x0 = 0; x0 < n * n; x0 += 8 * ES) {
-    double v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int x = x0 + u * ES + tid;
-      v[u] = x < n * n ? A[x] : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int x = x0 + u * ES + tid;
-      if (x < n * n) {
-        const int c = x / n, r = x - c * n;
-        S[c * LD + r] = v[u];
-      }
-    }
-  }
-  __syncthreads();
-  reduce_form_q<NMAX / 64>(S, LD, n, d, e, tau, pv, part);
-
-  // ---- 3. Q (column-major) and (d, e) out; the host runs the QL recurrence ----
-  double *Z = Zbase + tk.z_off;
-  for (int x = tid; x < n * n; x += ES) {
-    const int c = x / n, r = x - c * n;
-    Z[x] = S[c * LD + r];
-  }
-  double *DE = Zbase + tk.de_off;
-  for (int i = tid; i < n; i += ES) {
-    DE[i] = d[i];
-    DE[n + i] = e[i];
-  }
-}
-
 // ---- hybrid form: rotations recorded by the host, applied here ------------
 // Every QL sweep is a chain of rotations on consecutive index pairs
 // (i, i+1), i = top, top-1, ..., top-cnt+1.  The host sends one stream of
@@ -846,15 +374,9 @@ constexpr int RB = 1024;  // rotations staged in LDS per batch
 // stores position i+1, which the chain does not touch again.  A sweep runs
 // as chunks of 16 rotations, its remainder as chunks of 8, 4, 2 and 1, so
 // no chunk reaches past the sweep and none needs a mask.
-template <int LDC>  // LDC > 0: Q rows in LDS with that leading dimension (32-bit offsets)
 __device__ __forceinline__ void apply_stream(double *zc, int ld, int n, const RotMeta &mt,
                                              const double2 *__restrict__ R, double2 *Rs) {
-  auto at = [&](int p) -> double & {
-    if constexpr (LDC > 0)
-      return zc[p * LDC];
-    else
-      return zc[size_t(p) * ld];
-  };
+  auto at = [&](int p) -> double & { return zc[size_t(p) * ld]; };
   int segrem = 0, i = 0;
   double carry = 0;
   for (int b0 = 0; b0 < mt.nrot; b0 += RB) {
@@ -880,10 +402,7 @@ __device__ __forceinline__ void apply_stream(double *zc, int ld, int n, const Ro
       double2 g[C];
 #pragma unroll
       for (int t = 0; t < C; ++t) {
-        if constexpr (LDC > 0)
-          z[t] = zb[(C - 1 - t) * LDC];
-        else
-          z[t] = zb[size_t(C - 1 - t) * ld];
+        z[t] = zb[size_t(C - 1 - t) * ld];
         g[t] = Rs[q + t];
       }
 #pragma unroll
@@ -891,10 +410,7 @@ __device__ __forceinline__ void apply_stream(double *zc, int ld, int n, const Ro
         const double cz = g[t].x * z[t];
         const double up = fma(g[t].y, z[t], g[t].x * carry);
         carry = fma(-g[t].y, carry, cz);
-        if constexpr (LDC > 0)
-          zb[(C - t) * LDC] = up;  // position i - t + 1
-        else
-          zb[size_t(C - t) * ld] = up;
+        zb[size_t(C - t) * ld] = up;  // position i - t + 1
       }
       q += C;
       segrem -= C;
@@ -927,14 +443,11 @@ __device__ __forceinline__ void apply_stream(double *zc, int ld, int n, const Ro
 
 // Q <- Q G_1 G_2 ..., then this block's rows of the sorted eigenvectors
 // (column rank[c] of A is column c of Q) and, from the first block of a
-// matrix, the sorted eigenvalues.  LC > 0: the block's 64 rows of Q are
-// staged in LDS (n <= LC); LC == 0: they are updated in the workspace.
-template <int LC>
+// matrix, the sorted eigenvalues.  The rows are updated in the workspace.
 __global__ __launch_bounds__(AT) void k_syev_apply(const RotMeta *__restrict__ meta,
                                                    const double2 *__restrict__ rots, const double *__restrict__ evr, double *__restrict__ Abase,
                                                    double *__restrict__ Wbase, double *__restrict__ Zbase) {
   __shared__ double2 Rs[RB + AK];
-  __shared__ double Zs[LC > 0 ? (LC + 1) * AT : 1];
   const RotMeta mt = meta[blockIdx.x];
   const int n = mt.n;
   const int r0 = blockIdx.y * AT;
@@ -942,26 +455,9 @@ __global__ __launch_bounds__(AT) void k_syev_apply(const RotMeta *__restrict__ m
   const int lane = threadIdx.x;
   const int r = min(r0 + lane, n - 1);  // lanes past the last row redo row n-1 (same values)
   const bool act = r0 + lane < n;
-  const double *Zg = Zbase + mt.z_off + r;
   const double2 *R = rots + mt.rot_off;
-  double *zc;
-  int ld;
-  if constexpr (LC > 0) {
-    zc = Zs + lane;
-    ld = AT;
-    for (int c0 = 0; c0 < n; c0 += 16) {  // sixteen loads in flight
-      double v[16];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) v[u] = c0 + u < n ? Zg[size_t(c0 + u) * n] : 0.0;
-#pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (c0 + u < n) zc[(c0 + u) * AT] = v[u];
-    }
-  } else {
-    zc = Zbase + mt.z_off + r;
-    ld = n;
-  }
-  apply_stream<(LC > 0 ? AT : 0)>(zc, ld, n, mt, R, Rs);
+  double *zc = Zbase + mt.z_off + r;
+  apply_stream(zc, n, n, mt, R, Rs);
   // ranks to LDS (the rotation buffer is free now), then the sorted output
   const double *ev = evr + mt.ev_off, *rk = ev + n;
   int *rks = reinterpret_cast<int *>(Rs);
@@ -974,7 +470,7 @@ __global__ __launch_bounds__(AT) void k_syev_apply(const RotMeta *__restrict__ m
   __syncthreads();
   if (!act) return;
   double *__restrict__ A = Abase + mt.a_off + r;
-  for (int c = 0; c < n; ++c) A[size_t(rks[c]) * n] = zc[size_t(c) * ld];
+  for (int c = 0; c < n; ++c) A[size_t(rks[c]) * n] = zc[size_t(c) * n];
 }
 
 // sqrt(a^2 + b^2) without overflow or underflow of the squares
@@ -1111,20 +607,15 @@ class HostPool {
 
 }  // namespace
 
-// Our kernels for every matrix of the call (n <= EMAX).  `between` runs once
-// the tridiagonal forms are on the host, before the QL recurrences: work it
-// enqueues runs on the device while the host iterates.
+// This file's kernels for every matrix of the call (n <= EMAX): the kernels
+// reduce every matrix to tridiagonal form and build Q; the host runs the QL
+// recurrences; k_syev_apply applies the recorded rotations and writes the
+// sorted eigenpairs.
 int syev_own(itx_ctx *ctx, int nmat, const int32_t *ns, const int64_t *aoffs, double *Abase, const int64_t *woffs,
-             double *Wbase, double *whost, const std::function<int()> &between) {
-  if (nmat <= 0) return between();
-  // The kernels reduce every matrix to tridiagonal form and build Q; the
-  // host runs the QL recurrences; k_syev_apply applies the recorded
-  // rotations and writes the sorted eigenpairs.  Reduction size classes:
-  // LDS-resident up to 64 and up to 128, one workgroup per matrix over
-  // global memory up to 256 and up to 512, else one cooperative launch per
-  // matrix over the whole device.
+             double *Wbase, double *whost) {
+  if (nmat <= 0) return ITX_OK;
   // Workspace: every (d, e) first (one copy to the host), then every Q.
-  std::vector<EigTask> t64, t128, t256, t512, tg;
+  std::vector<EigTask> ts, tg;  // one workgroup per matrix; cooperative above 512 rows
   int64_t desize = 0, qsize = 0;
   for (int b = 0; b < nmat; ++b) {
     if (ns[b] < 0 || ns[b] > EMAX) return set_err(ctx, ITX_ERR_UNSUPPORTED, "itx_syev: n above 2048");
@@ -1137,21 +628,12 @@ int syev_own(itx_ctx *ctx, int nmat, const int32_t *ns, const int64_t *aoffs, do
     desize += 2 * int64_t(ns[b]);
     t.z_off = qsize;
     qsize += int64_t(ns[b]) * (ns[b] + 1);
-    if (ns[b] <= 64)
-      t64.push_back(t);
-    else if (ns[b] <= 128)
-      t128.push_back(t);
-    else if (ns[b] <= 256)
-      t256.push_back(t);
-    else if (ns[b] <= 512)
-      t512.push_back(t);
-    else
-      tg.push_back(t);
+    (ns[b] <= 512 ? ts : tg).push_back(t);
   }
   std::vector<EigTask> all;
-  for (auto *v : {&t64, &t128, &t256, &t512, &tg}) all.insert(all.end(), v->begin(), v->end());
+  for (auto *v : {&ts, &tg}) all.insert(all.end(), v->begin(), v->end());
   const int ntask = int(all.size());
-  if (ntask == 0) return between();
+  if (ntask == 0) return ITX_OK;
   for (auto &t : all) t.z_off += desize;
   const int64_t zsize = desize + qsize;
   const size_t tbytes = sizeof(EigTask) * size_t(ntask);
@@ -1169,17 +651,9 @@ int syev_own(itx_ctx *ctx, int nmat, const int32_t *ns, const int64_t *aoffs, do
   double *Z = reinterpret_cast<double *>(wsb + zoff);
   {
     const EigTask *q = dt;
-    if (!t64.empty()) hipLaunchKernelGGL(k_syev_lds<64>, dim3(unsigned(t64.size())), dim3(ES), 0, ctx->stream, q, Abase, Z);
-    q += t64.size();
-    if (!t128.empty())
-      hipLaunchKernelGGL(k_syev_lds<128>, dim3(unsigned(t128.size())), dim3(ES), 0, ctx->stream, q, Abase, Z);
-    q += t128.size();
-    if (!t256.empty())
-      hipLaunchKernelGGL((k_syev_mid<4, 4, 2, 8>), dim3(unsigned(t256.size())), dim3(MT), 0, ctx->stream, q, Abase, Z);
-    q += t256.size();
-    if (!t512.empty())
-      hipLaunchKernelGGL((k_syev_mid<8, 1, 2, 4>), dim3(unsigned(t512.size())), dim3(MT), 0, ctx->stream, q, Abase, Z);
-    q += t512.size();
+    if (!ts.empty())
+      hipLaunchKernelGGL(k_syev, dim3(unsigned(ts.size())), dim3(ET), 0, ctx->stream, q, Abase, Wbase, Z);
+    q += ts.size();
     // above 512: side by side, one workgroup each (time ~ the largest
     // n^3), or one after the other, each a cooperative launch over the
     // whole device (time ~ the sum of n^2) -- whichever the model of the
@@ -1235,10 +709,6 @@ int syev_own(itx_ctx *ctx, int nmat, const int32_t *ns, const int64_t *aoffs, do
     pool_free(ctx, ws);
     return hip_err(ctx, e, "itx_syev");
   }
-  if (int rb = between()) {
-    pool_free(ctx, ws);
-    return rb;
-  }
   // The QL recurrences, one matrix per task on the host threads, largest
   // first; every task writes its own rotations, sweep records, eigenvalues
   // and descending ranks, concatenated in matrix order afterwards.
@@ -1279,9 +749,8 @@ int syev_own(itx_ctx *ctx, int nmat, const int32_t *ns, const int64_t *aoffs, do
     HostPool::get().run(ntask, ql_task);
   else
     for (int j = 0; j < ntask; ++j) ql_task(j);
-  // apply classes: Q rows staged in LDS for n <= 64, 128, 256; else global
-  std::vector<RotMeta> cls[4];
-  int maxn[4] = {0, 0, 0, 0};
+  std::vector<RotMeta> meta;
+  int maxn = 0;
   size_t nrot = 0, nev = 0;
   for (int b = 0; b < ntask; ++b) {
     const QlOut &o = outs[size_t(b)];
@@ -1300,12 +769,9 @@ int syev_own(itx_ctx *ctx, int nmat, const int32_t *ns, const int64_t *aoffs, do
     mt.n = t.n;
     nrot += o.rots.size();
     nev += o.evr.size();
-    const int k = t.n <= 64 ? 0 : t.n <= 128 ? 1 : t.n <= 256 ? 2 : 3;
-    cls[k].push_back(mt);
-    maxn[k] = std::max(maxn[k], t.n);
+    meta.push_back(mt);
+    maxn = std::max(maxn, t.n);
   }
-  std::vector<RotMeta> meta;
-  for (auto &c : cls) meta.insert(meta.end(), c.begin(), c.end());
   const size_t mb = sizeof(RotMeta) * meta.size(), rb = sizeof(double2) * nrot, eb = sizeof(double) * nev;
   const size_t o_r = (mb + 255) & ~size_t(255), o_e = (o_r + rb + 255) & ~size_t(255);
   std::vector<char> host(o_e + eb);
@@ -1331,16 +797,8 @@ int syev_own(itx_ctx *ctx, int nmat, const int32_t *ns, const int64_t *aoffs, do
     const RotMeta *dm = reinterpret_cast<const RotMeta *>(u);
     const double2 *dr = reinterpret_cast<const double2 *>(u + o_r);
     const double *dv = reinterpret_cast<const double *>(u + o_e);
-    using Kfn = void (*)(const RotMeta *, const double2 *, const double *, double *, double *, double *);
-    const Kfn fns[4] = {k_syev_apply<64>, k_syev_apply<128>, k_syev_apply<256>, k_syev_apply<0>};
-    size_t first = 0;
-    for (int k = 0; k < 4; ++k) {
-      const size_t cnt = cls[k].size();
-      if (cnt)
-        hipLaunchKernelGGL(fns[k], dim3(unsigned(cnt), unsigned((maxn[k] + AT - 1) / AT)), dim3(AT), 0, ctx->stream,
-                           dm + first, dr, dv, Abase, Wbase, Z);
-      first += cnt;
-    }
+    hipLaunchKernelGGL(k_syev_apply, dim3(unsigned(meta.size()), unsigned((maxn + AT - 1) / AT)), dim3(AT), 0,
+                       ctx->stream, dm, dr, dv, Abase, Wbase, Z);
     e = hipGetLastError();
     if (e != hipSuccess) rc = hip_err(ctx, e, "itx_syev apply");
   }
@@ -1350,7 +808,7 @@ int syev_own(itx_ctx *ctx, int nmat, const int32_t *ns, const int64_t *aoffs, do
   return rc;
 }
 
-// ---- blocks above kOwnMax rows: rocSOLVER's divide-and-conquer dsyevd ----
+// ---- blocks above DC_MAX rows: rocSOLVER's divide-and-conquer dsyevd ----
 // ROCm's LAPACK in place of the reference's dsyev on -M: each block is
 // negated into a slot of its size class (N x N, column-major), whose
 // padding is c I with c = 1 + 2 n max|a_ij|, above every eigenvalue of -A; the
@@ -1362,11 +820,7 @@ int syev_own(itx_ctx *ctx, int nmat, const int32_t *ns, const int64_t *aoffs, do
 // per row for one matrix, and a batch of 8 costs little more than one --
 // so every block of a call goes into as few strided-batched calls as
 // possible: one, padded to the largest block, unless the slots would pass
-// 1 GiB.  When a call holds a block above kOwnMax rows, the blocks above
-// kJoinMin rows join that call (their own-kernel time would add to it);
-// otherwise every block stays on our kernels.
-constexpr int kOwnMax = 256;
-constexpr int kJoinMin = 128;
+// 1 GiB.
 constexpr int EMAX_LARGE = 8192;
 
 struct PadTask {
@@ -1526,9 +980,157 @@ int syev_large_finish(itx_ctx *ctx, LargeCall &lc, const double *Wbase, double *
   return ITX_OK;
 }
 
-// Every matrix of a call: small blocks (all of them with ITX_EIG_OWN=1, up
-// to EMAX) through our kernels, the others through rocSOLVER, enqueued
-// while the host runs the QL recurrences of the small ones.
+// ---- up to DC_MAX rows: reduction, divide and conquer, back-transformation ----
+struct DcCall {
+  std::vector<DcTask> tasks;
+  std::vector<int> mat;  // the caller's matrix of each task
+  const double *hw = nullptr;
+  const int *hstatus = nullptr;
+  unsigned long long seq = 0;
+};
+
+// Eigenvalues and states of a call, written by the device and read by the
+// host after the completion flag: coherent pinned memory of the context,
+// grown as needed.
+int eig_host(itx_ctx *ctx, size_t bytes) {
+  if (ctx->eig_host_bytes >= bytes) return ITX_OK;
+  ITX_CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  if (ctx->eig_host) hipHostFree(ctx->eig_host);
+  ctx->eig_host = nullptr;
+  ctx->eig_host_bytes = 0;
+  const size_t cap = std::max<size_t>(2 * bytes, size_t(1) << 16);
+  ITX_CHECK_HIP(ctx, hipHostMalloc(&ctx->eig_host, cap, hipHostMallocMapped | hipHostMallocCoherent));
+  ctx->eig_host_bytes = cap;
+  return ITX_OK;
+}
+
+// Enqueues everything; the workspace goes back to the stream-ordered pool.
+int syev_dc_launch(itx_ctx *ctx, std::vector<int> mats, const int32_t *ns, const int64_t *aoffs, double *Abase,
+                   const int64_t *woffs, double *Wbase, DcCall &call) {
+  const int nt = int(mats.size());
+  if (nt == 0) return ITX_OK;
+  // the matrices above 64 rows first (nb of them); the others take one launch
+  std::stable_partition(mats.begin(), mats.end(), [&](int b) { return ns[b] > 64; });
+  const int nb = int(std::count_if(mats.begin(), mats.end(), [&](int b) { return ns[b] > 64; }));
+  std::vector<TriTask> tri(static_cast<size_t>(nt));
+  std::vector<BackTask> back(static_cast<size_t>(nt));
+  call.tasks.resize(size_t(nt));
+  call.mat = mats;
+  int64_t off = 0, xsize = 0, neig = 0;
+  for (int i = 0; i < nt; ++i) {
+    const int b = mats[size_t(i)], n = ns[b];
+    TriTask &t = tri[size_t(i)];
+    DcTask &d = call.tasks[size_t(i)];
+    BackTask &k = back[size_t(i)];
+    t.n = d.n = k.n = n;
+    t.a_off = k.o_off = aoffs[b];
+    d.w_off = woffs[b];
+    d.p = dc_levels(n);
+    t.v_off = k.v_off = off;
+    off += int64_t(n) * n;
+    t.d_off = d.d_off = k.d_off = off;
+    off += 3 * int64_t(n);
+    d.q_off = off;
+    off += 4 * int64_t(n) * n;
+    d.x_off = off;
+    off += int64_t(AUX_SIZE(n));
+    k.s_off = d.q_off + dc_vectors(n);
+    d.r_off = k.r_off = neig;
+    neig += n;
+  }
+  const int64_t x0 = off;
+  for (TriTask &t : tri) {
+    t.x_off = x0 + xsize;
+    xsize += int64_t(tri_exchange(t.n));
+  }
+  off += xsize;
+  std::vector<int2> tb, db, bb;
+  std::vector<size_t> ends;
+  std::vector<DcLevel> levels;
+  tri_blocks(tri, nb, std::max(1, ctx->num_cus), tb, ends);
+  dc_blocks(call.tasks, nb, db, levels);
+  back_blocks(back, nb, bb);
+  int rc = eig_host(ctx, sizeof(double) * size_t(neig) + sizeof(int) * size_t(nt));
+  if (rc) return rc;
+  // one upload: the records, and the states and counter as zeros
+  const std::vector<int> zeros(size_t(nt) + 1, 0);
+  UploadPart parts[7];
+  size_t pos = 0;
+  auto part = [&](int i, const void *src, size_t bytes) {
+    parts[i] = UploadPart{src, pos, bytes};
+    pos = (pos + bytes + 255) & ~size_t(255);
+  };
+  part(0, tri.data(), sizeof(TriTask) * tri.size());
+  part(1, tb.data(), sizeof(int2) * tb.size());
+  part(2, call.tasks.data(), sizeof(DcTask) * call.tasks.size());
+  part(3, db.data(), sizeof(int2) * db.size());
+  part(4, back.data(), sizeof(BackTask) * back.size());
+  part(5, bb.data(), sizeof(int2) * bb.size());
+  part(6, zeros.data(), sizeof(int) * zeros.size());
+  const size_t o_rank = pos, o_w = (o_rank + sizeof(int) * size_t(neig) + 255) & ~size_t(255);
+  void *ws = nullptr;
+  rc = pool_alloc(ctx, o_w + sizeof(double) * size_t(off), &ws);
+  if (rc) return rc;
+  char *p = static_cast<char *>(ws);
+  rc = stage_upload_parts(ctx, p, parts, 7, o_rank);
+  if (rc) {
+    pool_free(ctx, ws);
+    return rc;
+  }
+  double *W = reinterpret_cast<double *>(p + o_w);
+  int *rank = reinterpret_cast<int *>(p + o_rank);
+  int *status = reinterpret_cast<int *>(p + parts[6].off);
+  auto at = [&](int i) { return p + parts[i].off; };
+  double *hw = static_cast<double *>(ctx->eig_host);
+  int *hstatus = reinterpret_cast<int *>(hw + neig);
+  call.hw = hw;
+  call.hstatus = hstatus;
+  call.seq = ++ctx->hres_seq;
+  const DcOut out{rank, hw, status, hstatus, reinterpret_cast<unsigned *>(status + nt),
+                  reinterpret_cast<unsigned long long *>(ctx->hres_dev + HRES_SLOTS), call.seq, nt};
+  const TriTask *dtri = reinterpret_cast<const TriTask *>(at(0));
+  const DcTask *ddc = reinterpret_cast<const DcTask *>(at(2));
+  const BackTask *dback = reinterpret_cast<const BackTask *>(at(4));
+  syev_small_launch(ctx, dtri, ddc, dback, nb, nt - nb, Abase, W, Wbase, out);
+  tri_launch(ctx, dtri, reinterpret_cast<const int2 *>(at(1)), ends, Abase, W, x0, size_t(xsize), status);
+  dc_launch(ctx, ddc, nb, reinterpret_cast<const int2 *>(at(3)), levels, W, Wbase, out);
+  back_launch(ctx, dback, reinterpret_cast<const int2 *>(at(5)), bb.size(), W, W, Abase, rank, status);
+  pool_free(ctx, ws);  // stream-ordered
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? ITX_OK : hip_err(ctx, e, "itx_syev");
+}
+
+// Waits for the eigenvalues and states; the vectors may still be under way.
+int syev_dc_finish(itx_ctx *ctx, const DcCall &call, const int32_t *ns, const int64_t *aoffs, double *Abase,
+                   const int64_t *woffs, double *Wbase, double *whost) {
+  if (call.tasks.empty()) return ITX_OK;
+  volatile unsigned long long *hflag = reinterpret_cast<volatile unsigned long long *>(ctx->hres + HRES_SLOTS);
+  const auto t0 = std::chrono::steady_clock::now();
+  for (long it = 0; *hflag != call.seq; ++it)
+    if ((it & 1023) == 1023 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(50)) {
+      ITX_CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
+      if (*hflag != call.seq) return set_err(ctx, ITX_ERR_HIP, "itx_syev: completion flag not set");
+      break;
+    }
+  std::atomic_thread_fence(std::memory_order_acquire);
+  std::vector<int32_t> rn;
+  std::vector<int64_t> ra, rw;
+  for (size_t i = 0; i < call.tasks.size(); ++i) {
+    const DcTask &t = call.tasks[i];
+    const int b = call.mat[i];
+    if (call.hstatus[i] == 1)
+      return set_err(ctx, ITX_ERR_NOCONV, "itx_syev: the matrix holds values that are not finite");
+    if (call.hstatus[i] == 2) {  // A is untouched: the path without meetings
+      rn.push_back(ns[b]);
+      ra.push_back(aoffs[b]);
+      rw.push_back(woffs[b]);
+    } else if (whost) {
+      std::memcpy(whost + t.w_off, call.hw + t.r_off, sizeof(double) * size_t(t.n));
+    }
+  }
+  return syev_own(ctx, int(rn.size()), rn.data(), ra.data(), Abase, rw.data(), Wbase, whost);
+}
+
 int syev_batched(itx_ctx *ctx, int nmat, const int32_t *ns, const int64_t *aoffs, double *Abase,
                  const int64_t *woffs, double *Wbase, double *whost) {
   if (nmat <= 0) return ITX_OK;
@@ -1538,17 +1140,17 @@ int syev_batched(itx_ctx *ctx, int nmat, const int32_t *ns, const int64_t *aoffs
   }();
   std::vector<int32_t> on;
   std::vector<int64_t> oa, ow;
+  std::vector<int> small;
   std::vector<PadTask> large;
-  bool any_large = false;
-  for (int b = 0; b < nmat; ++b) any_large = any_large || ns[b] > kOwnMax;
-  const int own_max = own_only ? EMAX : any_large ? kJoinMin : kOwnMax;
   for (int b = 0; b < nmat; ++b) {
     const int n = ns[b];
     if (n < 0 || n > (own_only ? EMAX : EMAX_LARGE))
       return set_err(ctx, ITX_ERR_UNSUPPORTED,
                      own_only ? "itx_syev: n above 2048 (ITX_EIG_OWN)" : "itx_syev: n above 8192");
     if (n == 0) continue;
-    if (n <= own_max) {
+    if (n <= DC_MAX) {
+      small.push_back(b);
+    } else if (own_only) {
       on.push_back(n);
       oa.push_back(aoffs[b]);
       ow.push_back(woffs[b]);
@@ -1560,16 +1162,22 @@ int syev_batched(itx_ctx *ctx, int nmat, const int32_t *ns, const int64_t *aoffs
       large.push_back(t);
     }
   }
+  DcCall call;
+  int rc = syev_dc_launch(ctx, small, ns, aoffs, Abase, woffs, Wbase, call);
+  if (rc) return rc;
   LargeCall lc;
-  int rc = syev_own(ctx, int(on.size()), on.data(), oa.data(), Abase, ow.data(), Wbase, whost,
-                    [&] { return syev_large_launch(ctx, std::move(large), Abase, Wbase, lc); });
+  rc = syev_large_launch(ctx, std::move(large), Abase, Wbase, lc);
+  const int rc1 = syev_dc_finish(ctx, call, ns, aoffs, Abase, woffs, Wbase, whost);
   const int rc2 = syev_large_finish(ctx, lc, Wbase, whost);
-  return rc ? rc : rc2;
+  if (!rc) rc = rc1 ? rc1 : rc2;
+  return rc ? rc : syev_own(ctx, int(on.size()), on.data(), oa.data(), Abase, ow.data(), Wbase, whost);
 }
 
 void eig_release(itx_ctx *ctx) {
   if (ctx->rocblas) rocblas_destroy_handle(static_cast<rocblas_handle>(ctx->rocblas));
   ctx->rocblas = nullptr;
+  if (ctx->eig_host) hipHostFree(ctx->eig_host);
+  ctx->eig_host = nullptr;
 }
 
 }  // namespace itx

@@ -113,6 +113,10 @@ struct itx_ctx {
   size_t scratch_bytes = 0;
   // rocblas handle of the large-block eigensolver (created on first use)
   void *rocblas = nullptr;
+  // eigenvalues and states that the eigensolver's kernels write for the
+  // host (coherent pinned memory, grown on demand, freed by eig_release)
+  void *eig_host = nullptr;
+  size_t eig_host_bytes = 0;
   // pinned host memory: reduction results written by the device
   // (hres, device view hres_dev; coherent, with a completion flag after
   // the HRES_SLOTS result slots) and the staging arena of uploads
@@ -141,7 +145,7 @@ struct itx_ctx {
 namespace itx {
 
 int set_err(itx_ctx *ctx, int code, const std::string &msg);
-// releases the eigensolver's library handle (itx_destroy)
+// releases the eigensolver's library handle and pinned memory (itx_destroy)
 void eig_release(itx_ctx *ctx);
 int hip_err(itx_ctx *ctx, hipError_t e, const char *where);
 
