@@ -26,7 +26,7 @@ INCLUDE = os.path.join(ROOT, "include")
 
 HIP_SOURCES = ["itx_runtime.hip", "itx_contract.hip", "itx_vec.hip", "itx_eig.hip", "itx_tridiag.hip", "itx_dc.hip", "itx_svd.hip"]
 EIG_HEADERS = [os.path.join(CSRC, "itx_eig.h"), os.path.join(CSRC, "itx_tri.h")]
-EIG_SOURCES = ("itx_eig.hip", "itx_tridiag.hip", "itx_dc.hip")
+EIG_SOURCES = ("itx_eig.hip", "itx_tridiag.hip", "itx_dc.hip", "itx_svd.hip")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # Packed FP32 instructions are disabled for all device code (they have
 # produced wrong results on this hardware); -O3 for the kernels.

@@ -15,16 +15,24 @@
 // vectors accurate without the refinement step the density-matrix method
 // needs.  Pairs are scheduled round-robin (k/2 disjoint pairs per round,
 // k-1 rounds per sweep), each pair reduced by a group of lanes.
+#include <algorithm>
 #include <cfloat>
 #include <cstring>
+#include <type_traits>
 
-#include "itx_internal.h"
+#include "itx_eig.h"
 
 namespace itx {
 namespace {
 
-constexpr int ST = 256;             // threads per matrix
+constexpr int ST = 1024;            // threads per matrix
 constexpr int SVD_MAX_SWEEPS = 60;  // sweeps before reporting no convergence
+// X and J in LDS (columns at odd pitches) when they fit, else in the workspace
+constexpr size_t SVD_LDS = 160 * 1024 - 512;  // of 160 KB: 100 x 100 fits
+__host__ __device__ inline size_t svd_lds(int m, int n) {
+  const size_t R = m < n ? m : n, C = m < n ? n : m;
+  return sizeof(double) * R * ((C | 1) + (R | 1));
+}
 
 struct SvdTask {
   int32_t m, n;
@@ -32,43 +40,58 @@ struct SvdTask {
   int64_t x_off;  // workspace: X (C x R), J (R x R), sigma (R), rank (R)
 };
 
-__device__ __forceinline__ double group_sum(double v, int G) {
-  for (int o = G >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+// sums of three values over the G lanes of a group, step by step so that
+// the three chains overlap
+template <int G>
+__device__ __forceinline__ void group_sums(double &a, double &b, double &c) {
+  if constexpr (G > 1) a += dpp_move<DPP_XOR1>(a), b += dpp_move<DPP_XOR1>(b), c += dpp_move<DPP_XOR1>(c);
+  if constexpr (G > 2) a += dpp_move<DPP_XOR2>(a), b += dpp_move<DPP_XOR2>(b), c += dpp_move<DPP_XOR2>(c);
+  if constexpr (G > 4)
+    a += dpp_move<DPP_HALF_MIRROR>(a), b += dpp_move<DPP_HALF_MIRROR>(b), c += dpp_move<DPP_HALF_MIRROR>(c);
+  if constexpr (G > 8) a += dpp_move<DPP_ROR8>(a), b += dpp_move<DPP_ROR8>(b), c += dpp_move<DPP_ROR8>(c);
+  if constexpr (G > 16) a = swap16_add(a, a), b = swap16_add(b, b), c = swap16_add(c, c);
+  if constexpr (G > 32) a = swap32_add(a, a), b = swap32_add(b, b), c = swap32_add(c, c);
 }
 
-__global__ __launch_bounds__(ST) void k_gesvd(const SvdTask *__restrict__ tasks, const double *__restrict__ Abase,
-                                              double *__restrict__ Ubase, double *__restrict__ Sbase,
-                                              double *__restrict__ Vbase, double *__restrict__ Wbase,
-                                              int *__restrict__ status) {
-  __shared__ int sh_rot;
-  const SvdTask tk = tasks[blockIdx.x];
+// One workgroup per matrix.  A sweep is R - 1 dependent rounds of R / 2
+// independent pairs, so a round's latency bounds it: a pair has up to 64
+// lanes, its columns come from LDS where the matrix fits, and a barrier
+// orders LDS only (blocks up to 37 x 37: 0.42 ms for some 10 sweeps, 1.1 us
+// a round; from the workspace, with 256 threads, 1.14 ms).
+template <bool LDS, int G>
+__device__ __forceinline__ void gesvd_run(const SvdTask &tk, const double *__restrict__ Abase,
+                                          double *__restrict__ Ubase, double *__restrict__ Sbase,
+                                          double *__restrict__ Vbase, double *__restrict__ Wbase,
+                                          int *__restrict__ status, double *lds, int *sh_rot) {
   const int m = tk.m, n = tk.n;
   const int R = min(m, n), C = max(m, n);
   const int tid = threadIdx.x;
-  if (R <= 0) {
-    if (tid == 0) status[blockIdx.x] = 0;
-    return;
-  }
   const double *__restrict__ A = Abase + tk.a_off;
-  double *__restrict__ X = Wbase + tk.x_off;
-  double *__restrict__ J = X + size_t(C) * R;
-  double *__restrict__ sig = J + size_t(R) * R;
+  const int PX = LDS ? (C | 1) : C, PJ = LDS ? (R | 1) : R;  // column pitches
+  double *X = LDS ? lds : Wbase + tk.x_off;
+  double *J = X + size_t(PX) * R;
+  double *__restrict__ sig = Wbase + tk.x_off + (LDS ? 0 : size_t(C) * R + size_t(R) * R);
   double *__restrict__ rnk = sig + R;
   const bool wide = m <= n;  // X = A^T
+  auto meet = [&]() {
+    if constexpr (LDS)
+      lds_barrier();
+    else
+      __syncthreads();
+  };
 
-  for (size_t x = tid; x < size_t(C) * R; x += ST) {
-    const size_t c = x % C, r = x / C;
-    X[x] = wide ? A[r + size_t(m) * c] : A[c + size_t(m) * r];
+  using Count = std::conditional_t<LDS, int, size_t>;
+  const Count cr = Count(C) * R, rr = Count(R) * R;
+  for (Count x = tid; x < cr; x += ST) {  // A read in its own order
+    const Count i = x % m, j = x / m;
+    (wide ? X[size_t(i) * PX + j] : X[size_t(j) * PX + i]) = A[x];
   }
-  for (size_t x = tid; x < size_t(R) * R; x += ST) J[x] = (x % R == x / R) ? 1.0 : 0.0;
-  if (tid == 0) sh_rot = 0;
+  for (Count x = tid; x < rr; x += ST) J[size_t(x / R) * PJ + x % R] = (x % R == x / R) ? 1.0 : 0.0;
+  if (tid < 2) sh_rot[tid] = 0;
   __syncthreads();
 
   // round-robin schedule over Rp (even) slots; slot R is a dummy when R is odd
   const int Rp = R + (R & 1), P = Rp / 2;
-  int G = 64;
-  while (G > 1 && G * P > ST) G >>= 1;
   const int NG = ST / G, grp = tid / G, g = tid % G;
   const double tol = 4.0 * DBL_EPSILON * sqrt(double(C));
 
@@ -76,7 +99,10 @@ __global__ __launch_bounds__(ST) void k_gesvd(const SvdTask *__restrict__ tasks,
   for (; sweep < SVD_MAX_SWEEPS; ++sweep) {
     for (int k = 0; k < Rp - 1; ++k) {
       for (int p = grp; p < P; p += NG) {
-        auto pos = [&](int x) { return x == 0 ? 0 : 1 + (x - 1 + k) % (Rp - 1); };
+        auto pos = [&](int x) {
+          const int y = x - 1 + k;
+          return x == 0 ? 0 : 1 + (y >= Rp - 1 ? y - (Rp - 1) : y);
+        };
         int a = pos(p), b = pos(Rp - 1 - p);
         if (a >= R || b >= R) continue;  // group-uniform
         if (a > b) {
@@ -84,59 +110,110 @@ __global__ __launch_bounds__(ST) void k_gesvd(const SvdTask *__restrict__ tasks,
           a = b;
           b = t;
         }
-        double *xa = X + size_t(a) * C, *xb = X + size_t(b) * C;
+        double *xa = X + size_t(a) * PX, *xb = X + size_t(b) * PX;
+        double *ja = J + size_t(a) * PJ, *jb = J + size_t(b) * PJ;
+        // the first four elements of a lane stay in registers from the sums
+        // to the rotation, and J's are on their way meanwhile
+        double xu[4], xv[4], ju[4], jv[4];
         double al = 0, be = 0, ga = 0;
-        for (int c = g; c < C; c += G) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int c = g + G * t;
+          xu[t] = c < C ? xa[c] : 0.0;
+          xv[t] = c < C ? xb[c] : 0.0;
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int c = g + G * t;
+          ju[t] = c < R ? ja[c] : 0.0;
+          jv[t] = c < R ? jb[c] : 0.0;
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          al = fma(xu[t], xu[t], al);
+          be = fma(xv[t], xv[t], be);
+          ga = fma(xu[t], xv[t], ga);
+        }
+#pragma unroll 2
+        for (int c = g + 4 * G; c < C; c += G) {
           const double u = xa[c], v = xb[c];
           al = fma(u, u, al);
           be = fma(v, v, be);
           ga = fma(u, v, ga);
         }
-        al = group_sum(al, G);
-        be = group_sum(be, G);
-        ga = group_sum(ga, G);
-        if (ga == 0.0 || al == 0.0 || be == 0.0 || fabs(ga) <= tol * sqrt(al) * sqrt(be)) continue;
-        const double zeta = (be - al) / (2.0 * ga);
-        const double t = copysign(1.0, zeta) / (fabs(zeta) + sqrt(fma(zeta, zeta, 1.0)));
-        const double cs = 1.0 / sqrt(fma(t, t, 1.0)), sn = cs * t;
-        for (int c = g; c < C; c += G) {
+        group_sums<G>(al, be, ga);
+        // rotate unless the pair is orthogonal to working precision; the
+        // products of the fast form stay in range for norms within 1e+-35
+        double cs, sn;
+        const double top = fmax(al, be), low = fmin(al, be);
+        if (top < 1e70 && low > 1e-70) {
+          if (ga * ga <= tol * tol * (al * be)) continue;
+          // t = tan of the angle that zeroes ga: the smaller root of t^2 + 2 zeta t - 1
+          const double dl = be - al, g2 = 2.0 * ga;
+          const double t = copysign(g2, dl >= 0.0 ? ga : -ga) * fast_rcp(fabs(dl) + fast_sqrt(fma(dl, dl, g2 * g2)));
+          cs = fast_rsqrt(fma(t, t, 1.0));
+          sn = cs * t;
+        } else {
+          if (ga == 0.0 || al == 0.0 || be == 0.0 || fabs(ga) <= tol * sqrt(al) * sqrt(be)) continue;
+          const double zeta = (be - al) / (2.0 * ga);
+          const double t = copysign(1.0, zeta) / (fabs(zeta) + sqrt(fma(zeta, zeta, 1.0)));
+          cs = 1.0 / sqrt(fma(t, t, 1.0));
+          sn = cs * t;
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int c = g + G * t;
+          if (c < C) {
+            xa[c] = cs * xu[t] - sn * xv[t];
+            xb[c] = sn * xu[t] + cs * xv[t];
+          }
+          if (c < R) {
+            ja[c] = cs * ju[t] - sn * jv[t];
+            jb[c] = sn * ju[t] + cs * jv[t];
+          }
+        }
+#pragma unroll 2
+        for (int c = g + 4 * G; c < C; c += G) {
           const double u = xa[c], v = xb[c];
           xa[c] = cs * u - sn * v;
           xb[c] = sn * u + cs * v;
         }
-        double *ja = J + size_t(a) * R, *jb = J + size_t(b) * R;
-        for (int r = g; r < R; r += G) {
+#pragma unroll 2
+        for (int r = g + 4 * G; r < R; r += G) {
           const double u = ja[r], v = jb[r];
           ja[r] = cs * u - sn * v;
           jb[r] = sn * u + cs * v;
         }
-        if (g == 0) sh_rot = 1;
+        if (g == 0) sh_rot[sweep & 1] = 1;
       }
-      __syncthreads();
+      meet();
     }
-    const int rot = sh_rot;
-    __syncthreads();  // every thread has read the flag before it is reset
+    // this sweep's flag was set before the round's barrier; the other one is
+    // cleared for the next sweep, whose rounds begin after the barrier below
+    const int rot = sh_rot[sweep & 1];
+    if (tid == 0) sh_rot[(sweep + 1) & 1] = 0;
+    meet();
     if (!rot) break;
-    if (tid == 0) sh_rot = 0;
-    __syncthreads();
   }
   if (sweep == SVD_MAX_SWEEPS) {
-    if (tid == 0) status[blockIdx.x] = 1;
+    if (tid == 0) *status = 1;
     return;
   }
 
   // singular values (column norms) and their descending stable ranks
   for (int r = grp; r < R; r += NG) {
-    const double *xr = X + size_t(r) * C;
+    const double *xr = X + size_t(r) * PX;
     double s = 0;
     for (int c = g; c < C; c += G) s = fma(xr[c], xr[c], s);
-    s = group_sum(s, G);
+    double o1 = 0, o2 = 0;
+    group_sums<G>(s, o1, o2);
     if (g == 0) sig[r] = sqrt(s);
   }
   __syncthreads();
   for (int r = tid; r < R; r += ST) {
     const double sr = sig[r];
     int rank = 0;
+#pragma unroll 4
     for (int j = 0; j < R; ++j) rank += (sig[j] > sr) || (sig[j] == sr && j < r);
     rnk[r] = double(rank);
   }
@@ -147,16 +224,51 @@ __global__ __launch_bounds__(ST) void k_gesvd(const SvdTask *__restrict__ tasks,
   double *__restrict__ Long = wide ? V : U;    // C x R: normalised columns of X
   double *__restrict__ Short = wide ? U : V;   // R x R: J
   for (int r = tid; r < R; r += ST) S[int(rnk[r])] = sig[r];
-  for (size_t x = tid; x < size_t(C) * R; x += ST) {
-    const size_t c = x % C, r = x / C;
+  for (Count x = tid; x < cr; x += ST) {
+    const Count c = x % C, r = x / C;
     const double sr = sig[r];
-    Long[size_t(rnk[r]) * C + c] = sr > 0.0 ? X[x] / sr : 0.0;
+    Long[size_t(rnk[r]) * C + c] = sr > 0.0 ? X[size_t(r) * PX + c] / sr : 0.0;
   }
-  for (size_t x = tid; x < size_t(R) * R; x += ST) {
-    const size_t i = x % R, r = x / R;
-    Short[size_t(rnk[r]) * R + i] = J[x];
+  for (Count x = tid; x < rr; x += ST) {
+    const Count i = x % R, r = x / R;
+    Short[size_t(rnk[r]) * R + i] = J[size_t(r) * PJ + i];
   }
-  if (tid == 0) status[blockIdx.x] = 0;
+  if (tid == 0) *status = 0;
+}
+
+__global__ __launch_bounds__(ST) void k_gesvd(const SvdTask *__restrict__ tasks, const double *__restrict__ Abase,
+                                              double *__restrict__ Ubase, double *__restrict__ Sbase,
+                                              double *__restrict__ Vbase, double *__restrict__ Wbase,
+                                              int *__restrict__ status, unsigned lds_bytes) {
+  extern __shared__ double lds[];
+  __shared__ int sh_rot[2];
+  const SvdTask tk = tasks[blockIdx.x];
+  int *st = status + blockIdx.x;
+  if (min(tk.m, tk.n) <= 0) {
+    if (threadIdx.x == 0) *st = 0;
+    return;
+  }
+  // as many lanes per pair as the threads allow for all pairs of a round
+  const int P = (min(tk.m, tk.n) + 1) / 2;
+  const bool in = svd_lds(tk.m, tk.n) <= lds_bytes;
+#define ITX_SVD(L, G) gesvd_run<L, G>(tk, Abase, Ubase, Sbase, Vbase, Wbase, st, lds, sh_rot)
+  if (in && P * 64 <= ST)
+    ITX_SVD(true, 64);
+  else if (in && P * 32 <= ST)
+    ITX_SVD(true, 32);
+  else if (in && P * 16 <= ST)
+    ITX_SVD(true, 16);
+  else if (in)
+    ITX_SVD(true, 8);  // at most 68 pairs fit
+  else if (P * 64 <= ST)
+    ITX_SVD(false, 64);
+  else if (P * 16 <= ST)
+    ITX_SVD(false, 16);
+  else if (P * 4 <= ST)
+    ITX_SVD(false, 4);
+  else
+    ITX_SVD(false, 1);
+#undef ITX_SVD
 }
 
 }  // namespace
@@ -194,9 +306,15 @@ extern "C" int itx_gesvd_batched(itx_ctx *ctx, int nmat, const int32_t *m, const
     return rc;
   }
   int *dst = reinterpret_cast<int *>(wsb + tbytes);
-  hipLaunchKernelGGL(itx::k_gesvd, dim3(unsigned(nmat)), dim3(itx::ST), 0, ctx->stream,
+  // LDS for the largest matrix that fits
+  size_t lds = 0;
+  for (int b = 0; b < nmat; ++b) {
+    const size_t need = itx::svd_lds(m[b], n[b]);
+    if (need <= itx::SVD_LDS) lds = std::max(lds, need);
+  }
+  hipLaunchKernelGGL(itx::k_gesvd, dim3(unsigned(nmat)), dim3(itx::ST), lds, ctx->stream,
                      reinterpret_cast<const itx::SvdTask *>(wsb), A, U, S, V, reinterpret_cast<double *>(wsb + woff),
-                     dst);
+                     dst, unsigned(lds));
   hipError_t e = hipGetLastError();
   std::vector<int> st(static_cast<size_t>(nmat), 0);
   if (e == hipSuccess) e = hipMemcpyAsync(st.data(), dst, sbytes, hipMemcpyDeviceToHost, ctx->stream);
