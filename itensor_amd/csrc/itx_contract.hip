@@ -1288,89 +1288,193 @@ __global__ __launch_bounds__(SK_ROWS) void k_skinny_q(const double *__restrict__
 }
 
 // Small-block contractions (C blocks of a few thousand elements: the QN
-// blocks of DMRG at moderate bond dimension): latency-bound, so FP64 VALU
-// arithmetic in every form.  A unit is a 64 x 32 tile of one C block; for
-// each task and 64-wide k chunk the A tile and the B tile are staged
-// cooperatively in LDS -- one round of independent loads, lanes packed
-// along the operand's unit stride -- then each thread accumulates 8
-// outputs of one row.  Same task/unit/table format as k_gemm.
-constexpr int SM_M = 64, SM_N = 32, SM_K = 64, SM_T = 256, SM_NPT = 8;
-constexpr int SM_LDA = SM_M + 1;  // pad: the k-contiguous staging stores hit distinct banks
+// blocks of DMRG at moderate bond dimension).  Latency-bound: what counts is
+// the number of dependent trips through memory of a unit, a 64 x 32 tile of
+// one C block.  FP64 form, on the matrix cores straight from memory: a wave
+// loads the fragments of 32 x 32 outputs for 16 k at once (rows over 16
+// lanes, 4 k over the lane quarters) while it multiplies the previous 16, and
+// the four waves share a unit's k: with up to 32 rows each takes every fourth
+// task (or, with fewer than four tasks, every fourth 16 k of each), above
+// that two waves per half of the rows.  The waves' sums meet in LDS once.
+// Staging both tiles in LDS for VALU arithmetic, the form before this one,
+// made two barriers and three such trips per 64 k and task; the last stage of
+// the dense chi = 32 chain (one 128 x 32 block, K = 160) took 31 us with its
+// reduction pass.
+// Same task/unit/table format as k_gemm.
+constexpr int SM_M = 64, SM_N = 32, SM_K = 64, SM_T = 256;
+constexpr int SMD_W = 8, SMD_T = 64 * SMD_W;  // waves of the FP64 form
+constexpr int SMD_P = 17;                     // its LDS row pitch
+
+// One operand's 32 rows (or columns) x 16 k of a wave.  Contiguous along k
+// (KC): lanes walk k, four rows per load (with lanes over rows each load
+// would touch 64 separate segments, which the address unit takes one by one:
+// 15 us for the chi = 32 block against 5), and the wave's own LDS buffer turns
+// them into fragments; else lanes walk the rows and the loads are fragments.
+template <bool KC>
+struct SmallOperand {
+  static constexpr int NR = KC ? 8 : 2;  // rows of a lane
+  const double *row[NR];
+  double x[8] = {};
+  // rows: first row, last valid row; tab: its row offsets
+  __device__ __forceinline__ void init(const double *base, int row0, int last, const int64_t *__restrict__ tab, int lane) {
+#pragma unroll
+    for (int p = 0; p < NR; ++p) {
+      const int r = KC ? 4 * p + (lane >> 4) : 16 * p + (lane & 15);
+      row[p] = base + tab[min(row0 + r, last)];
+    }
+  }
+  // two: the second group of 16 rows is in use
+  __device__ __forceinline__ void load(int k0, int K, const int64_t *__restrict__ tab, bool two, int lane) {
+    if constexpr (KC) {
+      const int64_t ko = tab[min(k0 + (lane & 15), K - 1)];
+#pragma unroll
+      for (int p = 0; p < 4; ++p) x[p] = row[p][ko];
+      if (two) {
+#pragma unroll
+        for (int p = 4; p < 8; ++p) x[p] = row[p][ko];
+      }
+    } else {
+      int64_t ko[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) ko[s] = tab[min(k0 + 4 * s + (lane >> 4), K - 1)];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) x[2 * s] = row[0][ko[s]];
+      if (two) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) x[2 * s + 1] = row[1][ko[s]];
+      }
+    }
+  }
+  // f[s][g]: fragment of k slot s, row group g
+  __device__ __forceinline__ void fragments(double (&f)[4][2], double *buf, int lane) const {
+    if constexpr (KC) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int p = 0; p < 8; ++p) buf[(4 * p + (lane >> 4)) * SMD_P + (lane & 15)] = x[p];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int g = 0; g < 2; ++g) f[s][g] = buf[(16 * g + (lane & 15)) * SMD_P + 4 * s + (lane >> 4)];
+    } else {
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int g = 0; g < 2; ++g) f[s][g] = x[2 * s + g];
+    }
+  }
+};
 
 template <bool AKC, bool BKC>
-__global__ __launch_bounds__(SM_T) void k_small(const double *__restrict__ A, const double *__restrict__ B,
-                                                double *__restrict__ C, const GemmTask *__restrict__ tasks,
-                                                const WorkUnit *__restrict__ units, int nunits,
-                                                const int64_t *__restrict__ tab, double alpha, double beta) {
-  __shared__ double As[SM_K * SM_LDA];
-  __shared__ double Bs[SM_K * SM_N];
-  const int tid = threadIdx.x;
-  const int mi = tid & (SM_M - 1), ng = tid >> 6;  // output row, group of 8 columns
+__global__ __launch_bounds__(SMD_T) void k_small(const double *__restrict__ A, const double *__restrict__ B,
+                                                 double *__restrict__ C, const GemmTask *__restrict__ tasks,
+                                                 const WorkUnit *__restrict__ units, int nunits,
+                                                 const int64_t *__restrict__ tab, double alpha, double beta) {
+  using v4 = MF<double>::v4;
+  constexpr int BUF = 32 * SMD_P;
+  __shared__ double lds[SMD_W * 2 * BUF];  // operand buffers of the waves, then their sums
+  static_assert(2 * BUF >= 16 * 64, "room for the sums");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r16 = lane & 15, q4 = lane >> 4;
+  double *bufA = lds + wave * 2 * BUF, *bufB = bufA + BUF;
+  double(*part)[16][64] = reinterpret_cast<double(*)[16][64]>(lds);
   for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
     const WorkUnit wu = units[u];
-    double acc[SM_NPT];
-#pragma unroll
-    for (int j = 0; j < SM_NPT; ++j) acc[j] = 0.0;
-    for (int t = wu.tbeg; t < wu.tend; ++t) {
-      const GemmTask tk = tasks[t];
-      const int rows = min(SM_M, tk.M - wu.m0), cols = min(SM_N, tk.N - wu.n0);
-      for (int k0 = 0; k0 < tk.K; k0 += SM_K) {
-        const int kc = min(SM_K, tk.K - k0);
-        __syncthreads();  // the previous chunk's tiles are no longer read
-        // A tile (rows x kc) -> As[k][m]; consecutive lanes follow A's
-        // unit stride (k when A is k-contiguous, else m), packed densely
-        {
-          const int na = rows * kc, lead = AKC ? kc : rows;
-          for (int e = tid; e < na; e += SM_T) {
-            const int q = e / lead, r = e - q * lead;
-            const int m = AKC ? q : r, k = AKC ? r : q;
-            As[k * SM_LDA + m] = A[tk.a_off + tab[tk.tAM + wu.m0 + m] + tab[tk.tAK + k0 + k]];
-          }
-        }
-        // B tile (kc x cols) -> Bs[k][n], likewise
-        {
-          const int nb = kc * cols, lead = BKC ? kc : cols;
-          for (int e = tid; e < nb; e += SM_T) {
-            const int q = e / lead, r = e - q * lead;
-            const int n = BKC ? q : r, k = BKC ? r : q;
-            Bs[k * SM_N + n] = B[tk.b_off + tab[tk.tBK + k0 + k] + tab[tk.tBN + wu.n0 + n]];
-          }
-          // columns beyond the block are read by the last column group
-          for (int e = tid; e < kc * (SM_N - cols); e += SM_T) {
-            const int k = e / (SM_N - cols), n = cols + (e - k * (SM_N - cols));
-            Bs[k * SM_N + n] = 0.0;
-          }
-        }
-        __syncthreads();
-        const double *bp = Bs + ng * SM_NPT;
-        for (int k = 0; k < kc; ++k) {
-          const double a = As[k * SM_LDA + mi];
-#pragma unroll
-          for (int j = 0; j < SM_NPT; ++j) acc[j] = fma(a, bp[k * SM_N + j], acc[j]);
-        }
-      }
-    }
-    if (wu.slot >= 0) {  // partial tile of a split unit (C is the workspace)
-      double *P = C + size_t(wu.slot) * (SM_M * SM_N);
-#pragma unroll
-      for (int j = 0; j < SM_NPT; ++j) P[(ng * SM_NPT + j) * SM_M + mi] = acc[j];
-      continue;
-    }
     const GemmTask t0 = tasks[wu.tbeg];
-    const int m = wu.m0 + mi;
-    if (m < t0.M) {
-      double *Cm = C + t0.c_off + tab[t0.tCM + m];
+    // the unit's end: its tile (pad: rows | columns << 8) inside the block
+    const int mend = min(t0.M, wu.m0 + (wu.pad & 255)), nend = min(t0.N, wu.n0 + (wu.pad >> 8));
+    const bool tall = mend - wu.m0 > 32;
+    const int mh = tall ? wave & 1 : 0, ks = tall ? wave >> 1 : wave, nks = tall ? SMD_W / 2 : SMD_W;
+    const int m0 = wu.m0 + 32 * mh;
+    const bool two_m = mend - m0 > 16, two_n = nend - wu.n0 > 16;
+    v4 acc[2][2];
 #pragma unroll
-      for (int j = 0; j < SM_NPT; ++j) {
-        const int n = wu.n0 + ng * SM_NPT + j;
-        if (n < t0.N && ng * SM_NPT + j < SM_N) {
-          double *cp = Cm + tab[t0.tCN + n];
-          double v = alpha * acc[j];
-          if (beta != 0.0) v += beta * (*cp);
-          *cp = v;
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int g = 0; g < 2; ++g) acc[i][g] = v4{0, 0, 0, 0};
+    // the table entries of the results, long before they are needed
+    const int fr = tall ? ks : wave >> 1;  // the fragment this wave finishes
+    const int64_t cm = tab[t0.tCM + min(m0 + 16 * (fr & 1) + r16, t0.M - 1)];
+    int64_t cn[4];
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+      cn[h] = tab[t0.tCN + min(wu.n0 + 16 * (fr >> 1) + MF<double>::orow(lane, tall ? h : 2 * (wave & 1) + (h & 1)),
+                               t0.N - 1)];
+    const bool share = wu.tend - wu.tbeg < nks;  // few tasks: share each one's k
+    const int kb = share ? 16 * ks : 0, kd = share ? 16 * nks : 16;
+    for (int t = share ? wu.tbeg : wu.tbeg + ks; t < wu.tend; t += share ? 1 : nks) {
+      const GemmTask tk = tasks[t];
+      if (kb >= tk.K) continue;
+      // rows past the block repeat its last one, k past the end is zeroed
+      SmallOperand<AKC> oa;
+      SmallOperand<BKC> ob;
+      oa.init(A + tk.a_off, m0, t0.M - 1, tab + tk.tAM, lane);
+      ob.init(B + tk.b_off, wu.n0, t0.N - 1, tab + tk.tBN, lane);
+      oa.load(kb, tk.K, tab + tk.tAK, two_m, lane);
+      ob.load(kb, tk.K, tab + tk.tBK, two_n, lane);
+      for (int k0 = kb; k0 < tk.K; k0 += kd) {
+        double a[4][2], b[4][2];
+        oa.fragments(a, bufA, lane);
+        ob.fragments(b, bufB, lane);
+        if (k0 + kd < tk.K) {
+          oa.load(k0 + kd, tk.K, tab + tk.tAK, two_m, lane);
+          ob.load(k0 + kd, tk.K, tab + tk.tBK, two_n, lane);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          if (k0 + 4 * s >= tk.K) break;  // uniform
+          const bool kv = k0 + 4 * s + q4 < tk.K;
+#pragma unroll
+          for (int g = 0; g < 2; ++g) {
+            a[s][g] = kv ? a[s][g] : 0.0;
+            b[s][g] = kv ? b[s][g] : 0.0;
+          }
+          acc[0][0] = MF<double>::mma(b[s][0], a[s][0], acc[0][0]);
+          if (two_m) acc[0][1] = MF<double>::mma(b[s][0], a[s][1], acc[0][1]);
+          if (two_n) acc[1][0] = MF<double>::mma(b[s][1], a[s][0], acc[1][0]);
+          if (two_m && two_n) acc[1][1] = MF<double>::mma(b[s][1], a[s][1], acc[1][1]);
         }
       }
     }
+    // sums of the waves of one half of the rows, each wave a part of them
+    __syncthreads();  // every wave is done with its buffers
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[wave][(2 * i + g) * 4 + r][lane] = acc[i][g][r];
+    __syncthreads();
+    // tall: wave (ks, mh) finishes fragment ks of its half; else the wave pair
+    // (2 f, 2 f + 1) the two halves of fragment f
+    const int ig = fr, i = ig >> 1, g = ig & 1;
+    const int m = m0 + 16 * g + r16;
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      const int r = tall ? h : 2 * (wave & 1) + (h & 1);
+      if (!tall && h > 1) break;
+      double v = 0.0;
+      if (tall) {
+#pragma unroll
+        for (int w = 0; w < SMD_W / 2; ++w) v += part[mh + 2 * w][ig * 4 + r][lane];
+      } else {
+#pragma unroll
+        for (int w = 0; w < SMD_W; ++w) v += part[w][ig * 4 + r][lane];
+      }
+      const int n = wu.n0 + 16 * i + MF<double>::orow(lane, r);
+      if (m >= mend || n >= nend) continue;
+      if (wu.slot >= 0) {  // partial tile of a split unit (C is the workspace)
+        C[size_t(wu.slot) * (SM_M * SM_N) + size_t(n - wu.n0) * SM_M + (m - wu.m0)] = v;
+      } else {
+        double *cp = C + t0.c_off + cm + cn[h];
+        v *= alpha;
+        if (beta != 0.0) v += beta * (*cp);
+        *cp = v;
+      }
+    }
+    __syncthreads();  // the sums are read before the next unit's operands
   }
 }
 
@@ -1822,7 +1926,7 @@ constexpr TileCfg kTiles[] = {
     {256, 64, 4, 2, 0.70, 0.55},   // 7: 8 waves
     {64, 256, 2, 4, 0.95, 1.00},   // 8: 8 waves
     {256, 128, 4, 2, 0.60, 0.50},  // 9: 8 waves, wave tile 64x64
-    {SM_M, SM_N, 0, 0, 1.0, 1.0},  // 10: small blocks (FP64 VALU)
+    {SM_M, SM_N, 0, 0, 1.0, 1.0},  // 10: small blocks
     {128, 128, 2, 4, 0.80, 0.85},  // 11: as 6 with 32-deep k stages
     {128, 64, 2, 2, 0.90, 0.95},   // 12: as 1 with 32-deep k stages
     {64, 128, 2, 2, 0.90, 0.95},   // 13: as 2 with 32-deep k stages
@@ -1925,7 +2029,7 @@ const void *kernel_of(int tile, int prec, bool akc, bool bkc, int *block, int ve
     return sk.one ? reinterpret_cast<const void *>(&k_skinny<2, true>)
                   : reinterpret_cast<const void *>(&k_skinny<2, false>);
   }
-  if (tile == kSmall) {  // FP64 on the VALU, FP32 / BF16x3 on the matrix cores
+  if (tile == kSmall) {
     *block = SM_T;
     if (prec == ITX_PREC_F32) {
       if (akc) return bkc ? reinterpret_cast<const void *>(&k_small_f32<true, true>)
@@ -1939,6 +2043,7 @@ const void *kernel_of(int tile, int prec, bool akc, bool bkc, int *block, int ve
       return bkc ? reinterpret_cast<const void *>(&k_small_bf16x3<false, true>)
                  : reinterpret_cast<const void *>(&k_small_bf16x3<false, false>);
     }
+    *block = SMD_T;
     if (akc) return bkc ? reinterpret_cast<const void *>(&k_small<true, true>)
                         : reinterpret_cast<const void *>(&k_small<true, false>);
     return bkc ? reinterpret_cast<const void *>(&k_small<false, true>)
@@ -2287,8 +2392,22 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
   auto finalize = [&](int best, itx_plan **pout) -> int {
     *pout = nullptr;
     if ((best == kDgemm || best == kDgemm2) && !dg_ok) return ITX_ERR_UNSUPPORTED;
-    const int tbm = (best == kSkinny && tinyq) ? SKQ_R * SK_ROWS : kTiles[best].bm;
-    const int tbn = (best == kSkinny) ? std::max(1, maxN) : kTiles[best].bn;
+    const int tbm0 = (best == kSkinny && tinyq) ? SKQ_R * SK_ROWS : kTiles[best].bm;
+    const int tbn0 = (best == kSkinny) ? std::max(1, maxN) : kTiles[best].bn;
+    int tbm = tbm0, tbn = tbn0;
+    if (best == kSmall && prec == ITX_PREC_F64 && !into) {
+      // Smaller units while they leave CUs idle: a unit's k loop is bound by
+      // the matrix cores of one CU (64 x 32 outputs: 32 cycles a k), its loads
+      // by its rows, so two units of half the size take half the time.  One
+      // 128 x 32 block with K = 160: 9.2 us as two units, 5 us as 16.
+      auto count = [&](int bm, int bn) {
+        int64_t n = 0;
+        for (auto &g : groups) n += int64_t((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn);
+        return n;
+      };
+      if (count(64, 32) < cus) tbm = 32;
+      if (count(32, 32) < cus / 2) tbm = tbn = 16;
+    }
     std::vector<WorkUnit> units, red;
     std::vector<double> ucost;
     std::vector<GemmTask> vt;  // device task list (st, or its k-chunks when split)
@@ -2302,17 +2421,22 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
       for (auto &g : groups) {
         double w = 0;
         for (int t = g.tb; t < g.te; ++t) w += double((st[t].K + SM_K - 1) / SM_K);
-        const double tiles = double((g.M + tbm - 1) / tbm) * double((g.N + tbn - 1) / tbn);
+        const double tiles = double((g.M + tbm0 - 1) / tbm0) * double((g.N + tbn0 - 1) / tbn0);
         total += w * tiles;
         maxw = std::max(maxw, w);
       }
       const double target = 2.0 * cus * tile_occupancy(kSmall, prec, akc, bkc);
       const double c = std::max(1.0, std::ceil(total / target));
-      split = maxw > 2.0 * c && total * (SM_M * SM_N) * 8.0 / c < double(size_t(1) << 30);
+      // Units of at least `least` k-chunks: reduced forms two (a one-chunk unit
+      // writes a partial tile for as many bytes as it reads); FP64 eight, one
+      // for each wave of a unit, which share its chunks anyway -- a split
+      // costs a second launch (4 us) where a chunk more costs a trip to memory
+      const int least = prec == ITX_PREC_F64 ? SMD_W : 2;
+      split = maxw > 2.0 * std::max(c, prec == ITX_PREC_F64 ? double(least) : 1.0) && total * (SM_M * SM_N) * 8.0 / c < double(size_t(1) << 30);
       if (split) {
-        // at least two k-chunks per unit: a one-chunk unit writes a
-        // partial tile for as many bytes as it reads
-        const int per = std::max(2, int(c));
+        tbm = tbm0;  // partial tiles are whole
+        tbn = tbn0;
+        const int per = std::max(least, int(c));
         for (auto &g : groups) {
           const int vb = int(vt.size());
           for (int t = g.tb; t < g.te; ++t)
@@ -2328,7 +2452,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
             for (int n0 = 0; n0 < g.N; n0 += tbn) {
               const int s0 = nslots;
               for (int a = vb; a < ve; a += per) {
-                units.push_back({a, std::min(ve, a + per), m0, n0, nslots++, 0});
+                units.push_back({a, std::min(ve, a + per), m0, n0, nslots++, tbm | tbn << 8});
                 ucost.push_back(double(std::min(ve, a + per) - a));
               }
               red.push_back({vb, s0, m0, n0, nslots, 0});
@@ -2349,7 +2473,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
           for (int sn = 0; sn < tn; sn += SUPN)
             for (int im = sm; im < std::min(tm, sm + SUPM); ++im)
               for (int in = sn; in < std::min(tn, sn + SUPN); ++in) {
-                units.push_back({g.tb, g.te, im * tbm, in * tbn, -1, 0});
+                units.push_back({g.tb, g.te, im * tbm, in * tbn, -1, best == kSmall ? tbm | tbn << 8 : 0});
                 ucost.push_back(g.ksum);
               }
       }
