@@ -16,6 +16,7 @@
 //   OpenMP path groups by output block for the same reason,
 //   itdata/qutil.h:271-349).
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <fstream>
@@ -27,6 +28,7 @@
 #include <queue>
 #include <sstream>
 #include <type_traits>
+#include <utility>
 
 #include <unordered_map>
 #include "itx_internal.h"
@@ -179,21 +181,8 @@ __global__ __launch_bounds__(64 * GM * GN) void k_gemm(const double *__restrict_
   // Units are spread so that each XCD (blocks b with equal b % 8 land on
   // the same XCD) walks a contiguous chunk of the unit list: neighbouring
   // tiles share A rows / B columns, which then stay in that XCD's L2.
-  const int G = gridDim.x, b = blockIdx.x;
-  int ustart, uend, ustep;
-  if (G % 8 == 0 && nunits >= G) {
-    const int nb = G / 8, x = b % 8, lb = b / 8;
-    const int chunk = (nunits + 7) / 8;
-    ustart = x * chunk + lb;
-    uend = min(nunits, (x + 1) * chunk);
-    ustep = nb;
-  } else {
-    ustart = b;
-    uend = nunits;
-    ustep = G;
-  }
 
-  for (int u = ustart; u < uend; u += ustep) {
+  for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
     const WorkUnit wu = units[u];
     v4 acc[FN][FM];
 #pragma unroll
@@ -289,35 +278,32 @@ __global__ __launch_bounds__(64 * GM * GN) void k_gemm(const double *__restrict_
   }
 }
 
-// ---- FP64 register-pipelined tile ----------------------------------------
-// 128 x 128 C tile, four waves of 64 x 64 (4 x 4 fragments of the f64
-// 16x16x4 MFMA), 16-deep k stages, for operands contiguous along k in
-// aligned pairs (the plan's vector-load condition).  A thread loads 16-byte
-// k pairs; an LDS row holds the 16 k of a stage contiguously (pitch 18
-// doubles: the 16 rows that a quarter-wave reads land on distinct 16-byte
-// bank groups), and a lane reads the 4 consecutive k of its fragment row
-// with two 16-byte reads.  MFMA s (0..3) of a stage takes k = 4q + s from
-// the lanes of quarter q, so every k of the stage enters once.
-// Pipeline (one barrier per stage): while the 64 MFMAs of stage n run from
+// ---- register-pipelined tiles ---------------------------------------------
+// FP64: k_pipe below.  FP32 (k_dgemm): 128 x 128 C tile, four waves of 64 x
+// 64 (4 x 4 fragments of the f32 16x16x4 MFMA), 16-deep k stages, for
+// operands contiguous along k in aligned pairs (the plan's vector-load
+// condition).  A thread loads 16-byte k pairs and rounds them to FP32 at the
+// LDS store; an LDS row holds the 16 k of a stage contiguously (pitch 18
+// doubles, 20 floats: the 16 rows that a quarter-wave reads land on distinct
+// 16-byte bank groups), and a lane reads the 4 consecutive k of its fragment
+// row with 16-byte reads.  MFMA s (0..3) of a stage takes k = 4q + s from the
+// lanes of quarter q, so every k of the stage enters once.
+// Pipeline (one barrier per stage): while the MFMAs of stage n run from
 // registers, the operands of stage n+1 are read from LDS, stage n+2 is
 // stored to LDS from the load registers, and the global loads of stage n+4
 // are issued into those registers (two register sets: loads have two
-// stages, about 8000 MFMA cycles, to arrive).
-// FP32 form: the same pipeline with operands rounded to FP32 at the LDS
-// store, LDS rows of 20 floats (80 bytes: again 16 distinct bank groups),
-// one 16-byte read per fragment row and the f32 16x16x4 MFMA.
+// stages to arrive).
 constexpr int DG_BK = 16, DG_NT = 256;
 template <typename T>
 struct DgCfg;
 template <>
 struct DgCfg<double> {
-  static constexpr int P = 18;   // LDS row pitch (elements)
-  static constexpr int RD = 16;  // LDS reads per stage and lane
+  static constexpr int P = 18;  // LDS row pitch (elements)
 };
 template <>
 struct DgCfg<float> {
   static constexpr int P = 20;
-  static constexpr int RD = 8;
+  static constexpr int RD = 8;  // LDS reads per stage and lane
 };
 
 struct DgRegs {  // one stage of one operand in flight: four 16-byte pairs
@@ -355,15 +341,6 @@ struct DgLoader {  // one operand: 128 rows x 16 k per stage, four 16-byte loads
       r.g[2 * p + 1] = v.y;
     }
   }
-  __device__ __forceinline__ void store(double *__restrict__ s, const DgRegs &r) const {
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      double2 v;
-      v.x = r.ok[p] ? r.g[2 * p] : 0.0;
-      v.y = r.ok[p] ? r.g[2 * p + 1] : 0.0;
-      *reinterpret_cast<double2 *>(s + (lr + 32 * p) * DgCfg<double>::P + 2 * lc) = v;
-    }
-  }
   __device__ __forceinline__ void store(float *__restrict__ s, const DgRegs &r) const {
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
@@ -378,31 +355,9 @@ struct DgLoader {  // one operand: 128 rows x 16 k per stage, four 16-byte loads
 template <typename T>
 struct DgFrag;
 template <>
-struct DgFrag<double> {  // a lane's operands of one stage: 4 fragments x 4 k, for A and for B
-  double2 a[4][2], b[4][2];
-};
-template <>
-struct DgFrag<float> {
+struct DgFrag<float> {  // a lane's operands of one stage: 4 fragments x 4 k, for A and for B
   float4 a[4], b[4];
 };
-
-__device__ __forceinline__ void dg_read(DgFrag<double> &f, const double *__restrict__ as,
-                                        const double *__restrict__ bs, int wm, int wn, int lane) {
-  const int r = lane & 15, q = lane >> 4;
-  constexpr int P = DgCfg<double>::P;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const double *pa = as + (wm * 64 + j * 16 + r) * P + 4 * q;
-    f.a[j][0] = *reinterpret_cast<const double2 *>(pa);
-    f.a[j][1] = *reinterpret_cast<const double2 *>(pa + 2);
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const double *pb = bs + (wn * 64 + i * 16 + r) * P + 4 * q;
-    f.b[i][0] = *reinterpret_cast<const double2 *>(pb);
-    f.b[i][1] = *reinterpret_cast<const double2 *>(pb + 2);
-  }
-}
 
 __device__ __forceinline__ void dg_read(DgFrag<float> &f, const float *__restrict__ as, const float *__restrict__ bs,
                                         int wm, int wn, int lane) {
@@ -413,8 +368,6 @@ __device__ __forceinline__ void dg_read(DgFrag<float> &f, const float *__restric
 #pragma unroll
   for (int i = 0; i < 4; ++i) f.b[i] = *reinterpret_cast<const float4 *>(bs + (wn * 64 + i * 16 + r) * P + 4 * q);
 }
-
-using dv4 = MF<double>::v4;
 
 __device__ __forceinline__ double dg_k(const double2 (&x)[2], int s) {
   return s == 0 ? x[0].x : s == 1 ? x[0].y : s == 2 ? x[1].x : x[1].y;
@@ -445,21 +398,8 @@ __global__ __launch_bounds__(DG_NT) void k_dgemm(const double *__restrict__ A, c
   const int wm = wave & 1, wn = wave >> 1;
 
   // XCD-contiguous unit chunks (as in k_gemm)
-  const int G = gridDim.x, b = blockIdx.x;
-  int ustart, uend, ustep;
-  if (G % 8 == 0 && nunits >= G) {
-    const int nb = G / 8, x = b % 8, lb = b / 8;
-    const int chunk = (nunits + 7) / 8;
-    ustart = x * chunk + lb;
-    uend = min(nunits, (x + 1) * chunk);
-    ustep = nb;
-  } else {
-    ustart = b;
-    uend = nunits;
-    ustep = G;
-  }
 
-  for (int u = ustart; u < uend; u += ustep) {
+  for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
     const WorkUnit wu = units[u];
     v4 acc[4][4];
 #pragma unroll
@@ -669,21 +609,8 @@ __global__ __launch_bounds__(DG_NT, 2) void k_dgemm2(const double *__restrict__ 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
 
-  const int G = gridDim.x, b = blockIdx.x;
-  int ustart, uend, ustep;
-  if (G % 8 == 0 && nunits >= G) {
-    const int nb = G / 8, x = b % 8, lb = b / 8;
-    const int chunk = (nunits + 7) / 8;
-    ustart = x * chunk + lb;
-    uend = min(nunits, (x + 1) * chunk);
-    ustep = nb;
-  } else {
-    ustart = b;
-    uend = nunits;
-    ustep = G;
-  }
 
-  for (int u = ustart; u < uend; u += ustep) {
+  for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
     const WorkUnit wu = units[u];
     v4 acc[4][4];
 #pragma unroll
@@ -783,6 +710,266 @@ __global__ __launch_bounds__(DG_NT, 2) void k_dgemm2(const double *__restrict__ 
           if (mv[j] && nv[i][r]) {
             const int64_t ad = cm[j] + cn[i][r];
             double v = alpha * double(acc[i][j][r]);
+            if (beta != 0.0) v += beta * Cb[ad];
+            Cb[ad] = v;
+          }
+        }
+  }
+}
+
+// ---- FP64 register-pipelined tiles of any size, layout and alignment ---------
+// The pipeline of k_dgemm (k order 4q + s) with (32 FM) x (32 FN) tiles.  Each
+// operand is loaded in aligned k pairs (V = 2, both operands), single elements
+// with the lanes along k (V = 1) or along the rows (V = 0: a wave takes four k
+// of a stage, so an operand contiguous along its rows coalesces).  Rows and
+// columns past the block load its last one and are not stored, so only the k
+// past the end has to be zeroed, in the last stages: in the steady state no
+// load or store has a condition, and they sit between the MFMAs by schedule
+// groups.  128 x 128 (FM = FN = 4): a stage is 1.87 us, 1.7 of it MFMA.
+// 64 x 64: four times the units for products that leave CUs idle with the
+// larger tile, two workgroups per CU.  Dense chain, first and last stage, from
+// k_gemm / k_dgemm: chi = 1024 773 + 728 to 624 + 593 us (the matrix cores
+// need 563 each), chi = 512 136 + 148 to 100 + 96, chi = 255 28 + 43 to 26.5 +
+// 28.5.
+template <int ROWS, int V>
+struct PipeLoader {  // one operand: ROWS x 16 k per stage; V = 0: lanes along the rows, a wave's 4 k each
+  static constexpr int LK = V ? DG_BK / (V ? V : 1) : 4, RS = DG_NT / LK, NP = ROWS / RS, NK = V ? 1 : 4;
+  static constexpr int NR = ROWS / 16;                                      // doubles of a thread
+  static constexpr int NLD = V == 2 ? NR / 2 : NR, NST = V == 1 ? NR : NR / 2;  // loads, LDS stores
+  int64_t roff[NP];
+  int64_t ko[2][NK];  // k offsets of the next two stages to load (slot = stage & 1)
+  int lr, lc;
+  __device__ __forceinline__ void init(int tid, int row0, int R, const int64_t *__restrict__ tabR) {
+    lc = V ? tid % LK : 4 * __builtin_amdgcn_readfirstlane(tid >> 6);
+    lr = V ? tid / LK : tid & 63;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) roff[p] = tabR[min(row0 + lr + RS * p, R - 1)];
+  }
+  __device__ __forceinline__ void fetch_k(int k0, int K, const int64_t *__restrict__ tabK, int slot) {
+    if constexpr (V) {
+      ko[slot][0] = tabK[min(k0 + V * lc, K - V)];
+    } else {
+#pragma unroll
+      for (int c = 0; c < NK; ++c) ko[slot][c] = tabK[min(k0 + lc + c, K - 1)];
+    }
+  }
+  __device__ __forceinline__ void load(const double *__restrict__ base, double (&r)[NR], int slot) const {
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      if constexpr (V == 2) {
+        const double2 v = *reinterpret_cast<const double2 *>(base + roff[p] + ko[slot][0]);
+        r[2 * p] = v.x;
+        r[2 * p + 1] = v.y;
+      } else {
+#pragma unroll
+        for (int c = 0; c < NK; ++c) r[NK * p + c] = (base + ko[slot][c])[roff[p]];
+      }
+    }
+  }
+  // k0: first k of the stage (TAIL: its k past K are zeroed)
+  template <bool TAIL>
+  __device__ __forceinline__ void store(double *__restrict__ s, const double (&r)[NR], int k0, int K) const {
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      double *d = s + (lr + RS * p) * DgCfg<double>::P;
+      if constexpr (V == 1) {
+        d[lc] = !TAIL || k0 + lc < K ? r[p] : 0.0;
+      } else if constexpr (V == 2) {
+        const bool ok = !TAIL || k0 + 2 * lc < K;
+        *reinterpret_cast<double2 *>(d + 2 * lc) = ok ? double2{r[2 * p], r[2 * p + 1]} : double2{0.0, 0.0};
+      } else {
+#pragma unroll
+        for (int c = 0; c < 4; c += 2) {
+          double2 v;
+          v.x = !TAIL || k0 + lc + c < K ? r[4 * p + c] : 0.0;
+          v.y = !TAIL || k0 + lc + c + 1 < K ? r[4 * p + c + 1] : 0.0;
+          *reinterpret_cast<double2 *>(d + lc + c) = v;
+        }
+      }
+    }
+  }
+};
+
+template <int F>
+struct PipeFrag {  // one operand of a stage: F fragments x 4 k
+  double2 x[F][2];
+  __device__ __forceinline__ void read(const double *__restrict__ s, int row0, int lane) {
+#pragma unroll
+    for (int j = 0; j < F; ++j) {
+      const double *p = s + (row0 + j * 16 + (lane & 15)) * DgCfg<double>::P + 4 * (lane >> 4);
+      x[j][0] = *reinterpret_cast<const double2 *>(p);
+      x[j][1] = *reinterpret_cast<const double2 *>(p + 2);
+    }
+  }
+};
+
+template <int FM, int FN, int VA, int VB>
+__global__ __launch_bounds__(DG_NT, FM * FN <= 4 ? 2 : 1) void k_pipe(
+    const double *__restrict__ A, const double *__restrict__ B, double *__restrict__ C,
+    const GemmTask *__restrict__ tasks, const WorkUnit *__restrict__ units, int nunits, const int64_t *__restrict__ tab,
+    double alpha, double beta) {
+  using v4 = MF<double>::v4;
+  constexpr int P = DgCfg<double>::P, BM = 32 * FM, BN = 32 * FN, NM = FM * FN;
+  using LA = PipeLoader<BM, VA>;
+  using LB = PipeLoader<BN, VB>;
+  __shared__ __align__(16) double As[2][BM * P];
+  __shared__ __align__(16) double Bs[2][BN * P];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = (wave & 1) * 16 * FM, wn = (wave >> 1) * 16 * FN;
+
+  for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
+    const WorkUnit wu = units[u];
+    v4 acc[FN][FM];
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+      for (int j = 0; j < FM; ++j) acc[i][j] = v4{0, 0, 0, 0};
+
+    for (int t = wu.tbeg; t < wu.tend; ++t) {
+      const GemmTask tk = tasks[t];
+      if (tk.K <= 0) continue;
+      LA la;
+      LB lb;
+      la.init(tid, wu.m0, tk.M, tab + tk.tAM);
+      lb.init(tid, wu.n0, tk.N, tab + tk.tBN);
+      const double *Ab = A + tk.a_off;
+      const double *Bb = B + tk.b_off;
+      const int64_t *tAK = tab + tk.tAK;
+      const int64_t *tBK = tab + tk.tBK;
+      const int K = tk.K, S = (K + DG_BK - 1) / DG_BK;
+      double ra0[LA::NR], rb0[LB::NR], ra1[LA::NR], rb1[LB::NR];  // load register sets
+#define ITX_PIPE_LOAD(st, ra, rb, slot)                   \
+  {                                                       \
+    la.load(Ab, ra, slot);                                \
+    lb.load(Bb, rb, slot);                                \
+    la.fetch_k(((st) + 2) * DG_BK, K, tAK, slot);         \
+    lb.fetch_k(((st) + 2) * DG_BK, K, tBK, slot);         \
+  }
+#define ITX_PIPE_STORE(tail, st, ra, rb)                                  \
+  {                                                                       \
+    la.template store<tail>(As[(st) & 1], ra, (st) * DG_BK, K);           \
+    lb.template store<tail>(Bs[(st) & 1], rb, (st) * DG_BK, K);           \
+  }
+      PipeFrag<FM> fa0, fa1;
+      PipeFrag<FN> fb0, fb1;
+      auto mfma = [&](const PipeFrag<FM> &fa, const PipeFrag<FN> &fb, int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < FN; ++i)
+#pragma unroll
+          for (int j = 0; j < FM; ++j) acc[i][j] = MF<double>::mma(dg_k(fb.x[i], s), dg_k(fa.x[j], s), acc[i][j]);
+      };
+      la.fetch_k(0, K, tAK, 0);
+      lb.fetch_k(0, K, tBK, 0);
+      la.fetch_k(DG_BK, K, tAK, 1);
+      lb.fetch_k(DG_BK, K, tBK, 1);
+      ITX_PIPE_LOAD(0, ra0, rb0, 0)
+      if (S > 1) ITX_PIPE_LOAD(1, ra1, rb1, 1)
+      __syncthreads();  // the previous task's LDS reads are done
+      ITX_PIPE_STORE(true, 0, ra0, rb0)
+      if (S > 2) ITX_PIPE_LOAD(2, ra0, rb0, 0)
+      __syncthreads();
+      fa0.read(As[0], wm, lane);
+      fb0.read(Bs[0], wn, lane);
+      if (S > 1) ITX_PIPE_STORE(true, 1, ra1, rb1)
+      if (S > 3) ITX_PIPE_LOAD(3, ra1, rb1, 1)
+      __syncthreads();
+      // stage n: read stage n+1, store n+2, load n+4 around its MFMAs
+#define ITX_PIPE_STEP(n, fa, fb, na, nb, ra, rb, slot)            \
+  {                                                               \
+    if ((n) + 1 < S) {                                            \
+      na.read(As[((n) + 1) & 1], wm, lane);                       \
+      nb.read(Bs[((n) + 1) & 1], wn, lane);                       \
+    }                                                             \
+    mfma(fa, fb, 0);                                              \
+    __builtin_amdgcn_sched_barrier(0);                            \
+    if ((n) + 2 < S) ITX_PIPE_STORE(true, (n) + 2, ra, rb)        \
+    if ((n) + 4 < S) ITX_PIPE_LOAD((n) + 4, ra, rb, slot)         \
+    __builtin_amdgcn_sched_barrier(0);                            \
+    mfma(fa, fb, 1);                                              \
+    mfma(fa, fb, 2);                                              \
+    mfma(fa, fb, 3);                                              \
+    __builtin_amdgcn_sched_barrier(0);                            \
+    __syncthreads();                                              \
+  }
+      // steady state (n + 4 < S): no conditions, the other instructions
+      // placed between the MFMAs
+#define ITX_PIPE_BODY(n, fa, fb, na, nb, ra, rb, id)                                             \
+  {                                                                                              \
+    na.read(As[((n) + 1) & 1], wm, lane);                                                        \
+    nb.read(Bs[((n) + 1) & 1], wn, lane);                                                        \
+    mfma(fa, fb, 0);                                                                             \
+    for (int g_ = 0; g_ < NM; ++g_) {                                                            \
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, id);                                        \
+      __builtin_amdgcn_sched_group_barrier(0x100, (2 * (FM + FN) + NM - 1) / NM, id);            \
+    }                                                                                            \
+    __builtin_amdgcn_sched_barrier(0);                                                           \
+    ITX_PIPE_STORE(false, (n) + 2, ra, rb)                                                       \
+    mfma(fa, fb, 1);                                                                             \
+    for (int g_ = 0; g_ < NM; ++g_) {                                                            \
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, id);                                        \
+      __builtin_amdgcn_sched_group_barrier(0x200, (LA::NST + LB::NST + NM - 1) / NM, id);        \
+    }                                                                                            \
+    __builtin_amdgcn_sched_barrier(0);                                                           \
+    ITX_PIPE_LOAD((n) + 4, ra, rb, id)                                                           \
+    mfma(fa, fb, 2);                                                                             \
+    for (int g_ = 0; g_ < NM; ++g_) {                                                            \
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, id);                                        \
+      __builtin_amdgcn_sched_group_barrier(0x006, 8, id);                                        \
+      __builtin_amdgcn_sched_group_barrier(0x020, (LA::NLD + LB::NLD + 2 + NM - 1) / NM, id);    \
+    }                                                                                            \
+    __builtin_amdgcn_sched_barrier(0);                                                           \
+    mfma(fa, fb, 3);                                                                             \
+    __builtin_amdgcn_sched_barrier(0);                                                           \
+    __syncthreads();                                                                             \
+  }
+      int n = 0;
+      for (; n + 5 < S; n += 2) {
+        ITX_PIPE_BODY(n, fa0, fb0, fa1, fb1, ra0, rb0, 0)
+        ITX_PIPE_BODY(n + 1, fa1, fb1, fa0, fb0, ra1, rb1, 1)
+      }
+      for (; n + 1 < S; n += 2) {
+        ITX_PIPE_STEP(n, fa0, fb0, fa1, fb1, ra0, rb0, 0)
+        ITX_PIPE_STEP(n + 1, fa1, fb1, fa0, fb0, ra1, rb1, 1)
+      }
+      if (n < S) ITX_PIPE_STEP(n, fa0, fb0, fa1, fb1, ra0, rb0, 0)
+#undef ITX_PIPE_BODY
+#undef ITX_PIPE_STEP
+#undef ITX_PIPE_STORE
+#undef ITX_PIPE_LOAD
+    }
+
+    if (wu.slot >= 0) {  // partial tile of a split unit (C is the workspace)
+      double *Pt = C + size_t(wu.slot) * (BM * BN);
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int j = 0; j < FM; ++j)
+            Pt[(wn + i * 16 + MF<double>::orow(lane, r)) * BM + wm + j * 16 + (lane & 15)] = acc[i][j][r];
+      continue;
+    }
+    const GemmTask t0 = tasks[wu.tbeg];
+    const int64_t *tCM = tab + t0.tCM;
+    const int64_t *tCN = tab + t0.tCN;
+    double *Cb = C + t0.c_off;
+    int64_t cm[FM], cn[FN][4];
+#pragma unroll
+    for (int j = 0; j < FM; ++j) cm[j] = tCM[min(wu.m0 + wm + j * 16 + (lane & 15), t0.M - 1)];
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) cn[i][r] = tCN[min(wu.n0 + wn + i * 16 + MF<double>::orow(lane, r), t0.N - 1)];
+#pragma unroll
+    for (int j = 0; j < FM; ++j)
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = wu.m0 + wm + j * 16 + (lane & 15), n = wu.n0 + wn + i * 16 + MF<double>::orow(lane, r);
+          if (m < t0.M && n < t0.N) {
+            const int64_t ad = cm[j] + cn[i][r];
+            double v = alpha * acc[i][j][r];
             if (beta != 0.0) v += beta * Cb[ad];
             Cb[ad] = v;
           }
@@ -963,21 +1150,8 @@ __global__ __launch_bounds__(64 * GM * GN) void k_gemm3(const double *__restrict
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave % GM, wn = wave / GM;
-  const int G = gridDim.x, b = blockIdx.x;
-  int ustart, uend, ustep;
-  if (G % 8 == 0 && nunits >= G) {
-    const int nb = G / 8, x = b % 8, lb = b / 8;
-    const int chunk = (nunits + 7) / 8;
-    ustart = x * chunk + lb;
-    uend = min(nunits, (x + 1) * chunk);
-    ustep = nb;
-  } else {
-    ustart = b;
-    uend = nunits;
-    ustep = G;
-  }
 
-  for (int u = ustart; u < uend; u += ustep) {
+  for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
     const WorkUnit wu = units[u];
     v4 acc[FN][FM];
 #pragma unroll
@@ -1205,11 +1379,13 @@ __global__ __launch_bounds__(SK_ROWS) void k_skinny_q(const double *__restrict__
     const GemmTask t0 = tasks[wu.tbeg];
     const int N = t0.N, M = t0.M;
     int mr[SKQ_R];
+    int64_t cr[SKQ_R];
     bool in[SKQ_R];
 #pragma unroll
     for (int h = 0; h < SKQ_R; ++h) {
       mr[h] = wu.m0 + tid + h * SK_ROWS;
       in[h] = mr[h] < M;
+      cr[h] = t0.c_off + tab[t0.tCM + min(mr[h], M - 1)];
     }
     double acc[SKQ_R][SKQ_N];
 #pragma unroll
@@ -1220,7 +1396,27 @@ __global__ __launch_bounds__(SK_ROWS) void k_skinny_q(const double *__restrict__
       // the next tasks whose stacked B rows fit the LDS tile
       int te = tc, kt = 0;
       while (te < wu.tend && kt + tasks[te].K <= SK_K) kt += tasks[te++].K;
-      __syncthreads();  // the previous chunk's B rows are no longer read
+      double av[SKQ_R][SKQ_G][SKQ_K];
+      int kk[SKQ_G];
+      auto fetch = [&](int t) {
+#pragma unroll
+        for (int q = 0; q < SKQ_G; ++q) {
+          kk[q] = 0;
+          if (t + q < te) {
+            const GemmTask tk = tasks[t + q];
+            kk[q] = tk.K;
+            const int64_t *tAK = tab + tk.tAK;
+#pragma unroll
+            for (int h = 0; h < SKQ_R; ++h) {
+              const double *Ar = A + tk.a_off + tab[tk.tAM + min(mr[h], M - 1)];
+#pragma unroll
+              for (int j = 0; j < SKQ_K; ++j) av[h][q][j] = (j < tk.K && in[h]) ? Ar[tAK[j]] : 0.0;
+            }
+          }
+        }
+      };
+      fetch(tc);  // on its way while B is staged
+      lds_barrier();  // the previous chunk's B rows are no longer read
       for (int t = tc, kb = 0; t < te; ++t) {
         const GemmTask tk = tasks[t];
         for (int x = tid; x < tk.K * N; x += SK_ROWS) {
@@ -1229,50 +1425,33 @@ __global__ __launch_bounds__(SK_ROWS) void k_skinny_q(const double *__restrict__
         }
         kb += tk.K;
       }
-      __syncthreads();
-      if (in[0]) {
-        for (int t = tc, kb = 0; t < te; t += SKQ_G) {
-          double av[SKQ_R][SKQ_G][SKQ_K];
-          int kk[SKQ_G];
+      lds_barrier();
+      for (int t = tc, kb = 0; t < te;) {
 #pragma unroll
-          for (int q = 0; q < SKQ_G; ++q) {
-            kk[q] = 0;
-            if (t + q < te) {
-              const GemmTask tk = tasks[t + q];
-              kk[q] = tk.K;
-              const int64_t *tAK = tab + tk.tAK;
+        for (int q = 0; q < SKQ_G; ++q) {
 #pragma unroll
-              for (int h = 0; h < SKQ_R; ++h) {
-                const double *Ar = A + tk.a_off + tab[tk.tAM + (in[h] ? mr[h] : mr[0])];
+          for (int j = 0; j < SKQ_K; ++j) {
+            if (j < kk[q]) {
 #pragma unroll
-                for (int j = 0; j < SKQ_K; ++j) av[h][q][j] = (j < tk.K && in[h]) ? Ar[tAK[j]] : 0.0;
-              }
+              for (int n = 0; n < SKQ_N; ++n)
+                if (n < N) {
+                  const double bv = Bs[(kb + j) * SKQ_N + n];
+#pragma unroll
+                  for (int h = 0; h < SKQ_R; ++h) acc[h][n] += av[h][q][j] * bv;
+                }
             }
           }
-#pragma unroll
-          for (int q = 0; q < SKQ_G; ++q) {
-#pragma unroll
-            for (int j = 0; j < SKQ_K; ++j) {
-              if (j < kk[q]) {
-#pragma unroll
-                for (int n = 0; n < SKQ_N; ++n)
-                  if (n < N) {
-                    const double bv = Bs[(kb + j) * SKQ_N + n];
-#pragma unroll
-                    for (int h = 0; h < SKQ_R; ++h) acc[h][n] += av[h][q][j] * bv;
-                  }
-              }
-            }
-            kb += kk[q];
-          }
+          kb += kk[q];
         }
+        t += SKQ_G;
+        if (t < te) fetch(t);
       }
       tc = te;
     }
 #pragma unroll
     for (int h = 0; h < SKQ_R; ++h) {
       if (in[h]) {
-        double *Cm = C + t0.c_off + tab[t0.tCM + mr[h]];
+        double *Cm = C + cr[h];
         const int64_t *tCN = tab + t0.tCN;
 #pragma unroll
         for (int n = 0; n < SKQ_N; ++n) {
@@ -1666,6 +1845,7 @@ static_assert(SM_T_RED == SM_T, "reduction pass block size");
 // Reduction pass of split plans: unit u = {task (for C's tables), first
 // slot, m0, n0, end slot}; C tile = alpha * (sum of the slots in order)
 // + beta * C.  A is the workspace; deterministic (fixed summation order).
+template <int TM, int TN>
 __global__ __launch_bounds__(SM_T) void k_reduce_tiles(const double *__restrict__ A,
                                                        const double *__restrict__ B, double *__restrict__ C,
                                                        const GemmTask *__restrict__ tasks,
@@ -1673,25 +1853,25 @@ __global__ __launch_bounds__(SM_T) void k_reduce_tiles(const double *__restrict_
                                                        const int64_t *__restrict__ tab, double alpha,
                                                        double beta) {
   (void)B;
-  // one item = one tile x one slice of SM_T of its SM_M * SM_N elements;
+  // one item = one tile x one slice of SM_T of its elements;
   // four independent partial sums keep several loads in flight
-  constexpr int PARTS = SM_M * SM_N / SM_T;
+  constexpr int PARTS = TM * TN / SM_T;
   for (int w = blockIdx.x; w < nunits * PARTS; w += gridDim.x) {
     const WorkUnit ru = units[w / PARTS];
     const GemmTask t0 = tasks[ru.tbeg];
     const int e = (w % PARTS) * SM_T + threadIdx.x;
-    const int n = e / SM_M, m = e - n * SM_M;
+    const int n = e / TM, m = e - n * TM;
     if (ru.m0 + m >= t0.M || ru.n0 + n >= t0.N) continue;
     const double *src = A + e;
     double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
     int q = ru.tend;
     for (; q + 4 <= ru.slot; q += 4) {
-      s0 += src[size_t(q) * (SM_M * SM_N)];
-      s1 += src[size_t(q + 1) * (SM_M * SM_N)];
-      s2 += src[size_t(q + 2) * (SM_M * SM_N)];
-      s3 += src[size_t(q + 3) * (SM_M * SM_N)];
+      s0 += src[size_t(q) * (TM * TN)];
+      s1 += src[size_t(q + 1) * (TM * TN)];
+      s2 += src[size_t(q + 2) * (TM * TN)];
+      s3 += src[size_t(q + 3) * (TM * TN)];
     }
-    for (; q < ru.slot; ++q) s0 += src[size_t(q) * (SM_M * SM_N)];
+    for (; q < ru.slot; ++q) s0 += src[size_t(q) * (TM * TN)];
     const double s = (s0 + s1) + (s2 + s3);
     double *cp = C + t0.c_off + tab[t0.tCM + ru.m0 + m] + tab[t0.tCN + ru.n0 + n];
     double v = alpha * s;
@@ -1910,34 +2090,38 @@ void colmajor_strides(int r, const int64_t *d, int64_t *s) {
   }
 }
 
-// MFMA tiles (BM x BN with GM x GN waves) and the small-block VALU path.
+// MFMA tiles (BM x BN with GM x GN waves), the skinny and the small-block kernels.
 struct TileCfg {
   int bm, bn, gm, gn;
-  double eff64, eff32;  // relative per-CU efficiency (MI355X measurements)
+  double eff32;  // relative per-CU efficiency of the reduced forms (MI355X measurements)
 };
 constexpr TileCfg kTiles[] = {
-    {128, 128, 2, 2, 0.55, 0.70},  // 0
-    {128, 64, 2, 2, 0.92, 1.00},   // 1
-    {64, 128, 2, 2, 0.92, 0.95},   // 2
-    {64, 64, 2, 2, 1.00, 0.95},    // 3
-    {32, 32, 2, 2, 0.50, 0.45},    // 4
-    {SK_ROWS, SK_N, 0, 0, 1.0, 1.0},  // 5: skinny (FP64 VALU, large M)
-    {128, 128, 2, 4, 0.80, 0.85},  // 6: 8 waves
-    {256, 64, 4, 2, 0.70, 0.55},   // 7: 8 waves
-    {64, 256, 2, 4, 0.95, 1.00},   // 8: 8 waves
-    {256, 128, 4, 2, 0.60, 0.50},  // 9: 8 waves, wave tile 64x64
-    {SM_M, SM_N, 0, 0, 1.0, 1.0},  // 10: small blocks
-    {128, 128, 2, 4, 0.80, 0.85},  // 11: as 6 with 32-deep k stages
-    {128, 64, 2, 2, 0.90, 0.95},   // 12: as 1 with 32-deep k stages
-    {64, 128, 2, 2, 0.90, 0.95},   // 13: as 2 with 32-deep k stages
-    {128, 128, 2, 2, 1.15, 0.85},  // 14: register-pipelined (k_dgemm), k-contiguous pairs only
-    {128, 128, 2, 2, 1.10, 0.85},  // 15: as 14, two workgroups per CU (k_dgemm2)
+    {128, 128, 2, 2, 0.70},  // 0
+    {128, 64, 2, 2, 1.00},   // 1
+    {64, 128, 2, 2, 0.95},   // 2
+    {64, 64, 2, 2, 0.95},    // 3
+    {32, 32, 2, 2, 0.45},    // 4
+    {SK_ROWS, SK_N, 0, 0, 1.0},  // 5: skinny (large M)
+    {128, 128, 2, 4, 0.85},  // 6: 8 waves
+    {256, 64, 4, 2, 0.55},   // 7: 8 waves
+    {64, 256, 2, 4, 1.00},   // 8: 8 waves
+    {256, 128, 4, 2, 0.50},  // 9: 8 waves, wave tile 64x64
+    {SM_M, SM_N, 0, 0, 1.0},  // 10: small blocks
+    {128, 128, 2, 4, 0.85},  // 11: as 6 with 32-deep k stages
+    {128, 64, 2, 2, 0.95},   // 12: as 1 with 32-deep k stages
+    {64, 128, 2, 2, 0.95},   // 13: as 2 with 32-deep k stages
+    {128, 128, 2, 2, 0.85},  // 14: FP32 register-pipelined (k_dgemm); FP64 as 17; k-contiguous pairs only
+    {128, 128, 2, 2, 0.85},  // 15: as 14, FP32 two workgroups per CU (k_dgemm2)
+    {64, 64, 2, 2, 0.0},     // 16: FP64 register-pipelined (k_pipe)
+    {128, 128, 2, 2, 0.0},   // 17: likewise
 };
-constexpr int kNumTiles = 16;
+constexpr int kNumTiles = 18;
+constexpr int kPipe64 = 16, kPipe128 = 17;
 constexpr int kDgemm = 14, kDgemm2 = 15;
 constexpr int kSkinny = 5;
 static_assert(kSkinny == kSkinnyTile, "tile index of the skinny path");
 constexpr int kSmall = 10;
+constexpr int kXcds = 8;
 constexpr int kSkinnyOcc = 3, kSkinnyQOcc = 4;
 
 // Kernel instantiation of a tile shape, operand layout and form.  All
@@ -1986,6 +2170,14 @@ const void *gemm3_fn_tile(int tile, bool akc, bool bkc, bool vec, bool split) {
   }
 }
 
+template <int F>
+const void *pipe_fn(bool akc, bool bkc, bool vec) {
+  if (akc && bkc && vec) return reinterpret_cast<const void *>(&k_pipe<F, F, 2, 2>);
+  if (akc)
+    return bkc ? reinterpret_cast<const void *>(&k_pipe<F, F, 1, 1>) : reinterpret_cast<const void *>(&k_pipe<F, F, 1, 0>);
+  return bkc ? reinterpret_cast<const void *>(&k_pipe<F, F, 0, 1>) : reinterpret_cast<const void *>(&k_pipe<F, F, 0, 0>);
+}
+
 template <typename T>
 const void *gemm_fn_tile(int tile, bool akc, bool bkc, bool vec) {
   switch (tile) {
@@ -2000,12 +2192,20 @@ const void *gemm_fn_tile(int tile, bool akc, bool bkc, bool vec) {
     case 11: return gemm_fn<T, 128, 128, 2, 4, 32>(akc, bkc, vec);
     case 12: return gemm_fn<T, 128, 64, 2, 2, 32>(akc, bkc, vec);
     case 13: return gemm_fn<T, 64, 128, 2, 2, 32>(akc, bkc, vec);
-    case 14:  // aligned k pairs: k_dgemm; otherwise (unaligned operands) tile 0's kernel
-      if (akc && bkc && vec) return reinterpret_cast<const void *>(&k_dgemm<T>);
-      return gemm_fn<T, 128, 128, 2, 2>(akc, bkc, false);
+    case 14:  // k-contiguous operands in aligned pairs; otherwise FP32 tile 0's kernel
     case 15:
-      if (akc && bkc && vec) return reinterpret_cast<const void *>(&k_dgemm2<T>);
-      return gemm_fn<T, 128, 128, 2, 2>(akc, bkc, false);
+      if constexpr (std::is_same_v<T, double>) {
+        return pipe_fn<4>(akc, bkc, vec);
+      } else {
+        if (akc && bkc && vec)
+          return tile == 14 ? reinterpret_cast<const void *>(&k_dgemm<T>) : reinterpret_cast<const void *>(&k_dgemm2<T>);
+        return gemm_fn<T, 128, 128, 2, 2>(akc, bkc, false);
+      }
+    case 16:  // FP64 only (build_plan)
+    case 17:
+      if constexpr (std::is_same_v<T, double>)
+        return tile == 16 ? pipe_fn<2>(akc, bkc, vec) : pipe_fn<4>(akc, bkc, vec);
+      return nullptr;
     default: return gemm_fn<T, 32, 32, 2, 2>(akc, bkc, vec);
   }
 }
@@ -2136,7 +2336,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
   int64_t extA = 1, extB = 1, extC = 1;
   // A is read along k if its unit-stride digit is a contracted one (else
   // along m); likewise B.  Decided on the first non-empty task.
-  bool akc = false, bkc = false, kc_set = false;
+  double akc_work = 0, bkc_work = 0;  // multiply-adds of tasks with k-contiguous operands less those of the others
 
   double flops = 0;
   // Everything a task needs besides its offsets follows from the block
@@ -2292,11 +2492,11 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
           return set_err(ctx, ITX_ERR_ARG, "contraction: dimensions of C do not match A and B");
     }
     if (fi.empty) continue;
-    if (!kc_set) {
-      kc_set = true;
-      akc = fi.akc;
-      bkc = fi.bkc;
-    }
+    // the tasks' common layout, by their work (K = 1 has none: at chi = 750
+    // the first block of the chain's products is 1 x 1 x 1)
+    const double work = fi.K > 1 ? double(fi.M) * double(fi.N) * double(fi.K) : 0.0;
+    akc_work += fi.akc ? work : -work;
+    bkc_work += fi.bkc ? work : -work;
     vecbits &= fi.vec;
     if (offs[3 * size_t(t)] % 2 || offs[3 * size_t(t) + 1] % 2) vecbits = 0;
     if (offs[3 * size_t(t)] % 4 || offs[3 * size_t(t) + 1] % 4) vecbits &= ~4;
@@ -2319,6 +2519,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     flops += 2.0 * double(fi.M) * double(fi.N) * double(fi.K);
     tasks.push_back(g);
   }
+  const bool akc = akc_work > 0, bkc = bkc_work > 0;
 
   // group tasks by C block, in C offset order and stable within a block
   // (keeps the planner's pair order): a counting sort over the distinct
@@ -2385,13 +2586,25 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
   for (auto &g : groups) maxKsum = std::max(maxKsum, g.ksum);
 
   // Build the device plan for one tile choice.
-  // the register-pipelined FP64 tile needs k-contiguous operands in aligned pairs
+  // tiles 14 and 15 need k-contiguous operands in aligned pairs
   const bool dg_ok = (prec == ITX_PREC_F64 || prec == ITX_PREC_F32) && akc && bkc && (vecbits & 1);
+  auto tile_ok = [&](int t) {
+    return ((t != kDgemm && t != kDgemm2) || dg_ok) && ((t != kPipe64 && t != kPipe128) || prec == ITX_PREC_F64);
+  };
   // skinny plans whose tasks all have K, N <= 8 run k_skinny_q: two rows per thread
   const bool tinyq = maxN <= SKQ_N && maxK <= SKQ_K;
+  // Units over k of the 64 x 64 tile for one product: as many as give every
+  // CU two workgroups, with at least 8 stages each (none where the scratch is
+  // the caller's).
+  auto pipe_split = [&]() {
+    if (st.size() != 1 || into) return 1;
+    const int64_t tiles = int64_t((st[0].M + 63) / 64) * ((st[0].N + 63) / 64);
+    const int64_t most = std::min<int64_t>(2 * cus / std::max<int64_t>(tiles, 1), st[0].K / (8 * DG_BK));
+    return int(std::max<int64_t>(1, std::min<int64_t>(most, 64)));
+  };
   auto finalize = [&](int best, itx_plan **pout) -> int {
     *pout = nullptr;
-    if ((best == kDgemm || best == kDgemm2) && !dg_ok) return ITX_ERR_UNSUPPORTED;
+    if (!tile_ok(best)) return ITX_ERR_UNSUPPORTED;
     const int tbm0 = (best == kSkinny && tinyq) ? SKQ_R * SK_ROWS : kTiles[best].bm;
     const int tbn0 = (best == kSkinny) ? std::max(1, maxN) : kTiles[best].bn;
     int tbm = tbm0, tbn = tbn0;
@@ -2413,7 +2626,31 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     std::vector<GemmTask> vt;  // device task list (st, or its k-chunks when split)
     int nslots = 0;
     bool split = false;
-    if (best == kSmall) {
+    const int slot_elems = best == kPipe64 ? 64 * 64 : SM_M * SM_N;
+    if (const int ns = best == kPipe64 ? pipe_split() : 1; ns > 1) {
+      // The k of a product with few tiles over several units: the k ranges
+      // outermost, so that an XCD's units share one range of A and B.
+      split = true;
+      const Grp &g = groups[0];
+      const int kc = ((st[0].K + ns - 1) / ns + DG_BK - 1) / DG_BK * DG_BK;
+      std::vector<std::array<int, 2>> at;
+      for (int m0 = 0; m0 < g.M; m0 += 64)
+        for (int n0 = 0; n0 < g.N; n0 += 64) at.push_back({m0, n0});
+      const int nk = (st[0].K + kc - 1) / kc;
+      for (int i = 0; i < nk; ++i) {
+        GemmTask x = st[0];
+        x.K = std::min(kc, st[0].K - i * kc);
+        x.tAK += i * kc;
+        x.tBK += i * kc;
+        vt.push_back(x);
+        for (size_t j = 0; j < at.size(); ++j) {
+          units.push_back({i, i + 1, at[j][0], at[j][1], int(j) * nk + i, 0});
+          ucost.push_back(0.0);  // in this order
+        }
+      }
+      for (size_t j = 0; j < at.size(); ++j) red.push_back({0, int(j) * nk, at[j][0], at[j][1], int(j + 1) * nk, 0});
+      nslots = int(at.size()) * nk;
+    } else if (best == kSmall) {
       // Split the k-chunk sequence of heavy tiles over several units when
       // the tiles alone cannot fill the device (few C blocks, long task
       // lists): chunk budget c per unit from the total work.
@@ -2490,8 +2727,88 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
       if (!sorted) {
         std::sort(ui.begin(), ui.end());
         std::vector<WorkUnit> su(units.size());
-        for (size_t i = 0; i < ui.size(); ++i) su[i] = units[size_t(ui[i].second)];
+        for (size_t i = 0; i < ui.size(); ++i) {
+          su[i] = units[size_t(ui[i].second)];
+          ucost[i] = -ui[i].first;
+        }
         units.swap(su);
+      }
+    }
+    if (groups.size() > 1 && !split ? units.size() > size_t(cus) : best != kSkinny && units.size() > 2 * kXcds) {
+      // Workgroup b runs on XCD b % 8 and takes units b, b + grid, ...: each
+      // XCD gets a list of units that share operands in its L2.  Equal units
+      // (one block, or the pieces of a split): eighths of the list.  Several
+      // blocks: pieces of at most 1/24 of the work spread by their cost, a
+      // piece the tiles of one block (they share rows of A and columns of B)
+      // or, for narrow tasks, the tiles at the same rows of the blocks that
+      // read the same blocks of A (B is a few numbers; an MPO stage reads
+      // each block of A for every channel it feeds).  chi = 1024 block-sparse
+      // chain, against the blocks from the heaviest down: 29.5 to 23.6, 23.4
+      // to 19.3 and 38.6 to 28.4 us; up to a unit per CU it gains nothing.
+      const size_t n = units.size();
+      std::array<std::vector<WorkUnit>, kXcds> lists;
+      if (split || groups.size() == 1) {
+        for (size_t i = 0, chunk = (n + kXcds - 1) / kXcds; i < n; ++i) lists[i / chunk].push_back(units[i]);
+      } else {
+        std::vector<int> head(vt.size());  // a block's first task -> its place in `open`
+        std::iota(head.begin(), head.end(), 0);
+        std::vector<int> open(vt.size(), -1);  // the latest piece of a block, or of a set's tile of rows
+        if (best == kSkinny) {
+          auto root = [&](int t) {
+            while (head[size_t(t)] != t) t = head[size_t(t)] = head[size_t(head[size_t(t)])];
+            return t;
+          };
+          std::unordered_map<int64_t, int> reader(2 * vt.size());  // block of A -> a block that reads it
+          for (auto &g : groups)
+            for (int t = g.tb; t < g.te; ++t)
+              head[size_t(root(g.tb))] = root(reader.emplace(vt[size_t(t)].a_off, g.tb).first->second);
+          std::vector<int> rows(vt.size(), 0);  // of a set, in tiles; then its place in `open`
+          for (auto &g : groups) {
+            int &r = rows[size_t(root(g.tb))];
+            r = std::max(r, (g.M + tbm - 1) / tbm);
+          }
+          int places = 0;
+          for (int &r : rows) places = std::exchange(r, places) + places;
+          for (auto &g : groups) open[size_t(g.tb)] = rows[size_t(root(g.tb))];
+          for (auto &g : groups) head[size_t(g.tb)] = open[size_t(g.tb)];
+          open.assign(size_t(places), -1);
+        }
+        std::vector<double> cost;  // of a piece
+        std::vector<int> of(n);    // a unit's piece
+        const double total = std::accumulate(ucost.begin(), ucost.end(), 0.0);
+        for (size_t i = 0; i < n; ++i) {
+          int &q = open[size_t(head[size_t(units[i].tbeg)] + (best == kSkinny ? units[i].m0 / tbm : 0))];
+          if (q < 0 || cost[size_t(q)] + ucost[i] > total / 24) {
+            q = int(cost.size());
+            cost.push_back(0.0);
+          }
+          cost[size_t(q)] += ucost[i];
+          of[i] = q;
+        }
+        std::vector<int> order(cost.size()), xcd(cost.size()), turn(n);
+        std::iota(order.begin(), order.end(), 0);
+        std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cost[size_t(a)] > cost[size_t(b)]; });
+        std::array<double, kXcds> load{};
+        for (int q : order) {
+          const auto x = std::min_element(load.begin(), load.end());
+          xcd[size_t(q)] = int(x - load.begin());
+          *x += cost[size_t(q)];
+        }
+        std::iota(turn.begin(), turn.end(), 0);
+        if (best == kSkinny) {  // a piece's units one after another
+          std::vector<int> place(cost.size() + 1, 0);
+          for (int q : of) ++place[size_t(q)];
+          int sum = 0;
+          for (int q : order) sum += std::exchange(place[size_t(q)], sum);
+          for (size_t i = 0; i < n; ++i) turn[size_t(place[size_t(of[i])]++)] = int(i);
+        }
+        for (int i : turn) lists[size_t(xcd[size_t(of[size_t(i)])])].push_back(units[size_t(i)]);
+      }
+      std::array<size_t, kXcds> at{};
+      for (size_t i = 0; i < n; ++i) {
+        size_t x = i % kXcds;
+        for (size_t y = 0; at[x] == lists[x].size(); ++y) x = y;  // its list is used up: the next units of another
+        units[i] = lists[x][at[x]++];
       }
     }
     auto *p = new itx_plan();
@@ -2510,8 +2827,9 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     p->fn_scalar = kernel_of(best, prec, akc, bkc, &p->block, 0, false, sk);
     p->nred = int(red.size());
     if (p->nred) {
-      p->fn_red = reinterpret_cast<const void *>(&k_reduce_tiles);
-      p->grid_red = int(std::min<int64_t>(int64_t(red.size()) * (SM_M * SM_N / SM_T), int64_t(cus) * 8));
+      p->fn_red = best == kPipe64 ? reinterpret_cast<const void *>(&k_reduce_tiles<64, 64>)
+                                  : reinterpret_cast<const void *>(&k_reduce_tiles<SM_M, SM_N>);
+      p->grid_red = int(std::min<int64_t>(int64_t(red.size()) * (slot_elems / SM_T), int64_t(cus) * 8));
     }
     if (std::getenv("ITX_PLAN_LOG"))
       std::fprintf(stderr, "[itx plan] tasks=%d units=%d tile=%dx%d%s grid=%d akc=%d bkc=%d flops=%.3e split=%d\n",
@@ -2525,7 +2843,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
       size_t o_red = (o_units + bu_bytes + 255) & ~size_t(255);
       size_t o_tab = (o_red + br_bytes + 255) & ~size_t(255);
       size_t o_ws = (o_tab + tab.size() * sizeof(int64_t) + 255) & ~size_t(255);
-      size_t total = o_ws + sizeof(double) * size_t(nslots) * (SM_M * SM_N);
+      size_t total = o_ws + sizeof(double) * size_t(nslots) * slot_elems;
       // the device image: tasks | units | reduction units | tables, each
       // 256-byte aligned, assembled in the staging arena
       const UploadPart parts[4] = {{vt.data(), 0, bt_bytes},
@@ -2571,29 +2889,37 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
   };
 
   // ---- tile selection ------------------------------------------------
-  // Skinny tasks (all N <= 32, K <= 64) take the VALU path.  Otherwise, in
-  // order: ITX_FORCE_TILE, the tuning table entry of this size class, a
-  // measurement of every MFMA tile when autotuning is on (result stored in
-  // the table), else the cost model: units (one per C tile, cost ~ tile
-  // area x summed K) scheduled LPT on CUs x occupancy slots.
+  // Narrow tasks (all N <= 32, K <= 64) over large C blocks take the skinny
+  // kernels, C blocks of at most 8192 elements (small QN blocks) the
+  // small-block kernels.  Otherwise, in order: ITX_FORCE_TILE, the tuning
+  // table entry of this size class, a measurement of every MFMA tile when
+  // autotuning is on (result stored in the table), else a cost model.
   int best = 0;
   const std::string key = tune_key(prec, akc, bkc, maxM, maxN, maxKsum, int(groups.size()));
   const char *force = std::getenv("ITX_FORCE_TILE");
-  // Narrow tasks (all N <= 32, K <= 64) over large C blocks take the
-  // skinny VALU path; C blocks of at most 8192 elements (small QN blocks)
-  // the small-block VALU path; everything else an MFMA tile.
   double rows = 0;
   for (auto &g : groups) rows += g.M;
   const double avg_rows = groups.empty() ? 0.0 : rows / double(groups.size());
   const bool narrow = maxN <= SK_N && maxK <= SK_K;
+  // FP64: the eight waves of a small-block unit share its k, and wait for
+  // each other, so they want more than four chunks of 16 k, and no more units
+  // than CUs (block-sparse chain, 32 x 32 tiles against small blocks: chi =
+  // 250 first stage, 1.5 chunks, 4.7 and 7.1 us; chi = 500 last stage, 14
+  // chunks of 156 tiles, 13.0 and 11.0; chi = 750, 19 of 326, 18.4 and 19.8)
+  double n32 = 0, chunks = 0;
+  for (auto &g : groups) {
+    const double n = double((g.M + 31) / 32) * double((g.N + 31) / 32);
+    n32 += n;
+    for (int t = g.tb; t < g.te; ++t) chunks += n * double((st[t].K + SM_K - 1) / SM_K);
+  }
+  const bool long_k = prec != ITX_PREC_F64 || (chunks > 4 * n32 && n32 <= cus);
   if (!st.empty() && !force && narrow && avg_rows >= 256) {
     best = kSkinny;
   } else if (!st.empty() && !force && double(maxM) * double(maxN) <= 8192.0) {
-    best = kSmall;
+    best = long_k ? kSmall : 4;
   } else if (force) {
     best = std::atoi(force);
-    if (best < 0 || best >= kNumTiles || (best == kSkinny && !narrow) || ((best == kDgemm || best == kDgemm2) && !dg_ok))
-      best = 0;
+    if (best < 0 || best >= kNumTiles || (best == kSkinny && !narrow) || !tile_ok(best)) best = 0;
   } else if (ctx->tune.count(key)) {
     best = ctx->tune[key];
   } else if (ctx->autotune && !into && !st.empty()) {
@@ -2633,6 +2959,54 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     pool_free(ctx, bufB);
     pool_free(ctx, bufC);
     ctx->tune[key] = best;
+  } else if (prec == ITX_PREC_F64) {
+    // 32 x 32 (k_gemm), 64 x 64 and 128 x 128 (k_pipe), one product also
+    // 64 x 64 over split k or the small-block kernel.  A unit costs its k
+    // stages of 16 and a few more for every task and for itself; `alone` is
+    // the time of a stage (us) of a workgroup that has its CU to itself,
+    // `shared` the CU's time per stage when it has several.  Fitted to the
+    // stages of the dense chain: k-contiguous operands from chi = 48 to 1024
+    // (chi = 512 last stage 152 us as 32 x 32, 96 as 64 x 64, 293 as 128 x
+    // 128; chi = 255 43, 28 (split eight ways), 168; chi = 1024 1040, 660,
+    // 593), others to the MPO stage of d = 4, k = 18 (chi = 32 21.6, 18.4,
+    // 50.6; chi = 330 1274, 676, 574), where the operator is read in single
+    // strided elements.
+    struct Model {
+      int tile, b;
+      double alone, shared, per_task, per_unit;
+    };
+    const double v1 = (vecbits & 1) ? 1.0 : 1.1;  // single loads
+    const Model kc[] = {{4, 32, 0.45, 0.28, 1, 1},
+                        {kPipe64, 64, 0.63 * v1, 0.50 * v1, 3, 2},
+                        {kPipe128, 128, 1.87 * v1, 1.87 * v1, 2, 1}};
+    const Model any[] = {{4, 32, 0.50, 0.50, 1, 1}, {kPipe64, 64, 0.70, 0.88, 3, 2}, {kPipe128, 128, 2.65, 2.65, 2, 1}};
+    const auto &models = akc && bkc ? kc : any;
+    best = 4;
+    double best_t = 1e300;
+    for (const Model &md : models) {
+      std::vector<double> costs;
+      double most = 0;
+      const int ns = md.tile == kPipe64 ? pipe_split() : 1;
+      for (auto &g : groups) {
+        double c = md.per_unit;
+        for (int t = g.tb; t < g.te; ++t) c += double((st[t].K + DG_BK - 1) / DG_BK) / ns + md.per_task;
+        const int64_t tiles = int64_t((g.M + md.b - 1) / md.b) * ((g.N + md.b - 1) / md.b) * ns;
+        most = std::max(most, c);
+        costs.insert(costs.end(), size_t(tiles), c);
+      }
+      double tt = std::max(most * md.alone, lpt_makespan(costs, cus) * md.shared);
+      if (ns > 1)  // the partial tiles and the second launch
+        tt += 5.0 + double(ns) * groups[0].M * groups[0].N * 16.0 / 4e6;
+      if (tt < best_t) {
+        best_t = tt;
+        best = md.tile;
+      }
+    }
+    if (st.size() == 1 && st[0].K <= 640) {  // above, its partial tiles cost more
+      const bool fine = n32 < cus / 2;  // as finalize sizes the units
+      const double n16 = double((st[0].M + 15) / 16) * double((st[0].N + 15) / 16);
+      if ((fine ? n16 : n32) <= cus && 2.0 + (fine ? 1.35 : 2.2) * ((st[0].K + 127) / 128) < best_t) best = kSmall;
+    }
   } else {
     double best_t = 1e300;
     // the 32-deep variants (11-13) are left to measurement (autotuner,
@@ -2647,18 +3021,14 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
         for (int64_t q = 0; q < tiles; ++q) costs.push_back(c);
       }
       if (costs.empty()) continue;
-      // workgroups resident per CU: for the reduced forms the tile's
-      // occupancy, or fewer when the units do not fill that many slots (a CU
-      // running one workgroup does not run it `occupancy` times slower;
-      // without this the FP32 form picked a 64 x 256 tile for 150 units of
-      // the chi = 1024 QN chain, 86 us against 40 us); the FP64 efficiencies
-      // were calibrated against the plain occupancy
-      const int occ_max = tile_occupancy(ti, prec, akc, bkc);
-      const int occ = prec == ITX_PREC_F64
-                          ? occ_max
-                          : int(std::max<int64_t>(1, std::min<int64_t>(occ_max, (int64_t(costs.size()) + cus - 1) / cus)));
-      const double eff = (prec == ITX_PREC_F64) ? ts.eff64 : ts.eff32;
-      const double tt = lpt_makespan(costs, int64_t(cus) * occ) * occ / eff;
+      // workgroups resident per CU: the tile's occupancy, or fewer when the
+      // units do not fill that many slots (a CU running one workgroup does not
+      // run it `occupancy` times slower; without this the FP32 form picked a
+      // 64 x 256 tile for 150 units of the chi = 1024 QN chain, 86 us against
+      // 40 us)
+      const int occ = int(std::max<int64_t>(
+          1, std::min<int64_t>(tile_occupancy(ti, prec, akc, bkc), (int64_t(costs.size()) + cus - 1) / cus)));
+      const double tt = lpt_makespan(costs, int64_t(cus) * occ) * occ / ts.eff32;
       if (tt < best_t * 0.97) {
         best_t = tt;
         best = ti;

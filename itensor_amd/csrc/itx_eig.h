@@ -85,14 +85,6 @@ __device__ __forceinline__ double read_lane(double v, int l) {  // l wave-unifor
   return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
 }
 
-// A workgroup barrier that orders LDS only: __syncthreads also waits for the
-// wave's global stores, a trip through memory per barrier.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // ---- reciprocals and square roots ---------------------------------------------
 // The hardware estimate (24 bits) refined by Newton's iteration, one step of
 // third order or two of second (error about one unit in the last place, for

@@ -15,6 +15,14 @@
 
 namespace itx {
 
+// A workgroup barrier that orders LDS only: __syncthreads also waits for the
+// wave's global stores, a trip through memory per barrier.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // One GEMM of a contraction: C[m,n] (+)= sum_k A[m,k] B[k,n], where the
 // element of A at logical (m,k) lives at a_off + tab[tAM+m] + tab[tAK+k]
 // (and likewise for B and C).  The offset tables carry the index

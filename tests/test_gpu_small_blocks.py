@@ -46,5 +46,6 @@ def _run(ctx, dev, shapes, aorder, border, alpha=1.5):
     [((40, 37), [23, 11])] * 300, [((70, 40), [33])] * 150,  # units of 64 and of 32 rows
     [((30, 30), [50] * 60)], [((90, 80), [64] * 40)] * 2,    # split over units
 ], ids=range(12))
-def test_small_blocks(ctx, dev, shapes, aorder, border):
+def test_small_blocks(ctx, dev, monkeypatch, shapes, aorder, border):
+    monkeypatch.setenv("ITX_FORCE_TILE", "10")  # also where the 32 x 32 tile is the default
     _run(ctx, dev, shapes, aorder, border)
