@@ -731,17 +731,19 @@ __global__ __launch_bounds__(DG_NT, 2) void k_dgemm2(const double *__restrict__ 
 // k_gemm / k_dgemm: chi = 1024 773 + 728 to 624 + 593 us (the matrix cores
 // need 563 each), chi = 512 136 + 148 to 100 + 96, chi = 255 28 + 43 to 26.5 +
 // 28.5.
-template <int ROWS, int V>
-struct PipeLoader {  // one operand: ROWS x 16 k per stage; V = 0: lanes along the rows, a wave's 4 k each
-  static constexpr int LK = V ? DG_BK / (V ? V : 1) : 4, RS = DG_NT / LK, NP = ROWS / RS, NK = V ? 1 : 4;
+template <typename T, int ROWS, int V>
+struct PipeLoader {  // one operand: ROWS x 16 k per stage; V = 0: lanes along the rows, a few k each
+  static constexpr int LK = V ? DG_BK / (V ? V : 1) : DG_NT / (ROWS < 64 ? ROWS : 64);
+  static constexpr int RS = DG_NT / LK, NP = ROWS / RS, NK = V ? 1 : DG_BK / LK;
   static constexpr int NR = ROWS / 16;                                      // doubles of a thread
-  static constexpr int NLD = V == 2 ? NR / 2 : NR, NST = V == 1 ? NR : NR / 2;  // loads, LDS stores
+  static constexpr int NLD = V == 2 ? NR / 2 : NR;                          // loads
+  static constexpr int NST = V == 1 || sizeof(T) == 4 ? NR : NR / 2;        // LDS stores
   int64_t roff[NP];
   int64_t ko[2][NK];  // k offsets of the next two stages to load (slot = stage & 1)
   int lr, lc;
   __device__ __forceinline__ void init(int tid, int row0, int R, const int64_t *__restrict__ tabR) {
-    lc = V ? tid % LK : 4 * __builtin_amdgcn_readfirstlane(tid >> 6);
-    lr = V ? tid / LK : tid & 63;
+    lc = V ? tid % LK : NK * (RS == 64 ? __builtin_amdgcn_readfirstlane(tid / RS) : tid / RS);
+    lr = V ? tid / LK : tid % RS;
 #pragma unroll
     for (int p = 0; p < NP; ++p) roff[p] = tabR[min(row0 + lr + RS * p, R - 1)];
   }
@@ -766,54 +768,66 @@ struct PipeLoader {  // one operand: ROWS x 16 k per stage; V = 0: lanes along t
       }
     }
   }
+  // where the fragment reads want k: FP64 k = 4q + s in the lanes of quarter
+  // q at MFMA s, FP32 k = 4s + q (the sums of k_gemm, to the last bit)
+  static __device__ __forceinline__ int place(int k) { return sizeof(T) == 8 ? k : 4 * (k & 3) + (k >> 2); }
   // k0: first k of the stage (TAIL: its k past K are zeroed)
   template <bool TAIL>
-  __device__ __forceinline__ void store(double *__restrict__ s, const double (&r)[NR], int k0, int K) const {
+  __device__ __forceinline__ void store(T *__restrict__ s, const double (&r)[NR], int k0, int K) const {
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-      double *d = s + (lr + RS * p) * DgCfg<double>::P;
-      if constexpr (V == 1) {
-        d[lc] = !TAIL || k0 + lc < K ? r[p] : 0.0;
-      } else if constexpr (V == 2) {
-        const bool ok = !TAIL || k0 + 2 * lc < K;
-        *reinterpret_cast<double2 *>(d + 2 * lc) = ok ? double2{r[2 * p], r[2 * p + 1]} : double2{0.0, 0.0};
-      } else {
+      T *d = s + (lr + RS * p) * DgCfg<T>::P;
+      constexpr int NE = V == 2 ? 2 : NK;  // consecutive k of a thread
 #pragma unroll
-        for (int c = 0; c < 4; c += 2) {
-          double2 v;
-          v.x = !TAIL || k0 + lc + c < K ? r[4 * p + c] : 0.0;
-          v.y = !TAIL || k0 + lc + c + 1 < K ? r[4 * p + c + 1] : 0.0;
-          *reinterpret_cast<double2 *>(d + lc + c) = v;
+      for (int c = 0; c < NE; c += 2) {
+        const T x = !TAIL || k0 + (V ? V : 1) * lc + c < K ? T(r[NE * p + c]) : T(0);
+        if constexpr (NE == 1) {
+          d[place(lc)] = x;
+        } else {
+          const int k = (V ? V : 1) * lc + c;
+          const T y = !TAIL || k0 + k + 1 < K ? T(r[NE * p + c + 1]) : T(0);
+          if constexpr (sizeof(T) == 8) {
+            *reinterpret_cast<double2 *>(d + k) = double2{x, y};
+          } else {
+            d[place(k)] = x;
+            d[place(k + 1)] = y;
+          }
         }
       }
     }
   }
 };
 
-template <int F>
+template <typename T, int F>
 struct PipeFrag {  // one operand of a stage: F fragments x 4 k
-  double2 x[F][2];
-  __device__ __forceinline__ void read(const double *__restrict__ s, int row0, int lane) {
+  using Quad = std::conditional_t<sizeof(T) == 8, double2[2], float4>;
+  Quad x[F];
+  __device__ __forceinline__ void read(const T *__restrict__ s, int row0, int lane) {
 #pragma unroll
     for (int j = 0; j < F; ++j) {
-      const double *p = s + (row0 + j * 16 + (lane & 15)) * DgCfg<double>::P + 4 * (lane >> 4);
-      x[j][0] = *reinterpret_cast<const double2 *>(p);
-      x[j][1] = *reinterpret_cast<const double2 *>(p + 2);
+      const T *p = s + (row0 + j * 16 + (lane & 15)) * DgCfg<T>::P + 4 * (lane >> 4);
+      if constexpr (sizeof(T) == 8) {
+        x[j][0] = *reinterpret_cast<const double2 *>(p);
+        x[j][1] = *reinterpret_cast<const double2 *>(p + 2);
+      } else {
+        x[j] = *reinterpret_cast<const float4 *>(p);
+      }
     }
   }
 };
 
-template <int FM, int FN, int VA, int VB>
+template <typename T, int FM, int FN, int VA, int VB>
 __global__ __launch_bounds__(DG_NT, FM * FN <= 4 ? 2 : 1) void k_pipe(
     const double *__restrict__ A, const double *__restrict__ B, double *__restrict__ C,
     const GemmTask *__restrict__ tasks, const WorkUnit *__restrict__ units, int nunits, const int64_t *__restrict__ tab,
     double alpha, double beta) {
-  using v4 = MF<double>::v4;
-  constexpr int P = DgCfg<double>::P, BM = 32 * FM, BN = 32 * FN, NM = FM * FN;
-  using LA = PipeLoader<BM, VA>;
-  using LB = PipeLoader<BN, VB>;
-  __shared__ __align__(16) double As[2][BM * P];
-  __shared__ __align__(16) double Bs[2][BN * P];
+  using v4 = typename MF<T>::v4;
+  constexpr int P = DgCfg<T>::P, BM = 32 * FM, BN = 32 * FN, NM = FM * FN;
+  constexpr int NRD = (sizeof(T) == 8 ? 2 : 1) * (FM + FN);  // LDS reads of a stage
+  using LA = PipeLoader<T, BM, VA>;
+  using LB = PipeLoader<T, BN, VB>;
+  __shared__ __align__(16) T As[2][BM * P];
+  __shared__ __align__(16) T Bs[2][BN * P];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = (wave & 1) * 16 * FM, wn = (wave >> 1) * 16 * FN;
 
@@ -850,13 +864,13 @@ __global__ __launch_bounds__(DG_NT, FM * FN <= 4 ? 2 : 1) void k_pipe(
     la.template store<tail>(As[(st) & 1], ra, (st) * DG_BK, K);           \
     lb.template store<tail>(Bs[(st) & 1], rb, (st) * DG_BK, K);           \
   }
-      PipeFrag<FM> fa0, fa1;
-      PipeFrag<FN> fb0, fb1;
-      auto mfma = [&](const PipeFrag<FM> &fa, const PipeFrag<FN> &fb, int s) __attribute__((always_inline)) {
+      PipeFrag<T, FM> fa0, fa1;
+      PipeFrag<T, FN> fb0, fb1;
+      auto mfma = [&](const PipeFrag<T, FM> &fa, const PipeFrag<T, FN> &fb, int s) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < FN; ++i)
 #pragma unroll
-          for (int j = 0; j < FM; ++j) acc[i][j] = MF<double>::mma(dg_k(fb.x[i], s), dg_k(fa.x[j], s), acc[i][j]);
+          for (int j = 0; j < FM; ++j) acc[i][j] = MF<T>::mma(dg_k(fb.x[i], s), dg_k(fa.x[j], s), acc[i][j]);
       };
       la.fetch_k(0, K, tAK, 0);
       lb.fetch_k(0, K, tBK, 0);
@@ -900,7 +914,7 @@ __global__ __launch_bounds__(DG_NT, FM * FN <= 4 ? 2 : 1) void k_pipe(
     mfma(fa, fb, 0);                                                                             \
     for (int g_ = 0; g_ < NM; ++g_) {                                                            \
       __builtin_amdgcn_sched_group_barrier(0x008, 1, id);                                        \
-      __builtin_amdgcn_sched_group_barrier(0x100, (2 * (FM + FN) + NM - 1) / NM, id);            \
+      __builtin_amdgcn_sched_group_barrier(0x100, (NRD + NM - 1) / NM, id);                      \
     }                                                                                            \
     __builtin_amdgcn_sched_barrier(0);                                                           \
     ITX_PIPE_STORE(false, (n) + 2, ra, rb)                                                       \
@@ -938,7 +952,7 @@ __global__ __launch_bounds__(DG_NT, FM * FN <= 4 ? 2 : 1) void k_pipe(
 #undef ITX_PIPE_LOAD
     }
 
-    if (wu.slot >= 0) {  // partial tile of a split unit (C is the workspace)
+    if (sizeof(T) == 8 && wu.slot >= 0) {  // partial tile of a split unit (C is the workspace)
       double *Pt = C + size_t(wu.slot) * (BM * BN);
 #pragma unroll
       for (int i = 0; i < FN; ++i)
@@ -946,7 +960,7 @@ __global__ __launch_bounds__(DG_NT, FM * FN <= 4 ? 2 : 1) void k_pipe(
         for (int r = 0; r < 4; ++r)
 #pragma unroll
           for (int j = 0; j < FM; ++j)
-            Pt[(wn + i * 16 + MF<double>::orow(lane, r)) * BM + wm + j * 16 + (lane & 15)] = acc[i][j][r];
+            Pt[(wn + i * 16 + MF<T>::orow(lane, r)) * BM + wm + j * 16 + (lane & 15)] = acc[i][j][r];
       continue;
     }
     const GemmTask t0 = tasks[wu.tbeg];
@@ -959,17 +973,17 @@ __global__ __launch_bounds__(DG_NT, FM * FN <= 4 ? 2 : 1) void k_pipe(
 #pragma unroll
     for (int i = 0; i < FN; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) cn[i][r] = tCN[min(wu.n0 + wn + i * 16 + MF<double>::orow(lane, r), t0.N - 1)];
+      for (int r = 0; r < 4; ++r) cn[i][r] = tCN[min(wu.n0 + wn + i * 16 + MF<T>::orow(lane, r), t0.N - 1)];
 #pragma unroll
     for (int j = 0; j < FM; ++j)
 #pragma unroll
       for (int i = 0; i < FN; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int m = wu.m0 + wm + j * 16 + (lane & 15), n = wu.n0 + wn + i * 16 + MF<double>::orow(lane, r);
+          const int m = wu.m0 + wm + j * 16 + (lane & 15), n = wu.n0 + wn + i * 16 + MF<T>::orow(lane, r);
           if (m < t0.M && n < t0.N) {
             const int64_t ad = cm[j] + cn[i][r];
-            double v = alpha * acc[i][j][r];
+            double v = alpha * double(acc[i][j][r]);
             if (beta != 0.0) v += beta * Cb[ad];
             Cb[ad] = v;
           }
@@ -2112,11 +2126,12 @@ constexpr TileCfg kTiles[] = {
     {64, 128, 2, 2, 0.95},   // 13: as 2 with 32-deep k stages
     {128, 128, 2, 2, 0.85},  // 14: FP32 register-pipelined (k_dgemm); FP64 as 17; k-contiguous pairs only
     {128, 128, 2, 2, 0.85},  // 15: as 14, FP32 two workgroups per CU (k_dgemm2)
-    {64, 64, 2, 2, 0.0},     // 16: FP64 register-pipelined (k_pipe)
+    {64, 64, 2, 2, 0.0},     // 16: register-pipelined (k_pipe), FP64 and FP32
     {128, 128, 2, 2, 0.0},   // 17: likewise
+    {32, 64, 2, 2, 0.0},     // 18: likewise, FP32
 };
-constexpr int kNumTiles = 18;
-constexpr int kPipe64 = 16, kPipe128 = 17;
+constexpr int kNumTiles = 19;
+constexpr int kPipe64 = 16, kPipe128 = 17, kPipe32 = 18;
 constexpr int kDgemm = 14, kDgemm2 = 15;
 constexpr int kSkinny = 5;
 static_assert(kSkinny == kSkinnyTile, "tile index of the skinny path");
@@ -2170,12 +2185,14 @@ const void *gemm3_fn_tile(int tile, bool akc, bool bkc, bool vec, bool split) {
   }
 }
 
-template <int F>
+template <typename T, int FM, int FN>
 const void *pipe_fn(bool akc, bool bkc, bool vec) {
-  if (akc && bkc && vec) return reinterpret_cast<const void *>(&k_pipe<F, F, 2, 2>);
+  if (akc && bkc && vec) return reinterpret_cast<const void *>(&k_pipe<T, FM, FN, 2, 2>);
   if (akc)
-    return bkc ? reinterpret_cast<const void *>(&k_pipe<F, F, 1, 1>) : reinterpret_cast<const void *>(&k_pipe<F, F, 1, 0>);
-  return bkc ? reinterpret_cast<const void *>(&k_pipe<F, F, 0, 1>) : reinterpret_cast<const void *>(&k_pipe<F, F, 0, 0>);
+    return bkc ? reinterpret_cast<const void *>(&k_pipe<T, FM, FN, 1, 1>)
+               : reinterpret_cast<const void *>(&k_pipe<T, FM, FN, 1, 0>);
+  return bkc ? reinterpret_cast<const void *>(&k_pipe<T, FM, FN, 0, 1>)
+             : reinterpret_cast<const void *>(&k_pipe<T, FM, FN, 0, 0>);
 }
 
 template <typename T>
@@ -2195,16 +2212,16 @@ const void *gemm_fn_tile(int tile, bool akc, bool bkc, bool vec) {
     case 14:  // k-contiguous operands in aligned pairs; otherwise FP32 tile 0's kernel
     case 15:
       if constexpr (std::is_same_v<T, double>) {
-        return pipe_fn<4>(akc, bkc, vec);
+        return pipe_fn<T, 4, 4>(akc, bkc, vec);
       } else {
         if (akc && bkc && vec)
           return tile == 14 ? reinterpret_cast<const void *>(&k_dgemm<T>) : reinterpret_cast<const void *>(&k_dgemm2<T>);
         return gemm_fn<T, 128, 128, 2, 2>(akc, bkc, false);
       }
-    case 16:  // FP64 only (build_plan)
-    case 17:
-      if constexpr (std::is_same_v<T, double>)
-        return tile == 16 ? pipe_fn<2>(akc, bkc, vec) : pipe_fn<4>(akc, bkc, vec);
+    case 16: return pipe_fn<T, 2, 2>(akc, bkc, vec);
+    case 17: return pipe_fn<T, 4, 4>(akc, bkc, vec);
+    case 18:  // FP32 only (build_plan)
+      if constexpr (std::is_same_v<T, float>) return pipe_fn<T, 1, 2>(akc, bkc, vec);
       return nullptr;
     default: return gemm_fn<T, 32, 32, 2, 2>(akc, bkc, vec);
   }
@@ -2274,6 +2291,12 @@ int tile_occupancy(int tile, int prec, bool akc, bool bkc) {
   }
   cache[key] = nb;
   return nb;
+}
+
+// lpt_makespan of n units of one cost
+double lpt_makespan(int64_t n, double cost, int64_t slots) {
+  if (n > 4 * slots) return double(n) * cost / double(slots) + 0.5 * cost;
+  return double((n + slots - 1) / slots) * cost;
 }
 
 // Makespan of units (costs) on `slots` identical workers, heaviest first
@@ -2589,7 +2612,8 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
   // tiles 14 and 15 need k-contiguous operands in aligned pairs
   const bool dg_ok = (prec == ITX_PREC_F64 || prec == ITX_PREC_F32) && akc && bkc && (vecbits & 1);
   auto tile_ok = [&](int t) {
-    return ((t != kDgemm && t != kDgemm2) || dg_ok) && ((t != kPipe64 && t != kPipe128) || prec == ITX_PREC_F64);
+    return ((t != kDgemm && t != kDgemm2) || dg_ok) && ((t != kPipe64 && t != kPipe128) || prec != ITX_PREC_BF16X3) &&
+           (t != kPipe32 || prec == ITX_PREC_F32);
   };
   // skinny plans whose tasks all have K, N <= 8 run k_skinny_q: two rows per thread
   const bool tinyq = maxN <= SKQ_N && maxK <= SKQ_K;
@@ -2597,7 +2621,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
   // CU two workgroups, with at least 8 stages each (none where the scratch is
   // the caller's).
   auto pipe_split = [&]() {
-    if (st.size() != 1 || into) return 1;
+    if (st.size() != 1 || into || prec != ITX_PREC_F64) return 1;  // FP32 sums keep their order
     const int64_t tiles = int64_t((st[0].M + 63) / 64) * ((st[0].N + 63) / 64);
     const int64_t most = std::min<int64_t>(2 * cus / std::max<int64_t>(tiles, 1), st[0].K / (8 * DG_BK));
     return int(std::max<int64_t>(1, std::min<int64_t>(most, 64)));
@@ -2959,80 +2983,102 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     pool_free(ctx, bufB);
     pool_free(ctx, bufC);
     ctx->tune[key] = best;
-  } else if (prec == ITX_PREC_F64) {
-    // 32 x 32 (k_gemm), 64 x 64 and 128 x 128 (k_pipe), one product also
-    // 64 x 64 over split k or the small-block kernel.  A unit costs its k
+  } else {
+    if (prec != ITX_PREC_F64) {
+      double best_t = 1e300;
+      // the 32-deep variants (11-13) are left to measurement (autotuner,
+      // ITX_FORCE_TILE): they only pay off for long K on large tiles
+      for (int ti : {0, 1, 2, 3, 4, 6, 7, 8, 9, kDgemm}) {
+        if (ti == kDgemm && !dg_ok) continue;
+        const TileCfg ts = kTiles[ti];
+        std::vector<double> costs;
+        int64_t n = 0;
+        double one = 0;
+        for (auto &g : groups) {
+          const int64_t tiles = int64_t((g.M + ts.bm - 1) / ts.bm) * ((g.N + ts.bn - 1) / ts.bn);
+          one = double(ts.bm) * ts.bn * (g.ksum + BK * (g.te - g.tb) + 8);
+          n += tiles;
+          if (groups.size() > 1) costs.insert(costs.end(), size_t(tiles), one);
+        }
+        if (!n) continue;
+        // workgroups resident per CU: the tile's occupancy, or fewer when the
+        // units do not fill that many slots (a CU running one workgroup does not
+        // run it `occupancy` times slower; without this the FP32 form picked a
+        // 64 x 256 tile for 150 units of the chi = 1024 QN chain, 86 us against
+        // 40 us)
+        const int occ = int(std::max<int64_t>(
+            1, std::min<int64_t>(tile_occupancy(ti, prec, akc, bkc), (n + cus - 1) / cus)));
+        const int64_t slots = int64_t(cus) * occ;
+        const double tt = (costs.empty() ? lpt_makespan(n, one, slots) : lpt_makespan(costs, slots)) * occ / ts.eff32;
+        if (tt < best_t * 0.97) {
+          best_t = tt;
+          best = ti;
+        }
+      }
+    }
+    // The pipelined tiles (k_pipe) and the 32 x 32 tile.  A unit costs its k
     // stages of 16 and a few more for every task and for itself; `alone` is
     // the time of a stage (us) of a workgroup that has its CU to itself,
-    // `shared` the CU's time per stage when it has several.  Fitted to the
-    // stages of the dense chain: k-contiguous operands from chi = 48 to 1024
-    // (chi = 512 last stage 152 us as 32 x 32, 96 as 64 x 64, 293 as 128 x
-    // 128; chi = 255 43, 28 (split eight ways), 168; chi = 1024 1040, 660,
-    // 593), others to the MPO stage of d = 4, k = 18 (chi = 32 21.6, 18.4,
-    // 50.6; chi = 330 1274, 676, 574), where the operator is read in single
-    // strided elements.
+    // `shared` the CU's time per stage when it has several; `any` for operands
+    // not contiguous along k.  Fitted to the stages of the dense chain, k-
+    // contiguous at chi = 48 to 1024, others to its MPO stage at d = 4, k = 18,
+    // where the operator is read in single strided elements.
+    // FP64, us as 32 x 32, 64 x 64, 128 x 128: last stage, chi = 255 43, 28
+    // (split eight ways), 168; chi = 512 152, 96, 293; chi = 1024 1040, 660,
+    // 593; MPO stage, chi = 32 21.6, 18.4, 50.6; chi = 330 1274, 676, 574.
+    // FP32, and 32 x 64 (before: 64 x 64 of k_gemm): last stage, chi = 256 37,
+    // 35.4, 91.5, 28.4 (69); chi = 512 139, 77, 177, 77 (134); chi = 1024 876,
+    // 440, 358, 516 (579).  Tile 14, where it is the best of those before, sums
+    // in another order and stays.
     struct Model {
-      int tile, b;
-      double alone, shared, per_task, per_unit;
+      int tile, bm, bn;
+      double alone, shared, any_alone, any_shared, per_task, per_unit;
     };
-    const double v1 = (vecbits & 1) ? 1.0 : 1.1;  // single loads
-    const Model kc[] = {{4, 32, 0.45, 0.28, 1, 1},
-                        {kPipe64, 64, 0.63 * v1, 0.50 * v1, 3, 2},
-                        {kPipe128, 128, 1.87 * v1, 1.87 * v1, 2, 1}};
-    const Model any[] = {{4, 32, 0.50, 0.50, 1, 1}, {kPipe64, 64, 0.70, 0.88, 3, 2}, {kPipe128, 128, 2.65, 2.65, 2, 1}};
-    const auto &models = akc && bkc ? kc : any;
-    best = 4;
+    const double v1 = (vecbits & 1) ? 1.0 : prec == ITX_PREC_F64 ? 1.1 : 1.2;  // single loads
+    const Model f64[] = {{4, 32, 32, 0.45, 0.28, 0.50, 0.50, 1, 1},
+                         {kPipe64, 64, 64, 0.63 * v1, 0.50 * v1, 0.70, 0.88, 3, 2},
+                         {kPipe128, 128, 128, 1.87 * v1, 1.87 * v1, 2.65, 2.65, 2, 1}};
+    const Model f32[] = {{4, 32, 32, 0.42, 0.17, 0.50, 0.50, 1, 1},
+                         {kPipe32, 32, 64, 0.28 * v1, 0.21 * v1, 0.75, 0.85, 2, 1},
+                         {kPipe64, 64, 64, 0.43 * v1, 0.33 * v1, 0.62, 0.83, 3, 2},
+                         {kPipe128, 128, 128, 1.13 * v1, 1.13 * v1, 1.80, 2.05, 2, 1}};
+    const Model *models = prec == ITX_PREC_F64 ? f64 : f32;
+    const size_t nm = prec == ITX_PREC_F64 ? std::size(f64)
+                      : prec == ITX_PREC_F32 && best != kDgemm ? std::size(f32) : 0;
+    if (nm) best = 4;
     double best_t = 1e300;
-    for (const Model &md : models) {
+    for (const Model *md = models; md < models + nm; ++md) {
       std::vector<double> costs;
-      double most = 0;
-      const int ns = md.tile == kPipe64 ? pipe_split() : 1;
+      int64_t n = 0;
+      double most = 0, bytes = 0;
+      const int ns = md->tile == kPipe64 ? pipe_split() : 1;
       for (auto &g : groups) {
-        double c = md.per_unit;
-        for (int t = g.tb; t < g.te; ++t) c += double((st[t].K + DG_BK - 1) / DG_BK) / ns + md.per_task;
-        const int64_t tiles = int64_t((g.M + md.b - 1) / md.b) * ((g.N + md.b - 1) / md.b) * ns;
+        double c = md->per_unit;
+        for (int t = g.tb; t < g.te; ++t) c += double((st[t].K + DG_BK - 1) / DG_BK) / ns + md->per_task;
+        const int64_t tiles = int64_t((g.M + md->bm - 1) / md->bm) * ((g.N + md->bn - 1) / md->bn) * ns;
         most = std::max(most, c);
-        costs.insert(costs.end(), size_t(tiles), c);
+        bytes += double(tiles) * g.ksum / ns * (md->bm + md->bn) * 8.0;
+        n += tiles;
+        if (groups.size() > 1) costs.insert(costs.end(), size_t(tiles), c);
       }
-      double tt = std::max(most * md.alone, lpt_makespan(costs, cus) * md.shared);
+      const bool kc = akc && bkc;
+      double tt = std::max(most * (kc ? md->alone : md->any_alone),
+                           (costs.empty() ? lpt_makespan(n, most, cus) : lpt_makespan(costs, cus)) *
+                               (kc ? md->shared : md->any_shared));
+      // what the L2s deliver, TB/s (chi = 1024: first stage 12.9, K = 1024;
+      // last stage 6.2, K = 5120)
+      tt = std::max(tt, bytes / (maxK > 2048 ? 6.2e6 : 12.9e6));
       if (ns > 1)  // the partial tiles and the second launch
         tt += 5.0 + double(ns) * groups[0].M * groups[0].N * 16.0 / 4e6;
       if (tt < best_t) {
         best_t = tt;
-        best = md.tile;
+        best = md->tile;
       }
     }
-    if (st.size() == 1 && st[0].K <= 640) {  // above, its partial tiles cost more
+    if (prec == ITX_PREC_F64 && st.size() == 1 && st[0].K <= 640) {  // above, its partial tiles cost more
       const bool fine = n32 < cus / 2;  // as finalize sizes the units
       const double n16 = double((st[0].M + 15) / 16) * double((st[0].N + 15) / 16);
       if ((fine ? n16 : n32) <= cus && 2.0 + (fine ? 1.35 : 2.2) * ((st[0].K + 127) / 128) < best_t) best = kSmall;
-    }
-  } else {
-    double best_t = 1e300;
-    // the 32-deep variants (11-13) are left to measurement (autotuner,
-    // ITX_FORCE_TILE): they only pay off for long K on large tiles
-    for (int ti : {0, 1, 2, 3, 4, 6, 7, 8, 9, kDgemm}) {
-      if (ti == kDgemm && !dg_ok) continue;
-      const TileCfg ts = kTiles[ti];
-      std::vector<double> costs;
-      for (auto &g : groups) {
-        const int64_t tiles = int64_t((g.M + ts.bm - 1) / ts.bm) * ((g.N + ts.bn - 1) / ts.bn);
-        const double c = double(ts.bm) * ts.bn * (g.ksum + BK * (g.te - g.tb) + 8);
-        for (int64_t q = 0; q < tiles; ++q) costs.push_back(c);
-      }
-      if (costs.empty()) continue;
-      // workgroups resident per CU: the tile's occupancy, or fewer when the
-      // units do not fill that many slots (a CU running one workgroup does not
-      // run it `occupancy` times slower; without this the FP32 form picked a
-      // 64 x 256 tile for 150 units of the chi = 1024 QN chain, 86 us against
-      // 40 us)
-      const int occ = int(std::max<int64_t>(
-          1, std::min<int64_t>(tile_occupancy(ti, prec, akc, bkc), (int64_t(costs.size()) + cus - 1) / cus)));
-      const double tt = lpt_makespan(costs, int64_t(cus) * occ) * occ / ts.eff32;
-      if (tt < best_t * 0.97) {
-        best_t = tt;
-        best = ti;
-      }
     }
   }
   return finalize(best, out);

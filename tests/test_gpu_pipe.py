@@ -15,8 +15,9 @@ SHAPES = [
 ]
 
 
-def _run(ctx, dev, shapes, aorder, border, tile, odd, alpha=1.5, beta=0.0):
+def _run(ctx, dev, shapes, aorder, border, tile, odd, alpha=1.5, beta=0.0, prec="f64"):
     """C (M x N) = alpha sum over tasks A_t B_t (+ beta C); several C blocks."""
+    eps = EPS if prec == "f64" else np.finfo(np.float32).eps
     rng = np.random.default_rng(len(shapes) + sum(map(sum, (s[1] for s in shapes))))
     A, B, offs, bA, bB, c0, refs = [], [], [], [], [], 0, []
     na = nb = 0
@@ -34,7 +35,7 @@ def _run(ctx, dev, shapes, aorder, border, tile, odd, alpha=1.5, beta=0.0):
             bound += np.abs(a) @ np.abs(b)
         refs.append((c0, ref, bound, sum(Ks)))
         c0 += M * N
-    p = ctx.plan_qn((-1, 1) if aorder == "km" else (1, -1), (-1, 2) if border == "kn" else (2, -1), (1, 2), offs, bA, bB)
+    p = ctx.plan_qn((-1, 1) if aorder == "km" else (1, -1), (-1, 2) if border == "kn" else (2, -1), (1, 2), offs, bA, bB, prec=prec)
     assert tile is None or p.info["tile"] == tile
     pad = np.zeros(odd)  # an operand 8 bytes off its allocation: single loads
     c = rng.standard_normal(c0)
@@ -43,7 +44,8 @@ def _run(ctx, dev, shapes, aorder, border, tile, odd, alpha=1.5, beta=0.0):
     got = dev.get(C, (c0,))
     for o, ref, bound, K in refs:
         x, y = (v[o:o + ref.size].reshape(ref.shape, order="F") for v in (got, c))
-        assert np.all(np.abs(x - alpha * ref - beta * y) <= (K + 70) * EPS * (alpha * bound + abs(beta * y)))
+        assert np.all(np.abs(x - alpha * ref - beta * y) <= (K + 70) * eps * (alpha * bound + abs(beta * y)))
+    return got
 
 
 @pytest.mark.parametrize("tile", [16, 17, None])
@@ -67,3 +69,15 @@ def test_pipe_beta(ctx, dev, monkeypatch, tile):
 ], ids=["tiny", "narrow"])
 def test_narrow_lists(ctx, dev, shapes):
     _run(ctx, dev, shapes, "mk", "kn", 5, 0)
+
+
+@pytest.mark.parametrize("aorder,border,odd", [("km", "kn", 0), ("km", "kn", 1), ("km", "nk", 0), ("mk", "kn", 0), ("mk", "nk", 1)])
+@pytest.mark.parametrize("shapes", SHAPES, ids=range(len(SHAPES)))
+def test_pipe_f32(ctx, dev, monkeypatch, shapes, aorder, border, odd):
+    """The FP32 tiles sum in one order: the same bits from all of them."""
+    got = []
+    for tile in (4, 16, 17, 18):
+        monkeypatch.setenv("ITX_FORCE_TILE", str(tile))
+        got.append(_run(ctx, dev, shapes, aorder, border, tile, odd, beta=0.25, prec="f32"))
+    for x in got[1:]:
+        assert np.array_equal(got[0], x)
