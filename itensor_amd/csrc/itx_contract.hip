@@ -717,115 +717,187 @@ __global__ __launch_bounds__(DG_NT, 2) void k_dgemm2(const double *__restrict__ 
   }
 }
 
-// ---- FP64 register-pipelined tiles of any size, layout and alignment ---------
-// The pipeline of k_dgemm (k order 4q + s) with (32 FM) x (32 FN) tiles.  Each
-// operand is loaded in aligned k pairs (V = 2, both operands), single elements
-// with the lanes along k (V = 1) or along the rows (V = 0: a wave takes four k
-// of a stage, so an operand contiguous along its rows coalesces).  Rows and
-// columns past the block load its last one and are not stored, so only the k
-// past the end has to be zeroed, in the last stages: in the steady state no
-// load or store has a condition, and they sit between the MFMAs by schedule
-// groups.  128 x 128 (FM = FN = 4): a stage is 1.87 us, 1.7 of it MFMA.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// The two BF16 terms of x and y (x in the low halves).  v_cvt_pk_bf16_f32
+// rounds to nearest even, as the integer form it replaced did for every float
+// but NaN, which now stays one.
+__device__ __forceinline__ void split_bf16x2(double x, double y, uint32_t &hi, uint32_t &lo) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  const f2 f{float(x), float(y)};
+  hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, b2));
+  const f2 r{f.x - __uint_as_float(hi << 16), f.y - __uint_as_float(hi & 0xFFFF0000u)};
+  lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, b2));
+}
+__device__ __forceinline__ void split_bf16(double x, unsigned short &hi, unsigned short &lo) {
+  uint32_t h, l;
+  split_bf16x2(x, 0.0, h, l);
+  hi = (unsigned short)h;
+  lo = (unsigned short)l;
+}
+
+// ---- register-pipelined tiles of any size, layout and alignment ---------------
+// The pipeline of k_dgemm in every form, with (32 FM) x (32 FN) tiles.  Each
+// operand is loaded in aligned runs of k (V = 2 or 4, both operands), single
+// elements with the lanes along k (V = 1) or along the rows (V = 0, so an
+// operand contiguous along its rows coalesces).  Rows and columns past the
+// block load its last one and are not stored, so only the k past the end has
+// to be zeroed, in the last stages: in the steady state no load or store has a
+// condition, and they sit between the MFMAs by schedule groups.
+// FP64 (k order 4q + s): a stage of 128 x 128 is 1.87 us, 1.7 of it MFMA.
 // 64 x 64: four times the units for products that leave CUs idle with the
 // larger tile, two workgroups per CU.  Dense chain, first and last stage, from
 // k_gemm / k_dgemm: chi = 1024 773 + 728 to 624 + 593 us (the matrix cores
 // need 563 each), chi = 512 136 + 148 to 100 + 96, chi = 255 28 + 43 to 26.5 +
 // 28.5.
-template <typename T, int ROWS, int V>
-struct PipeLoader {  // one operand: ROWS x 16 k per stage; V = 0: lanes along the rows, a few k each
-  static constexpr int LK = V ? DG_BK / (V ? V : 1) : DG_NT / (ROWS < 64 ? ROWS : 64);
-  static constexpr int RS = DG_NT / LK, NP = ROWS / RS, NK = V ? 1 : DG_BK / LK;
-  static constexpr int NR = ROWS / 16;                                      // doubles of a thread
-  static constexpr int NLD = V == 2 ? NR / 2 : NR;                          // loads
-  static constexpr int NST = V == 1 || sizeof(T) == 4 ? NR : NR / 2;        // LDS stores
+// FP32 (natural k order, the bits of k_gemm): operands arrive as FP64, so a
+// stage moves twice the bytes its MFMAs suggest; 128 x 128 1.13 us (0.82 of
+// MFMA), 64 x 64 0.33 with several workgroups on the CU, 0.43 alone.  chi = 512
+// 84 + 135 to 66 + 75 us, chi = 1024 596 + 539 to 380 + 350.  Stages of 32 k
+// gained 15% where one workgroup has a CU to itself and lost 5-10% elsewhere.
+// BF16x3 (bits of k_gemm3): the one wave of a SIMD also converts 32 elements a
+// lane and stage, about as long as its 48 MFMAs; 128 x 128 1.4 us for 32 k
+// (MFMA 0.32).  chi = 768 168 + 188 to 116 + 157 us, chi = 1024 343 + 289 to
+// 235 + 210.  Spreading the conversions over the stage by schedule groups made
+// 128 x 128 wait for its newest loads: 245 + 411 us.
+// T: double, float, or unsigned short for the two BF16 terms.  An LDS row:
+// the k of a stage; BF16x3 32 hi, then 32 lo terms (pitch 144 bytes).
+template <typename T>
+constexpr int kPipeBK = sizeof(T) == 2 ? 32 : DG_BK;
+template <typename T>
+constexpr int kPipePitch = sizeof(T) == 8 ? 18 : sizeof(T) == 4 ? 20 : 72;
+
+// One operand: ROWS rows of a stage; SP: pre-split words instead of FP64.
+template <typename T, int ROWS, int V, bool SP>
+struct PipeLoader {
+  using RT = std::conditional_t<SP, uint32_t, double>;
+  static constexpr int KB = kPipeBK<T>;
+  static constexpr int LK = V ? KB / (V ? V : 1) : DG_NT / (ROWS < 64 ? ROWS : 64);  // lanes along k
+  static constexpr int RS = DG_NT / LK, NP = ROWS / RS, NE = V ? V : KB / LK, NK = V ? 1 : NE;
+  static constexpr int NR = NP * NE;                                                 // elements of a thread
+  static constexpr int NLD = NR / (V == 0 ? 1 : SP ? V : V == 4 ? 2 : V);            // loads
+  static constexpr int NST = sizeof(T) == 8 ? (NE == 1 ? NR : NR / 2)                // LDS stores
+                             : sizeof(T) == 4 ? NR : 2 * NR / (NE < 4 ? NE : 4);
   int64_t roff[NP];
   int64_t ko[2][NK];  // k offsets of the next two stages to load (slot = stage & 1)
-  int lr, lc;
+  int lr, lc;         // first row; first k
   __device__ __forceinline__ void init(int tid, int row0, int R, const int64_t *__restrict__ tabR) {
-    lc = V ? tid % LK : NK * (RS == 64 ? __builtin_amdgcn_readfirstlane(tid / RS) : tid / RS);
+    lc = V ? V * (tid % LK) : NE * (RS == 64 ? __builtin_amdgcn_readfirstlane(tid / RS) : tid / RS);
     lr = V ? tid / LK : tid % RS;
 #pragma unroll
     for (int p = 0; p < NP; ++p) roff[p] = tabR[min(row0 + lr + RS * p, R - 1)];
   }
   __device__ __forceinline__ void fetch_k(int k0, int K, const int64_t *__restrict__ tabK, int slot) {
-    if constexpr (V) {
-      ko[slot][0] = tabK[min(k0 + V * lc, K - V)];
-    } else {
 #pragma unroll
-      for (int c = 0; c < NK; ++c) ko[slot][c] = tabK[min(k0 + lc + c, K - 1)];
-    }
+    for (int c = 0; c < NK; ++c) ko[slot][c] = tabK[min(k0 + lc + c, K - (V ? V : 1))];
   }
-  __device__ __forceinline__ void load(const double *__restrict__ base, double (&r)[NR], int slot) const {
+  __device__ __forceinline__ void load(const RT *__restrict__ base, RT (&r)[NR], int slot) const {
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-      if constexpr (V == 2) {
-        const double2 v = *reinterpret_cast<const double2 *>(base + roff[p] + ko[slot][0]);
-        r[2 * p] = v.x;
-        r[2 * p + 1] = v.y;
-      } else {
+      const RT *q = base + roff[p] + ko[slot][0];
+      if constexpr (V == 0) {
 #pragma unroll
         for (int c = 0; c < NK; ++c) r[NK * p + c] = (base + ko[slot][c])[roff[p]];
+      } else if constexpr (V == 1) {
+        r[p] = *q;
+      } else if constexpr (SP) {
+        const uint4 v = *reinterpret_cast<const uint4 *>(q);
+        r[4 * p] = v.x;
+        r[4 * p + 1] = v.y;
+        r[4 * p + 2] = v.z;
+        r[4 * p + 3] = v.w;
+      } else {
+#pragma unroll
+        for (int c = 0; c < V; c += 2) {
+          const double2 v = *reinterpret_cast<const double2 *>(q + c);
+          r[V * p + c] = v.x;
+          r[V * p + c + 1] = v.y;
+        }
       }
     }
   }
-  // where the fragment reads want k: FP64 k = 4q + s in the lanes of quarter
-  // q at MFMA s, FP32 k = 4s + q (the sums of k_gemm, to the last bit)
+  // Where the fragment reads want k: FP64 k = 4q + s in the lanes of quarter
+  // q at MFMA s, FP32 k = 4s + q (the sums of k_gemm, to the last bit).
   static __device__ __forceinline__ int place(int k) { return sizeof(T) == 8 ? k : 4 * (k & 3) + (k >> 2); }
   // k0: first k of the stage (TAIL: its k past K are zeroed)
   template <bool TAIL>
-  __device__ __forceinline__ void store(T *__restrict__ s, const double (&r)[NR], int k0, int K) const {
+  __device__ __forceinline__ void store(T *__restrict__ s, const RT (&r)[NR], int k0, int K) const {
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-      T *d = s + (lr + RS * p) * DgCfg<T>::P;
-      constexpr int NE = V == 2 ? 2 : NK;  // consecutive k of a thread
-#pragma unroll
-      for (int c = 0; c < NE; c += 2) {
-        const T x = !TAIL || k0 + (V ? V : 1) * lc + c < K ? T(r[NE * p + c]) : T(0);
+      T *d = s + (lr + RS * p) * kPipePitch<T>;
+      auto in = [&](int c) { return !TAIL || k0 + lc + c < K ? r[NE * p + c] : RT(0); };
+      if constexpr (sizeof(T) == 2) {
         if constexpr (NE == 1) {
-          d[place(lc)] = x;
-        } else {
-          const int k = (V ? V : 1) * lc + c;
-          const T y = !TAIL || k0 + k + 1 < K ? T(r[NE * p + c + 1]) : T(0);
-          if constexpr (sizeof(T) == 8) {
-            *reinterpret_cast<double2 *>(d + k) = double2{x, y};
+          uint32_t h = 0, l = 0;
+          if constexpr (SP) {
+            h = in(0);
+            l = h >> 16;
           } else {
-            d[place(k)] = x;
-            d[place(k + 1)] = y;
+            split_bf16x2(in(0), 0.0, h, l);
+          }
+          d[lc] = T(h);
+          d[KB + lc] = T(l);
+        } else {
+#pragma unroll
+          for (int c = 0; c < NE; c += 4) {
+            uint2 h, l;
+            if constexpr (SP) {
+              const uint32_t w0 = in(c), w1 = in(c + 1), w2 = in(c + 2), w3 = in(c + 3);
+              h = uint2{(w0 & 0xFFFFu) | (w1 << 16), (w2 & 0xFFFFu) | (w3 << 16)};
+              l = uint2{(w0 >> 16) | (w1 & 0xFFFF0000u), (w2 >> 16) | (w3 & 0xFFFF0000u)};
+            } else {
+              split_bf16x2(in(c), in(c + 1), h.x, l.x);
+              split_bf16x2(in(c + 2), in(c + 3), h.y, l.y);
+            }
+            *reinterpret_cast<uint2 *>(d + lc + c) = h;
+            *reinterpret_cast<uint2 *>(d + KB + lc + c) = l;
           }
         }
+      } else if constexpr (sizeof(T) == 8 && NE > 1) {
+#pragma unroll
+        for (int c = 0; c < NE; c += 2) *reinterpret_cast<double2 *>(d + lc + c) = double2{in(c), in(c + 1)};
+      } else {
+#pragma unroll
+        for (int c = 0; c < NE; ++c) d[place(lc + c)] = T(in(c));
       }
     }
   }
 };
 
 template <typename T, int F>
-struct PipeFrag {  // one operand of a stage: F fragments x 4 k
-  using Quad = std::conditional_t<sizeof(T) == 8, double2[2], float4>;
+struct PipeFrag {  // one operand of a stage: F fragments x 4 k (BF16x3: 8 k, both terms)
+  using Quad = std::conditional_t<sizeof(T) == 8, double2[2], std::conditional_t<sizeof(T) == 4, float4, bf16x8[2]>>;
   Quad x[F];
   __device__ __forceinline__ void read(const T *__restrict__ s, int row0, int lane) {
 #pragma unroll
     for (int j = 0; j < F; ++j) {
-      const T *p = s + (row0 + j * 16 + (lane & 15)) * DgCfg<T>::P + 4 * (lane >> 4);
+      const T *p = s + (row0 + j * 16 + (lane & 15)) * kPipePitch<T> + kPipeBK<T> / 4 * (lane >> 4);
       if constexpr (sizeof(T) == 8) {
         x[j][0] = *reinterpret_cast<const double2 *>(p);
         x[j][1] = *reinterpret_cast<const double2 *>(p + 2);
-      } else {
+      } else if constexpr (sizeof(T) == 4) {
         x[j] = *reinterpret_cast<const float4 *>(p);
+      } else {
+        x[j][0] = *reinterpret_cast<const bf16x8 *>(p);
+        x[j][1] = *reinterpret_cast<const bf16x8 *>(p + kPipeBK<T>);
       }
     }
   }
 };
 
-template <typename T, int FM, int FN, int VA, int VB>
+template <typename T, int FM, int FN, int VA, int VB, bool SP = false>
 __global__ __launch_bounds__(DG_NT, FM * FN <= 4 ? 2 : 1) void k_pipe(
     const double *__restrict__ A, const double *__restrict__ B, double *__restrict__ C,
     const GemmTask *__restrict__ tasks, const WorkUnit *__restrict__ units, int nunits, const int64_t *__restrict__ tab,
     double alpha, double beta) {
-  using v4 = typename MF<T>::v4;
-  constexpr int P = DgCfg<T>::P, BM = 32 * FM, BN = 32 * FN, NM = FM * FN;
-  constexpr int NRD = (sizeof(T) == 8 ? 2 : 1) * (FM + FN);  // LDS reads of a stage
-  using LA = PipeLoader<T, BM, VA>;
-  using LB = PipeLoader<T, BN, VB>;
+  using M = MF<std::conditional_t<sizeof(T) == 2, float, T>>;
+  using v4 = typename M::v4;
+  constexpr int P = kPipePitch<T>, KB = kPipeBK<T>, BM = 32 * FM, BN = 32 * FN;
+  constexpr int NM = sizeof(T) == 2 ? 3 * FM * FN / 4 : FM * FN;  // MFMAs of a quarter of a stage
+  constexpr int NRD = (sizeof(T) == 4 ? 1 : 2) * (FM + FN);  // LDS reads of a stage
+  using LA = PipeLoader<T, BM, VA, SP>;
+  using LB = PipeLoader<T, BN, VB, SP>;
   __shared__ __align__(16) T As[2][BM * P];
   __shared__ __align__(16) T Bs[2][BN * P];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -846,36 +918,46 @@ __global__ __launch_bounds__(DG_NT, FM * FN <= 4 ? 2 : 1) void k_pipe(
       LB lb;
       la.init(tid, wu.m0, tk.M, tab + tk.tAM);
       lb.init(tid, wu.n0, tk.N, tab + tk.tBN);
-      const double *Ab = A + tk.a_off;
-      const double *Bb = B + tk.b_off;
+      using RT = typename LA::RT;  // SP: the pointers are the split words, typed as FP64
+      const RT *Ab = reinterpret_cast<const RT *>(A) + tk.a_off;
+      const RT *Bb = reinterpret_cast<const RT *>(B) + tk.b_off;
       const int64_t *tAK = tab + tk.tAK;
       const int64_t *tBK = tab + tk.tBK;
-      const int K = tk.K, S = (K + DG_BK - 1) / DG_BK;
-      double ra0[LA::NR], rb0[LB::NR], ra1[LA::NR], rb1[LB::NR];  // load register sets
+      const int K = tk.K, S = (K + KB - 1) / KB;
+      RT ra0[LA::NR], rb0[LB::NR], ra1[LA::NR], rb1[LB::NR];  // load register sets
 #define ITX_PIPE_LOAD(st, ra, rb, slot)                   \
   {                                                       \
     la.load(Ab, ra, slot);                                \
     lb.load(Bb, rb, slot);                                \
-    la.fetch_k(((st) + 2) * DG_BK, K, tAK, slot);         \
-    lb.fetch_k(((st) + 2) * DG_BK, K, tBK, slot);         \
+    la.fetch_k(((st) + 2) * KB, K, tAK, slot);         \
+    lb.fetch_k(((st) + 2) * KB, K, tBK, slot);         \
   }
 #define ITX_PIPE_STORE(tail, st, ra, rb)                                  \
   {                                                                       \
-    la.template store<tail>(As[(st) & 1], ra, (st) * DG_BK, K);           \
-    lb.template store<tail>(Bs[(st) & 1], rb, (st) * DG_BK, K);           \
+    la.template store<tail>(As[(st) & 1], ra, (st) * KB, K);           \
+    lb.template store<tail>(Bs[(st) & 1], rb, (st) * KB, K);           \
   }
       PipeFrag<T, FM> fa0, fa1;
       PipeFrag<T, FN> fb0, fb1;
       auto mfma = [&](const PipeFrag<T, FM> &fa, const PipeFrag<T, FN> &fb, int s) __attribute__((always_inline)) {
+        if constexpr (sizeof(T) == 2) {  // a quarter of the fragments: the two cross terms, then hi * hi
 #pragma unroll
-        for (int i = 0; i < FN; ++i)
+          for (int e = 0; e < 3; ++e)
 #pragma unroll
-          for (int j = 0; j < FM; ++j) acc[i][j] = MF<T>::mma(dg_k(fb.x[i], s), dg_k(fa.x[j], s), acc[i][j]);
+            for (int h = s * FM * FN / 4; h < (s + 1) * FM * FN / 4; ++h)
+              acc[h / FM][h % FM] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  fb.x[h / FM][e == 1], fa.x[h % FM][e == 0], acc[h / FM][h % FM], 0, 0, 0);
+        } else {
+#pragma unroll
+          for (int i = 0; i < FN; ++i)
+#pragma unroll
+            for (int j = 0; j < FM; ++j) acc[i][j] = M::mma(dg_k(fb.x[i], s), dg_k(fa.x[j], s), acc[i][j]);
+        }
       };
       la.fetch_k(0, K, tAK, 0);
       lb.fetch_k(0, K, tBK, 0);
-      la.fetch_k(DG_BK, K, tAK, 1);
-      lb.fetch_k(DG_BK, K, tBK, 1);
+      la.fetch_k(KB, K, tAK, 1);
+      lb.fetch_k(KB, K, tBK, 1);
       ITX_PIPE_LOAD(0, ra0, rb0, 0)
       if (S > 1) ITX_PIPE_LOAD(1, ra1, rb1, 1)
       __syncthreads();  // the previous task's LDS reads are done
@@ -960,7 +1042,7 @@ __global__ __launch_bounds__(DG_NT, FM * FN <= 4 ? 2 : 1) void k_pipe(
         for (int r = 0; r < 4; ++r)
 #pragma unroll
           for (int j = 0; j < FM; ++j)
-            Pt[(wn + i * 16 + MF<T>::orow(lane, r)) * BM + wm + j * 16 + (lane & 15)] = acc[i][j][r];
+            Pt[(wn + i * 16 + M::orow(lane, r)) * BM + wm + j * 16 + (lane & 15)] = acc[i][j][r];
       continue;
     }
     const GemmTask t0 = tasks[wu.tbeg];
@@ -973,14 +1055,14 @@ __global__ __launch_bounds__(DG_NT, FM * FN <= 4 ? 2 : 1) void k_pipe(
 #pragma unroll
     for (int i = 0; i < FN; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) cn[i][r] = tCN[min(wu.n0 + wn + i * 16 + MF<T>::orow(lane, r), t0.N - 1)];
+      for (int r = 0; r < 4; ++r) cn[i][r] = tCN[min(wu.n0 + wn + i * 16 + M::orow(lane, r), t0.N - 1)];
 #pragma unroll
     for (int j = 0; j < FM; ++j)
 #pragma unroll
       for (int i = 0; i < FN; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int m = wu.m0 + wm + j * 16 + (lane & 15), n = wu.n0 + wn + i * 16 + MF<T>::orow(lane, r);
+          const int m = wu.m0 + wm + j * 16 + (lane & 15), n = wu.n0 + wn + i * 16 + M::orow(lane, r);
           if (m < t0.M && n < t0.N) {
             const int64_t ad = cm[j] + cn[i][r];
             double v = alpha * double(acc[i][j][r]);
@@ -1002,18 +1084,6 @@ __global__ __launch_bounds__(DG_NT, FM * FN <= 4 ? 2 : 1) void k_pipe(
 // the 16 rows read by a quarter-wave on distinct banks.
 constexpr int BK3 = 32;        // K depth of one LDS stage = one bf16 MFMA
 constexpr int LDK3 = BK3 + 8;  // bf16 elements per LDS row
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ uint32_t bf16_rne(uint32_t u) {  // upper 16 bits, round to nearest even
-  return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
-}
-__device__ __forceinline__ void split_bf16(double x, unsigned short &hi, unsigned short &lo) {
-  const float f = float(x);
-  const uint32_t h = bf16_rne(__float_as_uint(f));
-  const float rem = f - __uint_as_float(h << 16);
-  hi = (unsigned short)h;
-  lo = (unsigned short)bf16_rne(__float_as_uint(rem));
-}
 
 // The pre-split operand format: y[i] = hi | lo << 16 of split_bf16(x[i]).
 __global__ __launch_bounds__(256) void k_split_bf16(const double *__restrict__ x, uint32_t *__restrict__ y, size_t n) {
@@ -1123,15 +1193,13 @@ struct TileLoader3 {
 #pragma unroll
       for (int p = 0; p < NV; ++p) {
         const int idx = (lr + (NTH / LK) * p) * LDK3 + lk;
-        unsigned short h[4] = {0, 0, 0, 0}, l[4] = {0, 0, 0, 0};
+        uint2 h{0, 0}, l{0, 0};
         if (rok[p]) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) split_bf16(r[4 * p + e], h[e], l[e]);
+          split_bf16x2(r[4 * p], r[4 * p + 1], h.x, l.x);
+          split_bf16x2(r[4 * p + 2], r[4 * p + 3], h.y, l.y);
         }
-        *reinterpret_cast<uint2 *>(&sh[idx]) =
-            uint2{uint32_t(h[0]) | (uint32_t(h[1]) << 16), uint32_t(h[2]) | (uint32_t(h[3]) << 16)};
-        *reinterpret_cast<uint2 *>(&sl[idx]) =
-            uint2{uint32_t(l[0]) | (uint32_t(l[1]) << 16), uint32_t(l[2]) | (uint32_t(l[3]) << 16)};
+        *reinterpret_cast<uint2 *>(&sh[idx]) = h;
+        *reinterpret_cast<uint2 *>(&sl[idx]) = l;
       }
     } else {
 #pragma unroll
@@ -2166,6 +2234,22 @@ const void *gemm3_fn(bool akc, bool bkc, bool vec, bool split = false) {
              : reinterpret_cast<const void *>(&k_gemm3<BM, BN, GM, GN, false, false, 1>);
 }
 
+template <typename T, int FM, int FN>
+const void *pipe_fn(bool akc, bool bkc, bool vec, bool split = false) {
+  constexpr int V = sizeof(T) == 2 ? 4 : 2;
+  if constexpr (sizeof(T) == 2) {
+    if (split)
+      return vec ? reinterpret_cast<const void *>(&k_pipe<T, FM, FN, V, V, true>)
+                 : reinterpret_cast<const void *>(&k_pipe<T, FM, FN, 1, 1, true>);
+  }
+  if (akc && bkc && vec) return reinterpret_cast<const void *>(&k_pipe<T, FM, FN, V, V>);
+  if (akc)
+    return bkc ? reinterpret_cast<const void *>(&k_pipe<T, FM, FN, 1, 1>)
+               : reinterpret_cast<const void *>(&k_pipe<T, FM, FN, 1, 0>);
+  return bkc ? reinterpret_cast<const void *>(&k_pipe<T, FM, FN, 0, 1>)
+             : reinterpret_cast<const void *>(&k_pipe<T, FM, FN, 0, 0>);
+}
+
 const void *gemm3_fn_tile(int tile, bool akc, bool bkc, bool vec, bool split) {
   switch (tile) {
     case 0: return gemm3_fn<128, 128, 2, 2>(akc, bkc, vec, split);
@@ -2181,18 +2265,10 @@ const void *gemm3_fn_tile(int tile, bool akc, bool bkc, bool vec, bool split) {
     case 13: return gemm3_fn<64, 128, 2, 2>(akc, bkc, vec, split);
     case 14:
     case 15: return gemm3_fn<128, 128, 2, 2>(akc, bkc, vec, split);  // not chosen for BF16x3
+    case 16: return pipe_fn<unsigned short, 2, 2>(akc, bkc, vec, split);
+    case 17: return pipe_fn<unsigned short, 4, 4>(akc, bkc, vec, split);
     default: return gemm3_fn<32, 32, 2, 2>(akc, bkc, vec, split);
   }
-}
-
-template <typename T, int FM, int FN>
-const void *pipe_fn(bool akc, bool bkc, bool vec) {
-  if (akc && bkc && vec) return reinterpret_cast<const void *>(&k_pipe<T, FM, FN, 2, 2>);
-  if (akc)
-    return bkc ? reinterpret_cast<const void *>(&k_pipe<T, FM, FN, 1, 1>)
-               : reinterpret_cast<const void *>(&k_pipe<T, FM, FN, 1, 0>);
-  return bkc ? reinterpret_cast<const void *>(&k_pipe<T, FM, FN, 0, 1>)
-             : reinterpret_cast<const void *>(&k_pipe<T, FM, FN, 0, 0>);
 }
 
 template <typename T>
@@ -2359,6 +2435,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
   int64_t extA = 1, extB = 1, extC = 1;
   // A is read along k if its unit-stride digit is a contracted one (else
   // along m); likewise B.  Decided on the first non-empty task.
+  bool first_kc = false;  // of the first task
   double akc_work = 0, bkc_work = 0;  // multiply-adds of tasks with k-contiguous operands less those of the others
 
   double flops = 0;
@@ -2517,6 +2594,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     if (fi.empty) continue;
     // the tasks' common layout, by their work (K = 1 has none: at chi = 750
     // the first block of the chain's products is 1 x 1 x 1)
+    if (tasks.empty()) first_kc = fi.akc && fi.bkc;
     const double work = fi.K > 1 ? double(fi.M) * double(fi.N) * double(fi.K) : 0.0;
     akc_work += fi.akc ? work : -work;
     bkc_work += fi.bkc ? work : -work;
@@ -2612,8 +2690,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
   // tiles 14 and 15 need k-contiguous operands in aligned pairs
   const bool dg_ok = (prec == ITX_PREC_F64 || prec == ITX_PREC_F32) && akc && bkc && (vecbits & 1);
   auto tile_ok = [&](int t) {
-    return ((t != kDgemm && t != kDgemm2) || dg_ok) && ((t != kPipe64 && t != kPipe128) || prec != ITX_PREC_BF16X3) &&
-           (t != kPipe32 || prec == ITX_PREC_F32);
+    return ((t != kDgemm && t != kDgemm2) || dg_ok) && (t != kPipe32 || prec == ITX_PREC_F32);
   };
   // skinny plans whose tasks all have K, N <= 8 run k_skinny_q: two rows per thread
   const bool tinyq = maxN <= SKQ_N && maxK <= SKQ_K;
@@ -2839,6 +2916,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     p->prec = prec;
     p->tile = best;
     p->a_kcontig = akc;
+    p->split_ok = first_kc;
     p->b_kcontig = bkc;
     p->ntasks = int(vt.size());
     p->nunits = int(units.size());
@@ -2984,12 +3062,11 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     pool_free(ctx, bufC);
     ctx->tune[key] = best;
   } else {
-    if (prec != ITX_PREC_F64) {
+    if (prec == ITX_PREC_F32 && dg_ok) {
+      // Tile 14 where this model of the unpipelined tiles prefers it: it sums
+      // in another order than the rest.
       double best_t = 1e300;
-      // the 32-deep variants (11-13) are left to measurement (autotuner,
-      // ITX_FORCE_TILE): they only pay off for long K on large tiles
       for (int ti : {0, 1, 2, 3, 4, 6, 7, 8, 9, kDgemm}) {
-        if (ti == kDgemm && !dg_ok) continue;
         const TileCfg ts = kTiles[ti];
         std::vector<double> costs;
         int64_t n = 0;
@@ -3028,13 +3105,14 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     // 593; MPO stage, chi = 32 21.6, 18.4, 50.6; chi = 330 1274, 676, 574.
     // FP32, and 32 x 64 (before: 64 x 64 of k_gemm): last stage, chi = 256 37,
     // 35.4, 91.5, 28.4 (69); chi = 512 139, 77, 177, 77 (134); chi = 1024 876,
-    // 440, 358, 516 (579).  Tile 14, where it is the best of those before, sums
-    // in another order and stays.
+    // 440, 358, 516 (579).  BF16x3 (before: 64 x 64 of k_gemm3): chi = 256 23,
+    // 26, 53 (43); chi = 512 87, 53, 107 (85); chi = 1024 600, 315, 210 (343).
     struct Model {
       int tile, bm, bn;
       double alone, shared, any_alone, any_shared, per_task, per_unit;
     };
-    const double v1 = (vecbits & 1) ? 1.0 : prec == ITX_PREC_F64 ? 1.1 : 1.2;  // single loads
+    const bool vector = prec == ITX_PREC_BF16X3 ? vecbits & 2 : vecbits & 1;
+    const double v1 = vector ? 1.0 : prec == ITX_PREC_F64 ? 1.1 : prec == ITX_PREC_F32 ? 1.2 : 1.6;  // single loads
     const Model f64[] = {{4, 32, 32, 0.45, 0.28, 0.50, 0.50, 1, 1},
                          {kPipe64, 64, 64, 0.63 * v1, 0.50 * v1, 0.70, 0.88, 3, 2},
                          {kPipe128, 128, 128, 1.87 * v1, 1.87 * v1, 2.65, 2.65, 2, 1}};
@@ -3042,22 +3120,23 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
                          {kPipe32, 32, 64, 0.28 * v1, 0.21 * v1, 0.75, 0.85, 2, 1},
                          {kPipe64, 64, 64, 0.43 * v1, 0.33 * v1, 0.62, 0.83, 3, 2},
                          {kPipe128, 128, 128, 1.13 * v1, 1.13 * v1, 1.80, 2.05, 2, 1}};
-    const Model *models = prec == ITX_PREC_F64 ? f64 : f32;
-    const size_t nm = prec == ITX_PREC_F64 ? std::size(f64)
-                      : prec == ITX_PREC_F32 && best != kDgemm ? std::size(f32) : 0;
+    const Model bf[] = {{4, 32, 32, 0.28 * v1, 0.14 * v1, 0.45, 0.37, 1, 1},
+                        {kPipe64, 64, 64, 0.31 * v1, 0.235 * v1, 0.70, 0.73, 3, 2},
+                        {kPipe128, 128, 128, 0.65 * v1, 0.74 * v1, 1.65, 1.90, 2, 1}};
+    const Model *models = prec == ITX_PREC_F64 ? f64 : prec == ITX_PREC_F32 ? f32 : bf;
+    const size_t nm = best == kDgemm ? 0 : prec == ITX_PREC_F32 ? std::size(f32) : std::size(f64);
     if (nm) best = 4;
     double best_t = 1e300;
     for (const Model *md = models; md < models + nm; ++md) {
       std::vector<double> costs;
       int64_t n = 0;
-      double most = 0, bytes = 0;
+      double most = 0;
       const int ns = md->tile == kPipe64 ? pipe_split() : 1;
       for (auto &g : groups) {
         double c = md->per_unit;
         for (int t = g.tb; t < g.te; ++t) c += double((st[t].K + DG_BK - 1) / DG_BK) / ns + md->per_task;
         const int64_t tiles = int64_t((g.M + md->bm - 1) / md->bm) * ((g.N + md->bn - 1) / md->bn) * ns;
         most = std::max(most, c);
-        bytes += double(tiles) * g.ksum / ns * (md->bm + md->bn) * 8.0;
         n += tiles;
         if (groups.size() > 1) costs.insert(costs.end(), size_t(tiles), c);
       }
@@ -3065,9 +3144,6 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
       double tt = std::max(most * (kc ? md->alone : md->any_alone),
                            (costs.empty() ? lpt_makespan(n, most, cus) : lpt_makespan(costs, cus)) *
                                (kc ? md->shared : md->any_shared));
-      // what the L2s deliver, TB/s (chi = 1024: first stage 12.9, K = 1024;
-      // last stage 6.2, K = 5120)
-      tt = std::max(tt, bytes / (maxK > 2048 ? 6.2e6 : 12.9e6));
       if (ns > 1)  // the partial tiles and the second launch
         tt += 5.0 + double(ns) * groups[0].M * groups[0].N * 16.0 / 4e6;
       if (tt < best_t) {
@@ -3210,7 +3286,7 @@ int itx_plan_set_split(itx_ctx *ctx, itx_plan *plan, int on) {
   const bool want = on != 0;
   if (want == bool(plan->split)) return ITX_OK;
   if (want && (plan->prec != ITX_PREC_BF16X3 || plan->tile == itx::kSkinnyTile || plan->tile == 10 ||
-               !plan->a_kcontig || !plan->b_kcontig || plan->nred))
+               !plan->split_ok || plan->nred))
     return itx::set_err(ctx, ITX_ERR_UNSUPPORTED,
                         "itx_plan_set_split: pre-split operands need a BF16x3 MFMA plan with both operands "
                         "contiguous along the contracted index");

@@ -65,7 +65,8 @@ struct itx_plan {
   itx_ctx *ctx = nullptr;  // owner of the device block (its caching pool)
   int prec = ITX_PREC_F64;
   int tile = 0;        // index into the tile-shape table of the engine
-  bool a_kcontig = false, b_kcontig = false;
+  bool a_kcontig = false, b_kcontig = false;  // most of the work
+  bool split_ok = false;  // its first task has both (itx_plan_set_split)
   int ntasks = 0, nunits = 0;
   int grid = 0;
   double flops = 0;

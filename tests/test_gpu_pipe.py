@@ -17,7 +17,8 @@ SHAPES = [
 
 def _run(ctx, dev, shapes, aorder, border, tile, odd, alpha=1.5, beta=0.0, prec="f64"):
     """C (M x N) = alpha sum over tasks A_t B_t (+ beta C); several C blocks."""
-    eps = EPS if prec == "f64" else np.finfo(np.float32).eps
+    # BF16x3: both terms of an operand hold 16 bits, and lo * lo is dropped
+    eps = {"f64": EPS, "f32": np.finfo(np.float32).eps, "bf16x3": 2.0**-14}[prec]
     rng = np.random.default_rng(len(shapes) + sum(map(sum, (s[1] for s in shapes))))
     A, B, offs, bA, bB, c0, refs = [], [], [], [], [], 0, []
     na = nb = 0
@@ -73,11 +74,35 @@ def test_narrow_lists(ctx, dev, shapes):
 
 @pytest.mark.parametrize("aorder,border,odd", [("km", "kn", 0), ("km", "kn", 1), ("km", "nk", 0), ("mk", "kn", 0), ("mk", "nk", 1)])
 @pytest.mark.parametrize("shapes", SHAPES, ids=range(len(SHAPES)))
-def test_pipe_f32(ctx, dev, monkeypatch, shapes, aorder, border, odd):
-    """The FP32 tiles sum in one order: the same bits from all of them."""
+@pytest.mark.parametrize("prec,tiles", [("f32", (4, 16, 17, 18)), ("bf16x3", (4, 16, 17))])
+def test_pipe_same_bits(ctx, dev, monkeypatch, shapes, aorder, border, odd, prec, tiles):
+    """The FP32 and BF16x3 tiles sum in one order: the same bits from all of them."""
     got = []
-    for tile in (4, 16, 17, 18):
+    for tile in tiles:
         monkeypatch.setenv("ITX_FORCE_TILE", str(tile))
-        got.append(_run(ctx, dev, shapes, aorder, border, tile, odd, beta=0.25, prec="f32"))
+        got.append(_run(ctx, dev, shapes, aorder, border, tile, odd, beta=0.25, prec=prec))
     for x in got[1:]:
         assert np.array_equal(got[0], x)
+
+
+@pytest.mark.parametrize("tile", [16, 17])
+@pytest.mark.parametrize("M,N,K", [(65, 63, 32), (64, 70, 96), (130, 127, 35), (1, 1, 1)])
+def test_pipe_split_words(ctx, dev, monkeypatch, M, N, K, tile):
+    """Pre-split operands give the bits of the FP64 operands."""
+    monkeypatch.setenv("ITX_FORCE_TILE", str(tile))
+    rng = np.random.default_rng(M + N + K)
+    ops = [dev.put(rng.standard_normal(K * x)) for x in (M, N)]
+    words = [dev.empty(x.numel()) for x in ops]
+    for x, w in zip(ops, words):
+        ctx.split_bf16(x.data_ptr(), w.data_ptr(), x.numel())
+    p = ctx.plan_qn((-1, 1), (-1, 2), (1, 2), [0, 0, 0], [K, M], [K, N], prec="bf16x3")
+    C = dev.empty(M * N)
+    p.execute(ops[0].data_ptr(), ops[1].data_ptr(), C.data_ptr())
+    want = dev.get(C, (M * N,)).copy()
+    if K == 1:  # no contracted index: refused as before
+        with pytest.raises(Exception):
+            p.set_split(True)
+        return
+    p.set_split(True)
+    p.execute(words[0].data_ptr(), words[1].data_ptr(), C.data_ptr())
+    assert np.array_equal(want, dev.get(C, (M * N,)))
