@@ -88,7 +88,7 @@ def build_libitx(force: bool = True) -> str:
             f.result()
     tmp = out + ".tmp"
     # rocSOLVER (with rocBLAS) diagonalises the density-matrix blocks above
-    # 256 rows
+    # 512 rows
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", tmp, "-lrocsolver", "-lrocblas"])
     os.replace(tmp, out)
     return out

@@ -3141,9 +3141,10 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
         if (groups.size() > 1) costs.insert(costs.end(), size_t(tiles), c);
       }
       const bool kc = akc && bkc;
-      double tt = std::max(most * (kc ? md->alone : md->any_alone),
-                           (costs.empty() ? lpt_makespan(n, most, cus) : lpt_makespan(costs, cus)) *
-                               (kc ? md->shared : md->any_shared));
+      double tt = most * (kc ? md->alone : md->any_alone);
+      if (n > cus)
+        tt = std::max(tt, (costs.empty() ? lpt_makespan(n, most, cus) : lpt_makespan(costs, cus)) *
+                              (kc ? md->shared : md->any_shared));
       if (ns > 1)  // the partial tiles and the second launch
         tt += 5.0 + double(ns) * groups[0].M * groups[0].N * 16.0 / 4e6;
       if (tt < best_t) {
@@ -3157,7 +3158,11 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
       if ((fine ? n16 : n32) <= cus && 2.0 + (fine ? 1.35 : 2.2) * ((st[0].K + 127) / 128) < best_t) best = kSmall;
     }
   }
-  return finalize(best, out);
+  rc = finalize(best, out);
+  // the caller's scratch too small for the list of units: fewer, larger ones
+  if (rc == ITX_ERR_UNSUPPORTED && into && !force && best != kSkinny && best != kSmall)
+    rc = finalize(double(maxM) * double(maxN) <= 8192.0 ? kSmall : kPipe128, out);
+  return rc;
 }
 
 const void *plan_fn(const itx_plan *p, const double *A, const double *B) {
