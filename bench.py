@@ -251,7 +251,7 @@ def cpu_dmrg(N: int, maxdims):
 
 
 # kernels of the engine's tile indices that differ from the generic MFMA tile
-KERNEL_OF_TILE = {5: "k_skinny", 10: "k_small", 14: "k_dgemm", 15: "k_dgemm2"}
+KERNEL_OF_TILE = {5: "k_skinny", 10: "k_small", 14: "k_pipe", 15: "k_pipe", 16: "k_pipe", 17: "k_pipe", 18: "k_pipe"}
 
 
 def measured_traffic(chi: int, prec: str, stage: str):
@@ -466,6 +466,7 @@ def main():
                      "traffic_source": "profiles/pmc_dense_hpsi_chi1024.md (rocprofv3 FETCH_SIZE + WRITE_SIZE per "
                                        "dispatch, scaled by a 1 GiB copy: x2.0 / x1.0)",
                      "kernel": "%s (stage %d of %d of H*psi, tile %d)" % (
+                         "k_dgemm" if args.prec == "f32" and main_r["stage_tiles"][dom] in (14, 15) else
                          KERNEL_OF_TILE.get(main_r["stage_tiles"][dom], "k_gemm"), dom + 1, nst,
                          main_r["stage_tiles"][dom]),
                      "flops_per_launch": dom_flops, "avg_launch_ms": round(st[dom], 4)},
@@ -474,8 +475,8 @@ def main():
         # where this build's path differs from the north star's letter or the reference's algorithm
         "deviations": [
             "Davidson's small Rayleigh-Ritz eigenproblem (at most (niter+2)^2) is solved on the host in FP64",
-            "the density-matrix eigensolver runs its O(n^2) tridiagonal QL recurrence on host threads "
-            "(blocks up to 256 rows; reduction and rotations on the device); larger blocks go to rocSOLVER dsyevd",
+            "the density-matrix eigensolver runs on the device by divide and conquer up to 512 rows; "
+            "larger blocks go to rocSOLVER dsyevd",
             "the Hubbard MPO is the host AutoMPO's exact finite-state-machine MPO, not the reference's "
             "SVD-compressed one: the same operator, other link sectors",
             "a reduced-precision sweep reports the FP64 Rayleigh quotient of its last Ritz vector",
