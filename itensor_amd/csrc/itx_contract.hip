@@ -2847,10 +2847,14 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
       // chain, against the blocks from the heaviest down: 29.5 to 23.6, 23.4
       // to 19.3 and 38.6 to 28.4 us; up to a unit per CU it gains nothing.
       const size_t n = units.size();
-      std::array<std::vector<WorkUnit>, kXcds> lists;
+      std::vector<WorkUnit> su;
+      su.reserve(n);
       if (split || groups.size() == 1) {
-        for (size_t i = 0, chunk = (n + kXcds - 1) / kXcds; i < n; ++i) lists[i / chunk].push_back(units[i]);
+        const size_t chunk = (n + kXcds - 1) / kXcds;
+        for (size_t j = 0; j < chunk; ++j)
+          for (size_t i = j; i < n; i += chunk) su.push_back(units[i]);
       } else {
+        std::array<std::vector<WorkUnit>, kXcds> lists;
         std::vector<int> head(vt.size());  // a block's first task -> its place in `open`
         std::iota(head.begin(), head.end(), 0);
         std::vector<int> open(vt.size(), -1);  // the latest piece of a block, or of a set's tile of rows
@@ -2904,13 +2908,14 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
           for (size_t i = 0; i < n; ++i) turn[size_t(place[size_t(of[i])]++)] = int(i);
         }
         for (int i : turn) lists[size_t(xcd[size_t(of[size_t(i)])])].push_back(units[size_t(i)]);
+        std::array<size_t, kXcds> at{};
+        for (size_t i = 0; i < n; ++i) {
+          size_t x = i % kXcds;
+          for (size_t y = 0; at[x] == lists[x].size(); ++y) x = y;  // its list is used up: the next units of another
+          su.push_back(lists[x][at[x]++]);
+        }
       }
-      std::array<size_t, kXcds> at{};
-      for (size_t i = 0; i < n; ++i) {
-        size_t x = i % kXcds;
-        for (size_t y = 0; at[x] == lists[x].size(); ++y) x = y;  // its list is used up: the next units of another
-        units[i] = lists[x][at[x]++];
-      }
+      units.swap(su);
     }
     auto *p = new itx_plan();
     p->prec = prec;
@@ -3012,7 +3017,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
   for (auto &g : groups) {
     const double n = double((g.M + 31) / 32) * double((g.N + 31) / 32);
     n32 += n;
-    for (int t = g.tb; t < g.te; ++t) chunks += n * double((st[t].K + SM_K - 1) / SM_K);
+    for (int t = g.tb; t < g.te; ++t) chunks += n * double((st[t].K + 15) / 16);
   }
   const bool long_k = prec != ITX_PREC_F64 || (chunks > 4 * n32 && n32 <= cus);
   if (!st.empty() && !force && narrow && avg_rows >= 256) {
