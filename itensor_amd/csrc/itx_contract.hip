@@ -1443,8 +1443,10 @@ __global__ __launch_bounds__(SK_ROWS, 3) void k_skinny(const double *__restrict_
 // rows): a unit then sums many tiny tasks, and the per-task load round trip
 // and LDS barriers of k_skinny dominate.  Here the B tiles of as many tasks
 // as fit are staged in LDS at once (rows stacked), and the A elements of
-// SKQ_G tasks are loaded together before any is used.  Same accumulation
-// order as k_skinny (tasks in order, k in order), so the same results.
+// SKQ_G tasks are loaded together before any is used, those of the first
+// before B is staged.  Tasks in order, k in order.  Bound by the trips of a
+// unit (unit, tasks, tables, A and B, C) over two rounds of units: the MPO
+// stage of the chi = 1024 block-sparse chain 19.3 us for 26 MB.
 // Each thread computes two rows, SK_ROWS apart (units of 2 * SK_ROWS rows):
 // the per-unit task reads, B staging and barriers are shared by twice the
 // rows, and a thread has the loads of two rows in flight.
@@ -3316,7 +3318,7 @@ int itx_plan_set_split(itx_ctx *ctx, itx_plan *plan, int on) {
 
 int itx_plan_info(const itx_plan *plan, int *tile, int *form, int *ntasks, int *nunits) {
   if (!plan) return ITX_ERR_ARG;
-  // the skinny VALU path is HBM-bound and computes in FP64 in every form
+  // the skinny path is HBM-bound and computes in FP64 in every form
   const int f = plan->tile == itx::kSkinnyTile ? ITX_PREC_F64 : plan->prec;
   if (tile) *tile = plan->tile;
   if (form) *form = f;
