@@ -880,7 +880,7 @@ __global__ __launch_bounds__(ST) void k_syev_small(const TriTask *__restrict__ t
   __syncthreads();
   if (*st != 0) return;  // uniform
   const BackTask bt = back[b];
-  for (int c = QCB * (threadIdx.x >> 6); c < tk.n; c += QCB * (ST / 64)) back_run<1>(bt, c, W, W, A, out.rank);
+  for (int c = QCB * (threadIdx.x >> 6); c < tk.n; c += QCB * (ST / 64)) back_run<1, 4>(bt, c, W, W, A, out.rank);
 }
 
 }  // namespace

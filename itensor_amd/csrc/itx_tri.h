@@ -344,12 +344,14 @@ __device__ __forceinline__ void tri_run(const TriTask &tk, int g, const double *
 // X <- H_0 H_1 ... H_{n-3} X, one wave per QCB columns held in registers
 // (lanes over rows): the columns are independent, so a wave applies all
 // reflectors, last first, without meeting another one; the reflectors
-// stream from the L2, four of them under way (with one the trip to the L2
-// bounds the step: 78 us at n = 234).  Bound by the latency of a reflector: a
-// dot product, its sum over the lanes and an update.
-constexpr int QCB = 4, QPF = 4;
+// stream from the L2, QPF of them under way (with one the trip to the L2
+// bounds the step: 78 us at n = 234, 68 with four or eight).  Bound by the
+// latency of a reflector, 0.3 us: a dot product, its sum over the lanes and an
+// update.  RA = ceil(n / 64) exactly (with the next power of two and four
+// under way n = 300 took 177 us, now 101).
+constexpr int QCB = 4;
 
-template <int RA>
+template <int RA, int QPF>
 __device__ __forceinline__ void back_run(const BackTask &tk, int c0, const double *__restrict__ W,
                                          const double *__restrict__ S, double *__restrict__ O,
                                          const int *__restrict__ rank) {

@@ -40,14 +40,16 @@ __global__ __launch_bounds__(256) void k_back(const BackTask *__restrict__ tasks
   const BackTask tk = tasks[b.x];
   const int c0 = b.y + QCB * (threadIdx.x >> 6);
   if (c0 >= tk.n || status[b.x] != 0) return;  // no barrier below
-  if (tk.n <= 64)
-    back_run<1>(tk, c0, W, S, O, rank);
-  else if (tk.n <= 128)
-    back_run<2>(tk, c0, W, S, O, rank);
-  else if (tk.n <= 256)
-    back_run<4>(tk, c0, W, S, O, rank);
-  else
-    back_run<8>(tk, c0, W, S, O, rank);
+  switch ((tk.n + 63) / 64) {
+    case 1: return back_run<1, 8>(tk, c0, W, S, O, rank);
+    case 2: return back_run<2, 8>(tk, c0, W, S, O, rank);
+    case 3: return back_run<3, 8>(tk, c0, W, S, O, rank);
+    case 4: return back_run<4, 8>(tk, c0, W, S, O, rank);
+    case 5: return back_run<5, 8>(tk, c0, W, S, O, rank);
+    case 6: return back_run<6, 8>(tk, c0, W, S, O, rank);
+    case 7: return back_run<7, 8>(tk, c0, W, S, O, rank);
+    default: return back_run<8, 8>(tk, c0, W, S, O, rank);
+  }
 }
 
 }  // namespace
