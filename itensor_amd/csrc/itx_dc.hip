@@ -246,23 +246,24 @@ __device__ __forceinline__ void dc_small_run(const DcTask &tk, int sub, double *
 
   // the scale of T: its largest entry as a power of two, the same for every subtree
   double mx = 0.0;
-  bool bad = false;
+  bool nan = false;
   for (int e = lane; e < n; e += 64) {
     const double a = fabs(dv[e]), b = fabs(ev[e]);
-    bad = bad || !(a <= DBL_MAX) || !(b <= DBL_MAX);
+    nan = nan || a != a || b != b;
     mx = fmax(mx, fmax(a, b));
   }
-  if (__any(bad)) {  // not a number or infinite: no decomposition
-    if (tid == 0) atomicMax(status, 1);
-    mx = 0.0;
-  }
+  // not a number: no decomposition, except that a single row is its own
+  nan = __any(nan) && n > 1;
+  if (nan && tid == 0) atomicMax(status, 1);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
+  // beside an infinite entry every coupling is negligible: d as it stands
+  const bool loose = nan || !(mx <= DBL_MAX) || n == 1;
   int ex = 0;
-  if (mx > 0.0) (void)frexp(mx, &ex);
-  const bool dead = __any(bad);
-  auto scaled = [&](double v) { return dead ? 0.0 : ldexp(v, -ex); };
-  if (sub == 0 && tid == 0) aux[AUX_SCALE(n)] = dead ? 1.0 : ldexp(1.0, ex);
+  if (mx > 0.0 && !loose) (void)frexp(mx, &ex);
+  auto diagonal = [&](int g) { return loose ? (nan ? 0.0 : dv[g]) : ldexp(dv[g], -ex); };
+  auto coupling = [&](int g) { return loose ? 0.0 : ldexp(ev[g], -ex); };
+  if (sub == 0 && tid == 0) aux[AUX_SCALE(n)] = loose ? INFINITY : ldexp(1.0, ex);
 
   for (int x = tid; x < SB * SBP; x += ST) {
     Qa[x] = (x / SBP == x % SBP) ? 1.0 : 0.0;
@@ -272,7 +273,7 @@ __device__ __forceinline__ void dc_small_run(const DcTask &tk, int sub, double *
     double v = 0.0;
     if (i < cnt) {  // every boundary is torn: the diagonal loses both neighbours' |e|
       const int g = r0 + i;
-      v = scaled(dv[g]) - (g > 0 ? fabs(scaled(ev[g - 1])) : 0.0) - (g + 1 < n ? fabs(scaled(ev[g])) : 0.0);
+      v = diagonal(g) - (g > 0 ? fabs(coupling(g - 1)) : 0.0) - (g + 1 < n ? fabs(coupling(g)) : 0.0);
     }
     D[i] = v;
   }
@@ -288,7 +289,7 @@ __device__ __forceinline__ void dc_small_run(const DcTask &tk, int sub, double *
       ms = node_row(t, l, n, p) - r0;
       me = node_row(t + 1, l, n, p) - r0;
       md = node_row(2 * t + 1, l - 1, n, p) - r0;
-      if (md > ms && md < me) beta = scaled(ev[r0 + md - 1]);
+      if (md > ms && md < me) beta = coupling(r0 + md - 1);
     }
     // the rows of the merges that a wave's 16 columns belong to
     if (part == 0 && (i & 15) == 0) wspan[2 * (i >> 4)] = in ? ms : SB;
@@ -504,7 +505,7 @@ __global__ __launch_bounds__(PT) void k_dc_prep(const DcTask *__restrict__ tasks
   double *Q = W + tk.q_off + (par ? size_t(n) * n : 0) + size_t(r0) * n + r0;  // the merge's block
   const double *Dg = aux + AUX_D(n, par) + r0;
   const double scale = aux[AUX_SCALE(n)];
-  const double beta = W[tk.d_off + n + r0 + md - 1] / scale, rho = 2.0 * fabs(beta);
+  const double beta = scale <= DBL_MAX ? W[tk.d_off + n + r0 + md - 1] / scale : 0.0, rho = 2.0 * fabs(beta);
   for (int i = tid; i < m; i += PT) {
     double z = Q[size_t(i) * n + (i < md ? md - 1 : md)] * 0.70710678118654752440;
     if (i >= md && beta < 0.0) z = -z;
@@ -826,7 +827,7 @@ __device__ __forceinline__ void rank_run(const DcTask &tk, int index, double *__
   const int n = tk.n, tid = threadIdx.x;
   const double *aux = W + tk.x_off;
   const double *Dg = aux + AUX_D(n, tk.p > 6 ? (tk.p - 6) & 1 : 0);
-  const double scale = aux[AUX_SCALE(n)];
+  const double scaled = aux[AUX_SCALE(n)], scale = scaled <= DBL_MAX ? scaled : 1.0;
   for (int i = tid; i < n; i += blockDim.x) D[i] = Dg[i];
   __syncthreads();
   for (int i = tid; i < n; i += blockDim.x) {

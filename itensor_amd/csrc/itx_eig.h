@@ -153,7 +153,7 @@ __host__ __device__ constexpr size_t AUX_DS(int n) { return 2 * size_t(n); }    
 __host__ __device__ constexpr size_t AUX_ZS(int n) { return 3 * size_t(n); }            // their z
 __host__ __device__ constexpr size_t AUX_SEL(int n) { return 4 * size_t(n); }           // column of each (int)
 __host__ __device__ constexpr size_t AUX_K(int n) { return 5 * size_t(n); }             // poles of a merge (int)
-__host__ __device__ constexpr size_t AUX_SCALE(int n) { return 6 * size_t(n); }
+__host__ __device__ constexpr size_t AUX_SCALE(int n) { return 6 * size_t(n); }             // of d and e; infinite: unscaled, e ignored
 __host__ __device__ constexpr size_t AUX_SIZE(int n) { return 6 * size_t(n) + 2; }
 inline int dc_levels(int n) {
   int p = 0;

@@ -206,7 +206,8 @@ __device__ __forceinline__ void tri_run(const TriTask &tk, int g, const double *
     };
     const int q = k + 1;
     if constexpr (MULTI) {
-      const double pj = tau * wave_totals<XC>(y);
+      const double yt = wave_totals<XC>(y);
+      const double pj = tau != 0.0 ? tau * yt : 0.0;  // no reflector: also beside infinite entries
       if (lane % (64 / XC) == 0) {
         const int j = ci + cd * (lane / (64 / XC));
         if (j > k && j < n) publish(false, j, pj);
@@ -291,7 +292,7 @@ __device__ __forceinline__ void tri_run(const TriTask &tk, int g, const double *
         double ps = spk[i];
 #pragma unroll
         for (int w = 1; w < TNW; ++w) ps += spk[w * NR + i];
-        wp[a] = in ? tau * ps : 0.0;
+        wp[a] = in && tau != 0.0 ? tau * ps : 0.0;
       }
       c[a] = in ? sck[i] : 0.0;
       sm += v[a] * wp[a];

@@ -1,0 +1,50 @@
+"""The device eigensolver on entries outside the range of ordinary arithmetic,
+in one call with ordinary matrices."""
+import numpy as np
+import pytest
+
+from test_gpu_syev_dc import _check, _matrix, _solve
+
+pytestmark = pytest.mark.gpu
+
+
+def _check_diagonal(d, w, U):
+    """Exactly d in descending order, and the unit vectors that go with it."""
+    order = np.argsort(-d, kind="stable")
+    assert np.array_equal(w, d[order], equal_nan=True)
+    at = np.argmax(np.abs(U), axis=0)
+    assert np.array_equal(np.sort(at), np.arange(len(d)))
+    assert np.array_equal(np.abs(U), np.eye(len(d))[:, at])
+    assert np.array_equal(d[at], w, equal_nan=True)
+
+
+@pytest.mark.parametrize("x", [np.nan, np.inf, -np.inf, -3.0, 0.0, 5e-324])
+def test_syev_single_row(ctx, dev, x):
+    rng = np.random.default_rng(1)
+    mats = [np.array([[x]]), _matrix("random", 40, rng), np.array([[x]]), _matrix("random", 130, rng)]
+    got = _solve(ctx, dev, mats) if x == x else None
+    if got is None:  # the comparison of w and its host copy fails on not-a-number
+        A, w = dev.put(np.array([[x]])), dev.empty(1, fill=0.0)
+        ctx.syev(1, A.data_ptr(), w.data_ptr())
+        assert np.isnan(dev.get(w, (1,))[0]) and abs(dev.get(A, (1,))[0]) == 1.0
+        return
+    for X, (w, U) in zip(mats, got):
+        if len(X) == 1:
+            _check_diagonal(np.diag(X), w, U)
+        else:
+            _check(X, w, U)
+
+
+@pytest.mark.parametrize("n", [2, 3, 40, 64, 65, 100, 129, 200, 300])
+def test_syev_infinite_diagonal(ctx, dev, n):
+    rng = np.random.default_rng(n)
+    d = rng.permutation(np.arange(n) - n / 3.0)
+    d[rng.integers(n)] = np.inf
+    e = d.copy()
+    e[rng.integers(n)] = -np.inf
+    X = _matrix("random", 50, rng)
+    for M, (w, U) in zip((d, X, e), _solve(ctx, dev, [np.diag(d), X, np.diag(e)])):
+        if M is X:
+            _check(X, w, U)
+        else:
+            _check_diagonal(M, w, U)
