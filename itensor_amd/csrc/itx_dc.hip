@@ -261,6 +261,7 @@ __device__ __forceinline__ void dc_small_run(const DcTask &tk, int sub, double *
   const bool loose = nan || !(mx <= DBL_MAX) || n == 1;
   int ex = 0;
   if (mx > 0.0 && !loose) (void)frexp(mx, &ex);
+  ex = min(ex, 1023);  // 2^ex is a number too
   auto diagonal = [&](int g) { return loose ? (nan ? 0.0 : dv[g]) : ldexp(dv[g], -ex); };
   auto coupling = [&](int g) { return loose ? 0.0 : ldexp(ev[g], -ex); };
   if (sub == 0 && tid == 0) aux[AUX_SCALE(n)] = loose ? INFINITY : ldexp(1.0, ex);

@@ -1119,7 +1119,7 @@ int syev_dc_finish(itx_ctx *ctx, const DcCall &call, const int32_t *ns, const in
     const DcTask &t = call.tasks[i];
     const int b = call.mat[i];
     if (call.hstatus[i] == 1)
-      return set_err(ctx, ITX_ERR_NOCONV, "itx_syev: the matrix holds values that are not finite");
+      return set_err(ctx, ITX_ERR_NOCONV, "itx_syev: the reduction met values that are not a number");
     if (call.hstatus[i] == 2) {  // A is untouched: the path without meetings
       rn.push_back(ns[b]);
       ra.push_back(aoffs[b]);

@@ -48,3 +48,14 @@ def test_syev_infinite_diagonal(ctx, dev, n):
             _check(X, w, U)
         else:
             _check_diagonal(M, w, U)
+
+
+@pytest.mark.parametrize("n", [1, 2, 40, 100, 200])
+def test_syev_largest_numbers(ctx, dev, n):
+    """Entries of 2^1023 and more, whose scale as a power of two would not be a number."""
+    d = np.linspace(-1.75, 1.75, n) if n > 1 else np.array([1.5])
+    (w, U), = _solve(ctx, dev, [np.diag(d) * 2.0**1023])
+    assert np.array_equal(w, np.sort(d)[::-1] * 2.0**1023)
+    if n > 1:
+        (w, U), = _solve(ctx, dev, [np.array([[1.0, 0.25], [0.25, 1.0]]) * 2.0**1023])
+        assert np.max(np.abs(w * 2.0**-1023 - [1.25, 0.75])) <= 64 * np.finfo(float).eps
