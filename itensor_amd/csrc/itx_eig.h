@@ -118,16 +118,25 @@ struct TriTask {
 constexpr int TRI_MAX = 512;  // largest order
 // exchange doubles of a matrix of order n
 size_t tri_exchange(int n);
+// How long a workgroup waits for the others of its matrix: 2^20 polls, about
+// a second.  ITX_EIG_WAIT=polls[,1] shortens it for tests (0: every wait is
+// given up at once; 1: the last workgroup of each matrix is not launched).
+struct TriWait {
+  int polls = 1 << 20;
+  bool absent = false;
+};
+TriWait tri_wait();
 // Sets the workgroup count of the first ntasks tasks and lists the
 // workgroups (task, workgroup) in launch order; ends: the end of each launch
 // in the list.
-void tri_blocks(std::vector<TriTask> &tasks, int ntasks, int cus, std::vector<int2> &blocks, std::vector<size_t> &ends);
+void tri_blocks(std::vector<TriTask> &tasks, int ntasks, int cus, bool absent, std::vector<int2> &blocks,
+                std::vector<size_t> &ends);
 // Reduces every task: T = Q^T A Q, Q = H_0 H_1 ... H_{n-3}, H_k = I - tau_k
 // v_k v_k^T.  tasks, blocks: device copies; W: workspace, whose exchange
 // area is the nx doubles at x_off; status: one int per task (zero before the
 // call), set to 2 where the workgroups of a matrix did not meet.
 void tri_launch(itx_ctx *ctx, const TriTask *tasks, const int2 *blocks, const std::vector<size_t> &ends,
-                const double *A, double *W, int64_t x_off, size_t nx, int *status);
+                const double *A, double *W, int64_t x_off, size_t nx, int polls, int *status);
 // O <- Q S for the n x n matrix of every task: column c of S (at s_off) goes
 // to column rank[r_off + c] of O.  Tasks with a status are left out.
 struct BackTask {

@@ -1047,7 +1047,8 @@ int syev_dc_launch(itx_ctx *ctx, std::vector<int> mats, const int32_t *ns, const
   std::vector<int2> tb, db, bb;
   std::vector<size_t> ends;
   std::vector<DcLevel> levels;
-  tri_blocks(tri, nb, std::max(1, ctx->num_cus), tb, ends);
+  const TriWait wait = tri_wait();
+  tri_blocks(tri, nb, std::max(1, ctx->num_cus), wait.absent, tb, ends);
   dc_blocks(call.tasks, nb, db, levels);
   back_blocks(back, nb, bb);
   int rc = eig_host(ctx, sizeof(double) * size_t(neig) + sizeof(int) * size_t(nt));
@@ -1092,7 +1093,8 @@ int syev_dc_launch(itx_ctx *ctx, std::vector<int> mats, const int32_t *ns, const
   const DcTask *ddc = reinterpret_cast<const DcTask *>(at(2));
   const BackTask *dback = reinterpret_cast<const BackTask *>(at(4));
   syev_small_launch(ctx, dtri, ddc, dback, nb, nt - nb, Abase, W, Wbase, out);
-  tri_launch(ctx, dtri, reinterpret_cast<const int2 *>(at(1)), ends, Abase, W, x0, size_t(xsize), status);
+  tri_launch(ctx, dtri, reinterpret_cast<const int2 *>(at(1)), ends, Abase, W, x0, size_t(xsize), wait.polls,
+             status);
   dc_launch(ctx, ddc, nb, reinterpret_cast<const int2 *>(at(3)), levels, W, Wbase, out);
   back_launch(ctx, dback, reinterpret_cast<const int2 *>(at(5)), bb.size(), W, W, Abase, rank, status);
   pool_free(ctx, ws);  // stream-ordered

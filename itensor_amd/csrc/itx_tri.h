@@ -29,9 +29,12 @@ namespace {
 // meet in global memory: every value has its own place per step, filled with
 // a mark before the launch, and a reader polls the value itself until the
 // mark is gone -- one trip through memory instead of data, flag and data
-// again.  All values go through agent-scope atomics.  A wait is bounded;
-// workgroups that give up set the status and run to the end without waiting
-// again, and the host takes another path.
+// again.  All values go through agent-scope atomics.  A wait is bounded: a
+// lane that gives up sets the matrix's status and a mark of its workgroup, the
+// waiting lanes of other workgroups look at the status now and then, and a
+// workgroup that is marked runs to the end without waiting again, so that a
+// workgroup that never runs costs one bound and not one per step.  The host
+// then takes another path.
 // What bounds it is the latency of the n - 2 dependent steps: in one
 // workgroup 1.15 us a step at n = 64 and 1.6 at 128 (72 and 203 us in all;
 // the LDS-resident form before this one 174 and 519), across workgroups 2.8
@@ -42,7 +45,7 @@ constexpr int TNW = 4;            // waves per workgroup
 constexpr int TNT = 64 * TNW;
 constexpr int TXC = 4;            // columns per wave across workgroups
 constexpr unsigned long long TRI_MARK = 0x7FF8DEADBEEF4242ull;  // a quiet NaN no arithmetic makes
-constexpr int TRI_SPIN = 1 << 20;
+constexpr int TRI_LOOK = 1024;  // polls between looks at the status
 
 template <int RA, bool MULTI>
 constexpr int tri_lds() {  // doubles: per wave v, (v, w); twice p and column
@@ -51,7 +54,8 @@ constexpr int tri_lds() {  // doubles: per wave v, (v, w); twice p and column
 
 template <int RA, bool MULTI>
 __device__ __forceinline__ void tri_run(const TriTask &tk, int g, const double *__restrict__ Abase,
-                                        double *__restrict__ W, int *__restrict__ status, double *__restrict__ lds) {
+                                        double *__restrict__ W, int *__restrict__ status, double *__restrict__ lds,
+                                        int polls = 0, int *gave = nullptr) {
   constexpr int NR = 64 * RA;
   // rows and columns of the matrix that a thread holds
   constexpr int XR = MULTI ? RA : 4 * RA, XC = MULTI ? TXC : 4 * RA;
@@ -242,12 +246,16 @@ __device__ __forceinline__ void tri_run(const TriTask &tk, int g, const double *
       constexpr int U = 2 * NR / TNT;
       const int L = n - k - 1;
       unsigned long long b[U];
-      int spin = 0;
-      bool more;
 #pragma unroll
       for (int u = 0; u < U; ++u) b[u] = TRI_MARK;
-      do {
-        more = false;
+      for (int spin = 0; !dead; ++spin) {
+        if (spin >= polls || (spin % TRI_LOOK == TRI_LOOK - 1 &&
+                              __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+          *gave = 1;
+          atomicExch(status, 2);
+          break;
+        }
+        bool more = false;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           const int e = tid + TNT * u;
@@ -257,9 +265,8 @@ __device__ __forceinline__ void tri_run(const TriTask &tk, int g, const double *
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) more = more || (tid + TNT * u < 2 * L && b[u] == TRI_MARK);
-        if (more && ++spin > TRI_SPIN) dead = true;
-      } while (more && !dead);
-      if (more) atomicExch(status, 2);
+        if (!more) break;
+      }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int e = tid + TNT * u;
@@ -267,6 +274,7 @@ __device__ __forceinline__ void tri_run(const TriTask &tk, int g, const double *
       }
     }
     lds_barrier();
+    if constexpr (MULTI) dead = *gave != 0;
     // results of step k, stored here so that the trip through memory passes
     // behind the arithmetic and not before the next values are waited for
     if (MULTI ? gw == (qw ? qw - 1 : NWV - 1) : wave == (k & (TNW - 1))) {

@@ -1,6 +1,7 @@
 // Householder tridiagonal form of symmetric matrices, and products with its
 // orthogonal factor: the dense O(n^3) parts of the symmetric eigensolver.
 #include <algorithm>
+#include <cstdlib>
 
 #include "itx_tri.h"
 
@@ -10,20 +11,23 @@ namespace {
 // blocks[b] = (task, workgroup of the task)
 __global__ __launch_bounds__(TNT) void k_tridiag(const TriTask *__restrict__ tasks, const int2 *__restrict__ blocks,
                                                  const double *__restrict__ A, double *__restrict__ W,
-                                                 int *__restrict__ status) {
+                                                 int *__restrict__ status, int polls) {
   __shared__ __align__(16) double lds[tri_lds<8, true>()];
+  __shared__ int gave;  // a wave of this workgroup has given up a wait
   static_assert(tri_lds<8, true>() >= tri_lds<2, false>() && tri_lds<8, true>() >= tri_lds<4, true>(), "LDS of a class");
   const int2 b = blocks[blockIdx.x];
   const TriTask tk = tasks[b.x];
   int *st = status + b.x;
+  if (threadIdx.x == 0) gave = 0;
+  __syncthreads();
   if (tk.n <= 64)
     tri_run<1, false>(tk, 0, A, W, st, lds);
   else if (tk.n <= 128)
     tri_run<2, false>(tk, 0, A, W, st, lds);
   else if (tk.n <= 256)
-    tri_run<4, true>(tk, b.y, A, W, st, lds);
+    tri_run<4, true>(tk, b.y, A, W, st, lds, polls, &gave);
   else
-    tri_run<8, true>(tk, b.y, A, W, st, lds);
+    tri_run<8, true>(tk, b.y, A, W, st, lds, polls, &gave);
 }
 
 __global__ void k_mark(double *x, size_t n) {
@@ -58,7 +62,18 @@ static int tri_wgs(int n) { return n <= 128 ? 1 : (n + TNW * TXC - 1) / (TNW * T
 
 size_t tri_exchange(int n) { return n <= 128 ? 0 : size_t(n - 2) * 2 * size_t(n); }
 
-void tri_blocks(std::vector<TriTask> &tasks, int ntasks, int cus, std::vector<int2> &blocks, std::vector<size_t> &ends) {
+TriWait tri_wait() {
+  TriWait w;
+  if (const char *v = std::getenv("ITX_EIG_WAIT")) {
+    char *end = nullptr;
+    w.polls = int(std::min(std::max(std::strtol(v, &end, 10), 0l), long(w.polls)));
+    if (*end == ',') w.absent = std::atoi(end + 1) != 0;
+  }
+  return w;
+}
+
+void tri_blocks(std::vector<TriTask> &tasks, int ntasks, int cus, bool absent, std::vector<int2> &blocks,
+                std::vector<size_t> &ends) {
   // Workgroups that meet come first, in launches of at most one workgroup
   // per CU, so that all of a launch are resident together.
   if (ntasks == 0) return;
@@ -76,13 +91,13 @@ void tri_blocks(std::vector<TriTask> &tasks, int ntasks, int cus, std::vector<in
       meet = 0;
     }
     if (g > 1) meet += g;
-    for (int b = 0; b < g; ++b) blocks.push_back(make_int2(i, b));
+    for (int b = 0; b < (absent && g > 1 ? g - 1 : g); ++b) blocks.push_back(make_int2(i, b));
   }
   ends.push_back(blocks.size());
 }
 
 void tri_launch(itx_ctx *ctx, const TriTask *tasks, const int2 *blocks, const std::vector<size_t> &ends,
-                const double *A, double *W, int64_t x_off, size_t nx, int *status) {
+                const double *A, double *W, int64_t x_off, size_t nx, int polls, int *status) {
   if (nx)
     hipLaunchKernelGGL(k_mark, dim3(unsigned(std::min<size_t>((nx + 255) / 256, size_t(ctx->num_cus) * 8))), dim3(256),
                        0, ctx->stream, W + x_off, nx);
@@ -90,7 +105,7 @@ void tri_launch(itx_ctx *ctx, const TriTask *tasks, const int2 *blocks, const st
   for (size_t e : ends) {
     if (e > start)
       hipLaunchKernelGGL(k_tridiag, dim3(unsigned(e - start)), dim3(TNT), 0, ctx->stream, tasks, blocks + start, A, W,
-                         status);
+                         status, polls);
     start = e;
   }
 }
