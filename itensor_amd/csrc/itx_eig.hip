@@ -40,7 +40,10 @@ namespace {
 
 constexpr int ET = 512;       // threads per matrix of the batched global-memory reduction
 constexpr int EMAX = 2048;    // largest n
-constexpr int QL_MAXIT = 60;  // QL sweeps per eigenvalue before giving up
+// QL sweeps per eigenvalue before giving up, and n more: the first eigenvalues
+// of a large matrix with two eigenvalues only take up to n / 5 (86 at n = 512,
+// 211 at 1024).
+constexpr int QL_MAXIT = 60;
 
 struct EigTask {
   int32_t n, pad;
@@ -498,7 +501,7 @@ bool host_ql(int n, double *d, double *e, std::vector<double2> &rots) {
       for (; m < n - 1; ++m)
         if (std::fabs(e[m]) <= DBL_EPSILON * std::max(std::fabs(d[m]) + std::fabs(d[m + 1]), tst1)) break;
       if (m == l) break;
-      if (iter++ >= QL_MAXIT) return false;
+      if (iter++ >= QL_MAXIT + n) return false;
       double g = (d[l + 1] - d[l]) / (2.0 * e[l]);
       double r = pyth(g, 1.0);
       g = d[m] - d[l] + e[l] / (g + std::copysign(r, g));
