@@ -3022,15 +3022,19 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     for (int t = g.tb; t < g.te; ++t) chunks += n * double((st[t].K + 15) / 16);
   }
   const bool long_k = prec != ITX_PREC_F64 || (chunks > 4 * n32 && n32 <= cus);
+  // what a forced tile or a table entry must meet; an entry is shared by all
+  // sizes of its class, aligned and not
+  auto usable = [&](int t) { return t >= 0 && t < kNumTiles && (t != kSkinny || narrow) && tile_ok(t); };
+  const auto tuned = ctx->tune.find(key);
   if (!st.empty() && !force && narrow && avg_rows >= 256) {
     best = kSkinny;
   } else if (!st.empty() && !force && double(maxM) * double(maxN) <= 8192.0) {
     best = long_k ? kSmall : 4;
   } else if (force) {
     best = std::atoi(force);
-    if (best < 0 || best >= kNumTiles || (best == kSkinny && !narrow) || !tile_ok(best)) best = 0;
-  } else if (ctx->tune.count(key)) {
-    best = ctx->tune[key];
+    if (!usable(best)) best = 0;
+  } else if (tuned != ctx->tune.end() && usable(tuned->second)) {
+    best = tuned->second;
   } else if (ctx->autotune && !into && !st.empty()) {
     void *bufA = nullptr, *bufB = nullptr, *bufC = nullptr;
     int rc2 = pool_alloc(ctx, sizeof(double) * size_t(extA), &bufA);
@@ -3045,6 +3049,8 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     float best_ms = 1e30f;
     for (int ti = 0; ti < kNumTiles; ++ti) {
       if (ti == kSkinny || ti == kSmall) continue;
+      // in FP64 the kernel of kPipe128, which takes any alignment
+      if (prec == ITX_PREC_F64 && (ti == kDgemm || ti == kDgemm2)) continue;
       itx_plan *pc = nullptr;
       if (finalize(ti, &pc)) continue;
       const double *A = static_cast<const double *>(bufA), *B = static_cast<const double *>(bufB);
