@@ -133,8 +133,10 @@ int itx_contract_qn(itx_ctx *ctx,
  * and split-K partial tiles go into a static device array of the library,
  * 32 MiB per device, which each device holds until the process ends; a
  * contraction whose plan needs more returns ITX_ERR_UNSUPPORTED (the
- * message names both sizes).  The tile comes from the tuning table or the
- * cost model, never from the autotuner.  Every call on a device shares
+ * message names both sizes).  The result is itx_contract_qn's bit for bit
+ * where the array holds that call's plan; where it does not, partial tiles
+ * are given up first.  The tile comes from the tuning table or the cost
+ * model, never from the autotuner.  Every call on a device shares
  * that device's array: calls on one stream are ordered, calls that overlap
  * on one device (other contexts or streams) race.  Nothing in the array
  * needs to start at zero. */

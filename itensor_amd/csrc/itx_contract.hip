@@ -2696,11 +2696,11 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
   };
   // skinny plans whose tasks all have K, N <= 8 run k_skinny_q: two rows per thread
   const bool tinyq = maxN <= SKQ_N && maxK <= SKQ_K;
+  bool lean = false;  // a caller's scratch is too small for more and finer units
   // Units over k of the 64 x 64 tile for one product: as many as give every
-  // CU two workgroups, with at least 8 stages each (none where the scratch is
-  // the caller's).
+  // CU two workgroups, with at least 8 stages each.
   auto pipe_split = [&]() {
-    if (st.size() != 1 || into || prec != ITX_PREC_F64) return 1;  // FP32 sums keep their order
+    if (st.size() != 1 || lean || prec != ITX_PREC_F64) return 1;  // FP32 sums keep their order
     const int64_t tiles = int64_t((st[0].M + 63) / 64) * ((st[0].N + 63) / 64);
     const int64_t most = std::min<int64_t>(2 * cus / std::max<int64_t>(tiles, 1), st[0].K / (8 * DG_BK));
     return int(std::max<int64_t>(1, std::min<int64_t>(most, 64)));
@@ -2711,7 +2711,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     const int tbm0 = (best == kSkinny && tinyq) ? SKQ_R * SK_ROWS : kTiles[best].bm;
     const int tbn0 = (best == kSkinny) ? std::max(1, maxN) : kTiles[best].bn;
     int tbm = tbm0, tbn = tbn0;
-    if (best == kSmall && prec == ITX_PREC_F64 && !into) {
+    if (best == kSmall && prec == ITX_PREC_F64 && !lean) {
       // Smaller units while they leave CUs idle: a unit's k loop is bound by
       // the matrix cores of one CU (64 x 32 outputs: 32 cycles a k), its loads
       // by its rows, so two units of half the size take half the time.  One
@@ -3172,9 +3172,15 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     }
   }
   rc = finalize(best, out);
-  // the caller's scratch too small for the list of units: fewer, larger ones
-  if (rc == ITX_ERR_UNSUPPORTED && into && !force && best != kSkinny && best != kSmall)
-    rc = finalize(double(maxM) * double(maxN) <= 8192.0 ? kSmall : kPipe128, out);
+  // The plan of the ordinary call, and so its sums, wherever the caller's
+  // scratch holds it; else without partial tiles, then in larger units.
+  if (rc == ITX_ERR_UNSUPPORTED && into) {
+    lean = true;
+    rc = finalize(best, out);
+    const bool small = double(maxM) * double(maxN) <= 8192.0;
+    if (rc == ITX_ERR_UNSUPPORTED && !force && best != kSkinny && !(small && best == kSmall))
+      rc = finalize(small ? kSmall : kPipe128, out);
+  }
   return rc;
 }
 

@@ -182,7 +182,8 @@ constexpr int HRES_SLOTS = 64;  // pinned result slots (multi-dot up to 16)
 // unit lists, offset tables, split-K partial tiles -- is laid out there
 // instead of in the caching pool, and the tile comes from the tuning table
 // or the cost model (the autotuner, which allocates, is skipped); a plan
-// that does not fit fails with ITX_ERR_UNSUPPORTED.
+// that does not fit is laid out again with fewer partial tiles and units, and
+// fails with ITX_ERR_UNSUPPORTED if that does not fit either.
 int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t *labB,
                int rC, const int32_t *labC, int ntasks, const int64_t *offs,
                const int64_t *blkA, const int64_t *blkB, const int64_t *blkC_or_null,
