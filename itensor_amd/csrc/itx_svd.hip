@@ -25,7 +25,6 @@
 namespace itx {
 namespace {
 
-constexpr int ST = 1024;            // threads per matrix
 constexpr int SVD_MAX_SWEEPS = 60;  // sweeps before reporting no convergence
 // X and J in LDS (columns at odd pitches) when they fit, else in the workspace
 constexpr size_t SVD_LDS = 160 * 1024 - 512;  // of 160 KB: 100 x 100 fits
@@ -57,8 +56,9 @@ __device__ __forceinline__ void group_sums(double &a, double &b, double &c) {
 // independent pairs, so a round's latency bounds it: a pair has up to 64
 // lanes, its columns come from LDS where the matrix fits, and a barrier
 // orders LDS only (blocks up to 37 x 37: 0.42 ms for some 10 sweeps, 1.1 us
-// a round; from the workspace, with 256 threads, 1.14 ms).
-template <bool LDS, int G>
+// a round; from the workspace, with 256 threads, 1.14 ms).  ST: threads per
+// matrix, 1024 or, for large batches of small matrices, 256.
+template <int ST, bool LDS, int G>
 __device__ __forceinline__ void gesvd_run(const SvdTask &tk, const double *__restrict__ Abase,
                                           double *__restrict__ Ubase, double *__restrict__ Sbase,
                                           double *__restrict__ Vbase, double *__restrict__ Wbase,
@@ -236,6 +236,7 @@ __device__ __forceinline__ void gesvd_run(const SvdTask &tk, const double *__res
   if (tid == 0) *status = 0;
 }
 
+template <int ST>
 __global__ __launch_bounds__(ST) void k_gesvd(const SvdTask *__restrict__ tasks, const double *__restrict__ Abase,
                                               double *__restrict__ Ubase, double *__restrict__ Sbase,
                                               double *__restrict__ Vbase, double *__restrict__ Wbase,
@@ -250,24 +251,33 @@ __global__ __launch_bounds__(ST) void k_gesvd(const SvdTask *__restrict__ tasks,
   }
   // as many lanes per pair as the threads allow for all pairs of a round
   const int P = (min(tk.m, tk.n) + 1) / 2;
-  const bool in = svd_lds(tk.m, tk.n) <= lds_bytes;
-#define ITX_SVD(L, G) gesvd_run<L, G>(tk, Abase, Ubase, Sbase, Vbase, Wbase, st, lds, sh_rot)
-  if (in && P * 64 <= ST)
-    ITX_SVD(true, 64);
-  else if (in && P * 32 <= ST)
-    ITX_SVD(true, 32);
-  else if (in && P * 16 <= ST)
-    ITX_SVD(true, 16);
-  else if (in)
-    ITX_SVD(true, 8);  // at most 68 pairs fit
-  else if (P * 64 <= ST)
-    ITX_SVD(false, 64);
-  else if (P * 16 <= ST)
-    ITX_SVD(false, 16);
-  else if (P * 4 <= ST)
-    ITX_SVD(false, 4);
-  else
-    ITX_SVD(false, 1);
+#define ITX_SVD(L, G) gesvd_run<ST, L, G>(tk, Abase, Ubase, Sbase, Vbase, Wbase, st, lds, sh_rot)
+  if constexpr (ST == 256) {  // at most 64 rows and columns, in LDS
+    if (P * 64 <= ST)
+      ITX_SVD(true, 64);
+    else if (P * 32 <= ST)
+      ITX_SVD(true, 32);
+    else if (P * 16 <= ST)
+      ITX_SVD(true, 16);
+    else
+      ITX_SVD(true, 8);
+  } else {
+    const bool in = svd_lds(tk.m, tk.n) <= lds_bytes;
+    if (in && P * 64 <= ST)
+      ITX_SVD(true, 64);
+    else if (in && P * 32 <= ST)
+      ITX_SVD(true, 32);
+    else if (in)  // at most 51 pairs fit
+      ITX_SVD(true, 16);
+    else if (P * 64 <= ST)
+      ITX_SVD(false, 64);
+    else if (P * 16 <= ST)
+      ITX_SVD(false, 16);
+    else if (P * 4 <= ST)
+      ITX_SVD(false, 4);
+    else
+      ITX_SVD(false, 1);
+  }
 #undef ITX_SVD
 }
 
@@ -294,6 +304,16 @@ extern "C" int itx_gesvd_batched(itx_ctx *ctx, int nmat, const int32_t *m, const
     t.x_off = wsize;
     wsize += C * R + R * R + 2 * R;
   }
+  // A CU holds one workgroup of 1024 threads (83 registers) and five of 256:
+  // more small matrices than CUs take 256.  30 x 30 x 600 1.19 to 0.36 ms (four
+  // waves over the workspace took 0.85), 8 x 8 x 4000 0.77 to 0.45, 64 x 64 x
+  // 300 1.86 to 1.44; above 64 rows or columns it loses (80 x 80 x 512 2.9 to 5.6).
+  auto is_large = [](const itx::SvdTask &t) { return std::max(t.m, t.n) > 64; };
+  int nlarge = int(std::count_if(tasks.begin(), tasks.end(), is_large));
+  if (nmat - nlarge > ctx->num_cus)
+    std::stable_partition(tasks.begin(), tasks.end(), is_large);
+  else
+    nlarge = nmat;
   const size_t tbytes = sizeof(itx::SvdTask) * size_t(nmat), sbytes = sizeof(int) * size_t(nmat);
   const size_t woff = (tbytes + sbytes + 255) & ~size_t(255);
   void *ws = nullptr;
@@ -306,15 +326,19 @@ extern "C" int itx_gesvd_batched(itx_ctx *ctx, int nmat, const int32_t *m, const
     return rc;
   }
   int *dst = reinterpret_cast<int *>(wsb + tbytes);
-  // LDS for the largest matrix that fits
-  size_t lds = 0;
-  for (int b = 0; b < nmat; ++b) {
-    const size_t need = itx::svd_lds(m[b], n[b]);
-    if (need <= itx::SVD_LDS) lds = std::max(lds, need);
+  // large matrices first, 1024 threads each, then the small ones
+  for (int part = 0; part < 2; ++part) {
+    const int first = part ? nlarge : 0, count = part ? nmat - nlarge : nlarge;
+    if (!count) continue;
+    size_t lds = 0;  // for the largest matrix that fits
+    for (int b = first; b < first + count; ++b) {
+      const size_t need = itx::svd_lds(tasks[size_t(b)].m, tasks[size_t(b)].n);
+      if (need <= itx::SVD_LDS) lds = std::max(lds, need);
+    }
+    hipLaunchKernelGGL(part ? itx::k_gesvd<256> : itx::k_gesvd<1024>, dim3(unsigned(count)), dim3(part ? 256 : 1024), lds,
+                       ctx->stream, reinterpret_cast<const itx::SvdTask *>(wsb) + first, A, U, S, V,
+                       reinterpret_cast<double *>(wsb + woff), dst + first, unsigned(lds));
   }
-  hipLaunchKernelGGL(itx::k_gesvd, dim3(unsigned(nmat)), dim3(itx::ST), lds, ctx->stream,
-                     reinterpret_cast<const itx::SvdTask *>(wsb), A, U, S, V, reinterpret_cast<double *>(wsb + woff),
-                     dst, unsigned(lds));
   hipError_t e = hipGetLastError();
   std::vector<int> st(static_cast<size_t>(nmat), 0);
   if (e == hipSuccess) e = hipMemcpyAsync(st.data(), dst, sbytes, hipMemcpyDeviceToHost, ctx->stream);
