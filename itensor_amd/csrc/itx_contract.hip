@@ -1338,22 +1338,28 @@ __global__ __launch_bounds__(64 * GM * GN) void k_gemm3(const double *__restrict
 // from memory (16 rows x 4 k: with A contiguous along k in runs of 4, or
 // along m, a load instruction covers whole 128-byte lines) and the D^T tile
 // stores 16 consecutive m per column, the four row groups of a column back
-// to back.  No LDS and no barrier; 4 x SK_KS independent loads of A per lane
-// are in flight, three waves per SIMD.
-// ONE: every unit has one task with K <= 4 SK_KS, so the k offsets and B's
-// fragments are straight-line code (with the task and k loops around them
-// the registers allow two waves per SIMD: 104 against 84 us at chi = 1024).
+// to back.  No LDS and no barrier; 4 x S independent loads of A per lane are
+// in flight, S = 1, 3 or 5 (SK_KS) slots of 4 k by what is left of a task: with
+// five throughout, 500000 x 17 took 26 us for K = 1 (now 17.5) and 26 for K = 4
+// (now 22), and ten blocks of some 10000 x 16 with three tasks of K <= 2 24 us
+// (now 11).
+// One task per unit with K <= 4 KS is straight-line code, the k offsets and
+// B's fragments outside any loop (with the task and k loops around them the
+// registers allowed two waves per SIMD when this was first measured: 104
+// against 84 us at chi = 1024).
 // K = N = 20 (the dense Heisenberg MPO pair), chi = 32, 255, 768, 1024: 6,
-// 7, 32 and 84 us; one thread per row with B in LDS, the form before this
-// one, was bound by its K x N LDS reads and column tests: 22, 26, 84 and
-// 115 us.  Stores past the caches make this kernel faster at chi = 1024
-// (54 us) and the next stage, which reads C back, slower by more (the chain
-// 1514 against 1495 us).
+// 7, 32 and 75 us (84 before units of one block went by eighths to the XCDs);
+// one thread per row with B in LDS, the form before this one, was bound by its
+// K x N LDS reads and column tests: 22, 26, 84 and 115 us.  Stores past the
+// caches make this kernel faster at chi = 1024 (54 us) and the next stage,
+// which reads C back, slower by more (the chain 1514 against 1495 us).
 constexpr int SK_ROWS = 256, SK_N = 32, SK_K = 64;
-constexpr int SK_KS = 5;  // k slots (of 4) loaded together: K = 20 in one chunk
+constexpr int SK_KS = 5;  // most k slots (of 4) loaded together: K = 20 in one chunk
 constexpr int SK_G = 4;   // 16-row groups of a wave
 
-template <int NB, bool ONE>  // NB 16-column groups: 1 (N <= 16) or 2
+// NB 16-column groups: 1 (N <= 16) or 2; KS: one task per unit, K <= 4 KS (0:
+// any)
+template <int NB, int KS>
 __global__ __launch_bounds__(SK_ROWS, 3) void k_skinny(const double *__restrict__ A, const double *__restrict__ B,
                                                        double *__restrict__ C, const GemmTask *__restrict__ tasks,
                                                        const WorkUnit *__restrict__ units, int nunits,
@@ -1374,13 +1380,14 @@ __global__ __launch_bounds__(SK_ROWS, 3) void k_skinny(const double *__restrict_
     for (int i = 0; i < NB; ++i)
 #pragma unroll
       for (int g = 0; g < SK_G; ++g) acc[i][g] = v4{0, 0, 0, 0};
-    // 4 SK_KS k of one task: loads from clamped positions, zeroed where k
+    // 4 S k of one task: loads from clamped positions, zeroed where k
     // or the column is past the end, so no branch separates them
-    auto chunk = [&](const GemmTask &tk, int k0) {
-      double a[SK_KS][SK_G], b[SK_KS][NB];
-      int64_t ka[SK_KS];
+    auto chunk = [&](const GemmTask &tk, int k0, auto slots) __attribute__((always_inline)) {
+      constexpr int S = decltype(slots)::value;
+      double a[S][SK_G], b[S][NB];
+      int64_t ka[S];
 #pragma unroll
-      for (int s = 0; s < SK_KS; ++s) {
+      for (int s = 0; s < S; ++s) {
         const int k = k0 + 4 * s + q4;
         const bool kv = k < tk.K;
         ka[s] = tab[tk.tAK + (kv ? k : 0)];
@@ -1396,24 +1403,29 @@ __global__ __launch_bounds__(SK_ROWS, 3) void k_skinny(const double *__restrict_
       for (int g = 0; g < SK_G; ++g) {
         const double *Ar = A + tk.a_off + tab[tk.tAM + mr[g]];
 #pragma unroll
-        for (int s = 0; s < SK_KS; ++s) {
+        for (int s = 0; s < S; ++s) {
           const double x = Ar[ka[s]];
           a[s][g] = k0 + 4 * s + q4 < tk.K ? x : 0.0;
         }
       }
 #pragma unroll
-      for (int s = 0; s < SK_KS; ++s)
+      for (int s = 0; s < S; ++s)
 #pragma unroll
         for (int i = 0; i < NB; ++i)
 #pragma unroll
           for (int g = 0; g < SK_G; ++g) acc[i][g] = MF<double>::mma(b[s][i], a[s][g], acc[i][g]);
     };
-    if constexpr (ONE) {
-      if (t0.K > 0) chunk(t0, 0);
+    if constexpr (KS > 0) {
+      if (t0.K > 0) chunk(t0, 0, std::integral_constant<int, KS>{});
     } else {
       for (int t = wu.tbeg; t < wu.tend; ++t) {
         const GemmTask tk = tasks[t];
-        for (int k0 = 0; k0 < tk.K; k0 += 4 * SK_KS) chunk(tk, k0);
+        int k0 = 0;
+        for (; tk.K - k0 > 12; k0 += 4 * SK_KS) chunk(tk, k0, std::integral_constant<int, SK_KS>{});
+        if (tk.K - k0 > 4)
+          chunk(tk, k0, std::integral_constant<int, 3>{});
+        else if (tk.K > k0)
+          chunk(tk, k0, std::integral_constant<int, 1>{});
       }
     }
     int64_t cm[SK_G];
@@ -2309,8 +2321,16 @@ const void *gemm_fn_tile(int tile, bool akc, bool bkc, bool vec) {
 struct Skinny {
   int maxn = SK_N;    // largest N of the tasks
   bool tiny = false;  // every task has K <= 8 and N <= 8
-  bool one = false;   // one task per C block, K <= 4 SK_KS
+  int slots = 0;      // of 4 k, one task per C block (0: several, or K > 4 SK_KS)
 };
+
+template <int NB>
+const void *skinny_fn(int slots) {
+  return slots == 0   ? reinterpret_cast<const void *>(&k_skinny<NB, 0>)
+         : slots == 1 ? reinterpret_cast<const void *>(&k_skinny<NB, 1>)
+         : slots <= 3 ? reinterpret_cast<const void *>(&k_skinny<NB, 3>)
+                      : reinterpret_cast<const void *>(&k_skinny<NB, SK_KS>);
+}
 
 // Entry point and workgroup size of a plan's kernel.
 const void *kernel_of(int tile, int prec, bool akc, bool bkc, int *block, int vec = 0, bool split = false,
@@ -2318,11 +2338,7 @@ const void *kernel_of(int tile, int prec, bool akc, bool bkc, int *block, int ve
   if (tile == kSkinny) {  // HBM-bound: FP64 arithmetic in every form
     *block = SK_ROWS;
     if (sk.tiny) return reinterpret_cast<const void *>(&k_skinny_q);
-    if (sk.maxn <= 16)
-      return sk.one ? reinterpret_cast<const void *>(&k_skinny<1, true>)
-                    : reinterpret_cast<const void *>(&k_skinny<1, false>);
-    return sk.one ? reinterpret_cast<const void *>(&k_skinny<2, true>)
-                  : reinterpret_cast<const void *>(&k_skinny<2, false>);
+    return sk.maxn <= 16 ? skinny_fn<1>(sk.slots) : skinny_fn<2>(sk.slots);
   }
   if (tile == kSmall) {
     *block = SM_T;
@@ -2936,7 +2952,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     const int occ = best == kSkinny && tinyq ? kSkinnyQOcc : tile_occupancy(best, prec, akc, bkc);
     p->grid = int(std::min<int64_t>(int64_t(units.size()), int64_t(cus) * occ));
     p->vec = (akc && bkc) ? vecbits : 0;
-    const Skinny sk{maxN, tinyq, st.size() == groups.size() && maxK <= 4 * SK_KS};
+    const Skinny sk{maxN, tinyq, st.size() == groups.size() && maxK <= 4 * SK_KS ? (maxK + 3) / 4 : 0};
     // Small blocks of the reduced forms with tasks of one chunk: lanes along the
     // rows also where k is contiguous.  Along k most would idle (23 blocks of up
     // to 60 x 15, K <= 8, BF16x3 6.2 and 9.3 us; K <= 40 14.2 and 18.8; K <= 64

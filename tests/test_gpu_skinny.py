@@ -45,3 +45,25 @@ def test_skinny_tasks_of_one_block(ctx, dev, dims):
     ref = sum(x.T @ y for x, y in zip(A, B))
     K = sum(k for _, _, k in dims)
     assert np.all(np.abs(dev.get(c, (M, N)) - ref) <= (K + 3) * EPS * sum(np.abs(x.T) @ np.abs(y) for x, y in zip(A, B)))
+
+
+@pytest.mark.parametrize("N", [9, 16, 17, 32])
+@pytest.mark.parametrize("Ks", [[1], [4], [5], [12], [13], [20], [21], [24], [25], [32], [33], [1, 4], [3, 5, 12], [13, 2], [64, 1]])
+def test_skinny_slots(ctx, dev, Ks, N):
+    """Remainders of k in one, three and five slots of four, one task and several."""
+    rng = np.random.default_rng(sum(Ks) + N)
+    M = 321
+    A, B = [rng.standard_normal((k, M)) for k in Ks], [rng.standard_normal((k, N)) for k in Ks]
+    offs, blkA, blkB, a, b = [], [], [], 0, 0
+    for k in Ks:
+        offs += [a, b, 0]
+        blkA += [k, M]
+        blkB += [k, N]
+        a, b = a + k * M, b + k * N
+    p = ctx.plan_qn((-1, 1), (-1, 2), (1, 2), offs, blkA, blkB)
+    assert p.info["tile"] == 5
+    Ad, Bd, c = dev.put(np.concatenate([x.ravel(order="F") for x in A])), dev.put(np.concatenate([x.ravel(order="F") for x in B])), dev.empty(M * N)
+    p.execute(Ad.data_ptr(), Bd.data_ptr(), c.data_ptr())
+    ref = sum(x.T @ y for x, y in zip(A, B))
+    bound = (sum(Ks) + 3) * EPS * sum(np.abs(x.T) @ np.abs(y) for x, y in zip(A, B))
+    assert np.all(np.abs(dev.get(c, (M, N)) - ref) <= bound)
