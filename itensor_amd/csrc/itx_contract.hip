@@ -2855,7 +2855,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     }
     if (split               ? best == kPipe64 && units.size() > 2 * kXcds
         : groups.size() > 1 ? units.size() > size_t(cus)
-                            : best != kSkinny && units.size() > size_t(cus)) {
+                            : best != kSkinny && units.size() > 2 * kXcds) {
       // Workgroup b runs on XCD b % 8 and takes units b, b + grid, ...: each
       // XCD gets a list of units that share operands in its L2.  Equal units
       // (one block, or the pieces of a product split over k): eighths of the list.  Several
@@ -2865,10 +2865,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
       // read the same blocks of A (B is a few numbers; an MPO stage reads
       // each block of A for every channel it feeds).  chi = 1024 block-sparse
       // chain, against the blocks from the heaviest down: 29.5 to 23.6, 23.4
-      // to 19.3 and 38.6 to 28.4 us; up to a unit per CU it gains nothing for
-      // several blocks, and for one it lost more often than it gained (127 x 262
-      // x 2556 in BF16x3 42 and 53 us, 399 x 572 x 697 in FP64 22.7 and 25.3; 234
-      // x 96 x 3379 in BF16x3 92 and 81).  The
+      // to 19.3 and 38.6 to 28.4 us; up to a unit per CU it gains nothing.  The
       // pieces of split small blocks stay in their order, a tile's k ranges
       // round robin: tiles then meet the same k on an XCD (90 x 90 x 60000 in
       // FP32 150 us as eighths, 125 in order).
