@@ -2873,9 +2873,12 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
       std::vector<WorkUnit> su;
       su.reserve(n);
       if (split || groups.size() == 1) {
-        const size_t chunk = (n + kXcds - 1) / kXcds;
-        for (size_t j = 0; j < chunk; ++j)
-          for (size_t i = j; i < n; i += chunk) su.push_back(units[i]);
+        // the first n % 8 XCDs have one more: every round of eight is whole
+        const size_t len = n / kXcds, more = n % kXcds;
+        for (size_t i = 0; i < n; ++i) {
+          const size_t x = i % kXcds;
+          su.push_back(units[x * len + std::min(x, more) + i / kXcds]);
+        }
       } else {
         std::array<std::vector<WorkUnit>, kXcds> lists;
         std::vector<int> head(vt.size());  // a block's first task -> its place in `open`
