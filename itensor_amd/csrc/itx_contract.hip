@@ -2853,9 +2853,9 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
         units.swap(su);
       }
     }
-    if (split               ? best == kPipe64 && units.size() > 2 * kXcds
-        : groups.size() > 1 ? units.size() > size_t(cus)
-                            : best != kSkinny && units.size() > 2 * kXcds) {
+    if (groups.size() > 1 && !split ? units.size() > size_t(cus)
+                                    : best != kSkinny && units.size() > 2 * kXcds &&
+                                          (groups.size() > 1 || !split || best == kPipe64)) {
       // Workgroup b runs on XCD b % 8 and takes units b, b + grid, ...: each
       // XCD gets a list of units that share operands in its L2.  Equal units
       // (one block, or the pieces of a product split over k): eighths of the list.  Several
@@ -2866,9 +2866,11 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
       // each block of A for every channel it feeds).  chi = 1024 block-sparse
       // chain, against the blocks from the heaviest down: 29.5 to 23.6, 23.4
       // to 19.3 and 38.6 to 28.4 us; up to a unit per CU it gains nothing.  The
-      // pieces of split small blocks stay in their order, a tile's k ranges
-      // round robin: tiles then meet the same k on an XCD (90 x 90 x 60000 in
-      // FP32 150 us as eighths, 125 in order).
+      // pieces of one split small block stay in their order, a tile's k ranges
+      // round robin: its tiles then meet the same k on an XCD (90 x 90 x 60000 in
+      // FP32 150 us as eighths, 125 in order); those of several blocks, whose
+      // tiles share less, do not (chain at chi = 640, last stage in BF16x3 25 us as
+      // eighths, 32 in order).
       const size_t n = units.size();
       std::vector<WorkUnit> su;
       su.reserve(n);
