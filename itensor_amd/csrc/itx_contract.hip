@@ -2960,11 +2960,11 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     const Skinny sk{maxN, tinyq, st.size() == groups.size() && maxK <= 4 * SK_KS ? (maxK + 3) / 4 : 0};
     // Small blocks of the reduced forms with short tasks: lanes along the rows
     // also where k is contiguous.  Along k most would idle (23 blocks of up to 60
-    // x 15, K <= 8, BF16x3 6.2 and 9.3 us; K <= 40 14.2 and 18.8).  At K <= 64
-    // neither leads (15.7 and 16.9; 36 blocks of up to 66 x 66 16.7 and 14.4);
-    // with longer k the rows' lines lie apart (90 x 90 x 60000 up to 1.4 times
-    // as long).
-    const bool rows_only = best == kSmall && prec != ITX_PREC_F64 && maxK <= 48;
+    // x 15, K <= 8, BF16x3 6.2 and 9.3 us; block-sparse chain at chi = 110, K <=
+    // 8, BF16x3 33.6 and 34.5).  Above 24 k it depends on the number of rows: the
+    // chain at chi = 400 (K <= 28) 48.4 and 49.7 us, 52 blocks of up to 42 x 42 x
+    // 42 13.8 and 12.5.
+    const bool rows_only = best == kSmall && prec != ITX_PREC_F64 && maxK <= 24;
     p->fn = kernel_of(best, prec, akc && !rows_only, bkc && !rows_only, &p->block, p->vec, false, sk);
     p->fn_scalar = kernel_of(best, prec, akc && !rows_only, bkc && !rows_only, &p->block, 0, false, sk);
     p->nred = int(red.size());

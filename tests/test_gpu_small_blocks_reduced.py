@@ -1,4 +1,4 @@
-"""The FP32 and BF16x3 small-block kernels either side of the k (64) up to
+"""The FP32 and BF16x3 small-block kernels either side of the k (24) up to
 which lanes walk the rows in every layout: the layout does not enter the sums."""
 import numpy as np
 import pytest
@@ -39,9 +39,9 @@ def _run(ctx, dev, shapes, aorder, border, prec):
 
 @pytest.mark.parametrize("prec", ["f32", "bf16x3"])
 @pytest.mark.parametrize("shapes", [
-    [((1, 1), [1])], [((65, 33), [8, 1, 3])], [((63, 31), [64, 5])], [((64, 32), [65, 2])], [((60, 15), [1, 8])] * 23,
+    [((1, 1), [1])], [((65, 33), [8, 1, 3])], [((63, 31), [24, 5])], [((61, 30), [25, 24])], [((64, 32), [65, 2])], [((60, 15), [1, 8])] * 23,
     [((40, 37), [64] * 7), ((5, 9), [3])], [((90, 80), [64] * 40)] * 2, [((90, 90), [3000])],  # split over units
-], ids=range(8))
+], ids=range(9))
 def test_small_blocks_reduced(ctx, dev, shapes, prec):
     got = [_run(ctx, dev, shapes, a, b, prec) for a in ("km", "mk") for b in ("kn", "nk")]
     assert all(np.array_equal(got[0], x) for x in got[1:])
