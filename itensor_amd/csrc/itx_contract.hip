@@ -2455,6 +2455,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
   // along m); likewise B.  Decided on the first non-empty task.
   bool first_kc = false;  // of the first task
   double akc_work = 0, bkc_work = 0;  // multiply-adds of tasks with k-contiguous operands less those of the others
+  double run_work = 0;                // those of tasks with no operand in short runs, less those of the others
 
   double flops = 0;
   // Everything a task needs besides its offsets follows from the block
@@ -2467,6 +2468,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     int64_t tAM, tCM, tBN, tCN, tAK, tBK;
     int64_t am, cm, bn, cn, ak, bk;
     bool akc, bkc, empty;
+    bool arow, brow;  // read along the rows (columns of B), in runs of 16 or all
     int vec;  // bit 0: k runs of 2 usable by both operands, bit 1: runs of 4 (bit 2: below)
   };
   std::vector<DimInfo> infos;
@@ -2566,6 +2568,12 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
         if (c[i].s1 % al) return false;
       return true;
     };
+    auto row_runs = [&](const Digits &d, int64_t n) {
+      Digit c[ITX_MAX_RANK];
+      return column(d, true, c) > 0 && c[0].s1 == 1 && c[0].dim >= std::min<int64_t>(16, n);
+    };
+    fi.arow = !fi.akc && row_runs(dm, M);
+    fi.brow = !fi.bkc && row_runs(dn, N);
     if (fi.akc && fi.bkc) {
       if (aligned(dm, true, 2) && aligned(dn, true, 2)) {
         if (runs(dk, true, K, 2, 2) && runs(dk, false, K, 2, 2)) fi.vec |= 1;
@@ -2616,6 +2624,7 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     const double work = fi.K > 1 ? double(fi.M) * double(fi.N) * double(fi.K) : 0.0;
     akc_work += fi.akc ? work : -work;
     bkc_work += fi.bkc ? work : -work;
+    run_work += (fi.akc || fi.arow) && (fi.bkc || fi.brow) ? work : -work;
     vecbits &= fi.vec;
     if (offs[3 * size_t(t)] % 2 || offs[3 * size_t(t) + 1] % 2) vecbits = 0;
     if (offs[3 * size_t(t)] % 4 || offs[3 * size_t(t) + 1] % 4) vecbits &= ~4;
@@ -3142,10 +3151,14 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     // The pipelined tiles (k_pipe) and the 32 x 32 tile.  A unit costs its k
     // stages of 16 and a few more for every task and for itself; `alone` is
     // the time of a stage (us) of a workgroup that has its CU to itself,
-    // `shared` the CU's time per stage when it has several; `any` for operands
-    // not contiguous along k.  Fitted to the stages of the dense chain, k-
-    // contiguous at chi = 48 to 1024, others to its MPO stage at d = 4, k = 18,
-    // where the operator is read in single strided elements.
+    // `shared` the CU's time per stage when it has several, by layout: both
+    // operands contiguous along k; each along k or in runs of 16 rows; others.
+    // Fitted to the stages of the dense chain at chi = 48 to 1024 and to products
+    // of 600 to 4000 rows and columns with K = 8 to 1151; the last layout to its
+    // MPO stage at d = 4, k = 18, where the operator is read in single strided
+    // elements.  One class for the last two took 128 x 128 where 64 x 64 is
+    // better: 3362 x 1159 x 32 along rows 21.5 and 12.7 us in FP32, 20 and 13 in
+    // BF16x3, 1500 x 1500 x 200 37 and 29 in FP64.
     // FP64, us as 32 x 32, 64 x 64, 128 x 128: last stage, chi = 255 43, 28
     // (split eight ways), 168; chi = 512 152, 96, 293; chi = 1024 1040, 660,
     // 593; MPO stage, chi = 32 21.6, 18.4, 50.6; chi = 330 1274, 676, 574.
@@ -3155,20 +3168,25 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
     // 26, 53 (43); chi = 512 87, 53, 107 (85); chi = 1024 600, 315, 210 (343).
     struct Model {
       int tile, bm, bn;
-      double alone, shared, any_alone, any_shared, per_task, per_unit;
+      double per_task, per_unit;
+      double alone[3], shared[3];  // by layout: along k, along k or rows, other
     };
     const bool vector = prec == ITX_PREC_BF16X3 ? vecbits & 2 : vecbits & 1;
     const double v1 = vector ? 1.0 : prec == ITX_PREC_F64 ? 1.1 : prec == ITX_PREC_F32 ? 1.2 : 1.6;  // single loads
-    const Model f64[] = {{4, 32, 32, 0.45, 0.28, 0.50, 0.50, 1, 1},
-                         {kPipe64, 64, 64, 0.63 * v1, 0.50 * v1, 0.70, 0.88, 3, 2},
-                         {kPipe128, 128, 128, 1.87 * v1, 1.87 * v1, 2.65, 2.65, 2, 1}};
-    const Model f32[] = {{4, 32, 32, 0.42, 0.17, 0.50, 0.50, 1, 1},
-                         {kPipe32, 32, 64, 0.28 * v1, 0.21 * v1, 0.75, 0.85, 2, 1},
-                         {kPipe64, 64, 64, 0.43 * v1, 0.33 * v1, 0.62, 0.83, 3, 2},
-                         {kPipe128, 128, 128, 1.13 * v1, 1.13 * v1, 1.80, 2.05, 2, 1}};
-    const Model bf[] = {{4, 32, 32, 0.28 * v1, 0.14 * v1, 0.45, 0.37, 1, 1},
-                        {kPipe64, 64, 64, 0.31 * v1, 0.235 * v1, 0.70, 0.73, 3, 2},
-                        {kPipe128, 128, 128, 0.65 * v1, 0.74 * v1, 1.65, 1.90, 2, 1}};
+    const double w1 = vector ? 1.0 : prec == ITX_PREC_F64 ? 1.2 : prec == ITX_PREC_F32 ? 1.25 : 1.4;  // of 32 x 32
+    const double s4 = maxK > 2048 ? 0.28 : 0.22;  // with long k its operands leave the L2
+    const int lay = akc && bkc ? 0 : run_work > 0 ? 1 : 2;
+    const bool dear = lay < 2;  // a unit's own time: behind the slow stages of the last layout it is short
+    const Model f64[] = {{4, 32, 32, 1, 1, {0.45 * w1, 0.50, 0.50}, {s4 * w1, 0.27, 0.50}},
+                         {kPipe64, 64, 64, 3, dear ? 1.0 : 2.0, {0.56, 0.64, 0.70}, {0.50 * v1, 0.54, 0.88}},
+                         {kPipe128, 128, 128, 2, dear ? 1.5 : 1.0, {1.87 * v1, 2.00, 2.65}, {1.87 * v1, 2.05, 2.65}}};
+    const Model f32[] = {{4, 32, 32, 1, 1, {0.42 * w1, 0.45, 0.50}, {0.18 * w1, 0.24, 0.50}},
+                         {kPipe32, 32, 64, 2, dear ? 3.0 : 1.0, {0.28 * v1, 0.40, 0.75}, {0.21 * v1, 0.27, 0.85}},
+                         {kPipe64, 64, 64, 3, 2, {0.43 * v1, 0.45, 0.62}, {0.33 * v1, 0.37, 0.83}},
+                         {kPipe128, 128, 128, 2, dear ? 3.0 : 1.0, {1.13 * v1, 1.31, 1.80}, {1.13 * v1, 1.40, 2.05}}};
+    const Model bf[] = {{4, 32, 32, 1, dear ? 3.0 : 1.0, {0.28 * w1, 0.42, 0.45}, {0.14 * w1, 0.23, 0.37}},
+                        {kPipe64, 64, 64, 3, dear ? 3.0 : 2.0, {0.31 * v1, 0.49, 0.70}, {0.235 * v1, 0.30, 0.73}},
+                        {kPipe128, 128, 128, 2, dear ? 4.0 : 1.0, {0.65 * v1, 0.95, 1.65}, {0.74 * v1, 1.00, 1.90}}};
     const Model *models = prec == ITX_PREC_F64 ? f64 : prec == ITX_PREC_F32 ? f32 : bf;
     const size_t nm = best == kDgemm ? 0 : prec == ITX_PREC_F32 ? std::size(f32) : std::size(f64);
     if (nm) best = 4;
@@ -3186,11 +3204,9 @@ int build_plan(itx_ctx *ctx, int rA, const int32_t *labA, int rB, const int32_t 
         n += tiles;
         if (groups.size() > 1) costs.insert(costs.end(), size_t(tiles), c);
       }
-      const bool kc = akc && bkc;
-      double tt = most * (kc ? md->alone : md->any_alone);
+      double tt = most * md->alone[lay];
       if (n > cus)
-        tt = std::max(tt, (costs.empty() ? lpt_makespan(n, most, cus) : lpt_makespan(costs, cus)) *
-                              (kc ? md->shared : md->any_shared));
+        tt = std::max(tt, (costs.empty() ? lpt_makespan(n, most, cus) : lpt_makespan(costs, cus)) * md->shared[lay]);
       if (ns > 1)  // the partial tiles and the second launch
         tt += 5.0 + double(ns) * groups[0].M * groups[0].N * 16.0 / 4e6;
       if (tt < best_t) {
