@@ -178,10 +178,7 @@ __global__ __launch_bounds__(64 * GM * GN) void k_gemm(const double *__restrict_
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave % GM, wn = wave / GM;
 
-  // Units are spread so that each XCD (blocks b with equal b % 8 land on
-  // the same XCD) walks a contiguous chunk of the unit list: neighbouring
-  // tiles share A rows / B columns, which then stay in that XCD's L2.
-
+  // the planner has dealt the list to the XCDs (blocks b with equal b % 8)
   for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
     const WorkUnit wu = units[u];
     v4 acc[FN][FM];
@@ -396,8 +393,6 @@ __global__ __launch_bounds__(DG_NT) void k_dgemm(const double *__restrict__ A, c
   __shared__ __align__(16) T Bs[2][128 * P];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
-
-  // XCD-contiguous unit chunks (as in k_gemm)
 
   for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
     const WorkUnit wu = units[u];
@@ -1568,9 +1563,9 @@ __global__ __launch_bounds__(SK_ROWS) void k_skinny_q(const double *__restrict__
 // one C block.  FP64 form, on the matrix cores straight from memory: a wave
 // loads the fragments of 32 x 32 outputs for 16 k at once (rows over 16
 // lanes, 4 k over the lane quarters) while it multiplies the previous 16, and
-// the four waves share a unit's k: with up to 32 rows each takes every fourth
-// task (or, with fewer than four tasks, every fourth 16 k of each), above
-// that two waves per half of the rows.  The waves' sums meet in LDS once.
+// the eight waves share a unit's k: with up to 32 rows each takes every eighth
+// task (or, with fewer than eight tasks, every eighth 16 k of each), above
+// that four waves per half of the rows.  The waves' sums meet in LDS once.
 // Staging both tiles in LDS for VALU arithmetic, the form before this one,
 // made two barriers and three such trips per 64 k and task; the last stage of
 // the dense chi = 32 chain (one 128 x 32 block, K = 160) took 31 us with its

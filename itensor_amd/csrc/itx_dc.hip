@@ -54,8 +54,8 @@ struct SecSums {
 };
 // A step interpolates the sums below and above by one pole each, at d[j] and
 // d[j+1]; after the first one the nearer pole keeps its own weight (the
-// fixed-weight form), which converges in one step less: 4 evaluations on
-// average.  A step below 1e-8 of mu is the last one: the next would be of
+// fixed-weight method: Li, LAPACK Working Note 89 (1993)), which converges in
+// one step less: 4 evaluations on average.  A step below 1e-8 of mu is the last one: the next would be of
 // the order of its square.
 template <class Weight, class Sums>
 __device__ __forceinline__ void secular_root(int j, int k, const double *d, double wsum, Weight weight, Sums sums,

@@ -37,8 +37,8 @@ namespace {
 // then takes another path.
 // What bounds it is the latency of the n - 2 dependent steps: in one
 // workgroup 1.15 us a step at n = 64 and 1.6 at 128 (72 and 203 us in all;
-// the LDS-resident form before this one 174 and 519), across workgroups 2.8
-// us at n = 234, 1.3 of them the trip through memory (0.65 ms; one workgroup
+// the LDS-resident form before this one 174 and 519), across workgroups 2.5
+// us at n = 234, 1.3 of them the trip through memory (0.59 ms; one workgroup
 // over the L2 2.7 ms).  Four columns per wave: with eight, on half the
 // workgroups, the update costs what the trip gains.
 constexpr int TNW = 4;            // waves per workgroup
