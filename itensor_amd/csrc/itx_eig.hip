@@ -64,6 +64,16 @@ __device__ __forceinline__ double bsum(double v, double *red) {
   return s;
 }
 
+__device__ __forceinline__ double bmax(double v, double *red) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  for (int i = 0; i < ET / 64; ++i) v = fmax(v, red[i]);
+  return v;
+}
+
 // Reduction and Q: A in global memory (overwritten by the reflectors), W as
 // scratch for p, Q into the workspace.  One workgroup per matrix: used when a
 // batch holds several matrices that are cheaper side by side than one after
@@ -87,13 +97,36 @@ __global__ __launch_bounds__(ET) void k_syev(const EigTask *__restrict__ tasks, 
     double *col = A + size_t(k) * n + (k + 1);  // x = A[k+1:, k]
     double s = 0;
     for (int i = 1 + tid; i < L; i += ET) s += col[i] * col[i];
-    const double sigma = bsum(s, red);
-    const double x0 = col[0];
-    double tau = 0, alpha = x0;
+    double sigma = bsum(s, red);
+    const double x0 = col[0], s2 = x0 * x0 + sigma;
+    double tau = 0, alpha = x0, x = x0;
+    int ex = 0;
+    // v in units of the column, a power of two, so that neither its squares nor
+    // products with much larger columns leave the range of numbers
+    if (s2 > 1e-280 && s2 < 1e280) {
+      ex = __builtin_amdgcn_frexp_exp(s2) >> 1;
+      sigma = ldexp(sigma, -2 * ex);
+      for (int i = 1 + tid; i < L; i += ET) col[i] = ldexp(col[i], -ex);
+      x = ldexp(x0, -ex);
+    } else if (sigma == sigma) {
+      double m = fabs(x0);
+      for (int i = 1 + tid; i < L; i += ET) m = fmax(m, fabs(col[i]));
+      m = bmax(m, red);
+      if (m > 0 && m <= DBL_MAX) {
+        (void)frexp(m, &ex);
+        s = 0;
+        for (int i = 1 + tid; i < L; i += ET) {
+          col[i] = ldexp(col[i], -ex);
+          s += col[i] * col[i];
+        }
+        sigma = bsum(s, red);
+        x = ldexp(x0, -ex);
+      }
+    }
     if (sigma > 0) {
-      const double mu = sqrt(x0 * x0 + sigma);
-      const double v0 = (x0 <= 0) ? x0 - mu : x0 + mu;
-      alpha = (x0 <= 0) ? mu : -mu;
+      const double mu = sqrt(x * x + sigma);
+      const double v0 = (x <= 0) ? x - mu : x + mu;
+      alpha = ldexp((x <= 0) ? mu : -mu, ex);
       tau = 2.0 / (v0 * v0 + sigma);
       __syncthreads();
       if (tid == 0) col[0] = v0;  // col now holds v

@@ -4,6 +4,8 @@
 // Householder reduction; Golub & Van Loan, "Matrix Computations", 8.3.
 #pragma once
 
+#include <cfloat>
+
 #include "itx_eig.h"
 
 namespace itx {
@@ -110,7 +112,8 @@ __device__ __forceinline__ void tri_run(const TriTask &tk, int g, const double *
     return r;
   };
   // the reflector of column q (rows > q + 1 of c and x0 = c[q + 1]), the same
-  // in every wave
+  // in every wave; v in units of the column, a power of two, so that products
+  // with much larger columns stay numbers
   auto reflect = [&](int q, double x0) __attribute__((always_inline)) {
     double sg = 0.0;
 #pragma unroll
@@ -119,22 +122,48 @@ __device__ __forceinline__ void tri_run(const TriTask &tk, int g, const double *
     sg = wave_total(sg);
     double alpha = x0, v0 = x0;
     tau = 0.0;
-    if (sg > 0.0) {
-      const double s2 = x0 * x0 + sg;
-      // a scalar branch: the slow forms are otherwise computed beside the fast ones
-      if (__builtin_amdgcn_readfirstlane(s2 > 1e-280 && s2 < 1e280)) {
-        const double mu = fast_sqrt(s2);
-        v0 = (x0 <= 0) ? x0 - mu : x0 + mu;
-        alpha = (x0 <= 0) ? mu : -mu;
-        tau = 2.0 * fast_rcp(v0 * v0 + sg);
-      } else {
-        const double mu = sqrt(s2);
-        v0 = (x0 <= 0) ? x0 - mu : x0 + mu;
-        alpha = (x0 <= 0) ? mu : -mu;
-        tau = 2.0 / (v0 * v0 + sg);
+    const double s2 = x0 * x0 + sg;
+    // scalar branches: the slow forms are otherwise computed beside the fast ones
+    if (__builtin_amdgcn_readfirstlane(s2 > 1e-280 && s2 < 1e280)) {
+      if (__builtin_amdgcn_readfirstlane(sg > 0.0)) {
+        const int ex = __builtin_amdgcn_frexp_exp(s2) >> 1;
+        const double x = ldexp(x0, -ex), ss = ldexp(sg, -2 * ex), mu = fast_sqrt(ldexp(s2, -2 * ex));
+        v0 = (x <= 0) ? x - mu : x + mu;
+        alpha = ldexp((x <= 0) ? mu : -mu, ex);
+#pragma unroll
+        for (int a = 0; a < RA; ++a) c[a] = ldexp(c[a], -ex);
+        tau = 2.0 * fast_rcp(v0 * v0 + ss);
       }
     } else if (sg != sg) {
       tau = sg;  // not a number: carried into d and e
+    } else {
+      // The squares leave the range of numbers, as in the last columns of a
+      // matrix whose rank is small or whose rows are graded.
+      double m = fabs(x0);
+#pragma unroll
+      for (int a = 0; a < RA; ++a)
+        if (lane + 64 * a > q + 1) m = fmax(m, fabs(c[a]));
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+      if (m > DBL_MAX) {
+        alpha = (x0 <= 0) ? m : -m;
+      } else if (m > 0.0) {
+        int ex;
+        (void)frexp(m, &ex);
+        sg = 0.0;
+#pragma unroll
+        for (int a = 0; a < RA; ++a) {
+          c[a] = ldexp(c[a], -ex);
+          if (lane + 64 * a > q + 1) sg += c[a] * c[a];
+        }
+        sg = wave_total(sg);
+        if (sg > 0.0) {
+          const double x = ldexp(x0, -ex), mu = sqrt(x * x + sg);
+          v0 = (x <= 0) ? x - mu : x + mu;
+          alpha = ldexp((x <= 0) ? mu : -mu, ex);
+          tau = 2.0 / (v0 * v0 + sg);
+        }
+      }
     }
 #pragma unroll
     for (int a = 0; a < RA; ++a) {

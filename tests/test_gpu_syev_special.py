@@ -3,6 +3,7 @@ in one call with ordinary matrices."""
 import numpy as np
 import pytest
 
+from itensor_amd.itx import ItxError
 from test_gpu_syev_dc import _check, _matrix, _solve
 
 pytestmark = pytest.mark.gpu
@@ -59,3 +60,52 @@ def test_syev_largest_numbers(ctx, dev, n):
     if n > 1:
         (w, U), = _solve(ctx, dev, [np.array([[1.0, 0.25], [0.25, 1.0]]) * 2.0**1023])
         assert np.max(np.abs(w * 2.0**-1023 - [1.25, 0.75])) <= 64 * np.finfo(float).eps
+
+
+def _rank_one(n):
+    return np.ones((n, n))
+
+
+def _graded(n):
+    rng = np.random.default_rng(n)
+    d = 10.0 ** (-0.4 * np.arange(n))
+    Y = rng.standard_normal((n, n))
+    return d[:, None] * (Y + Y.T) * d
+
+
+def _graded_up(n):
+    return _graded(n)[::-1, ::-1].copy()
+
+
+@pytest.mark.parametrize("wait", [None, "0"])
+@pytest.mark.parametrize("scale", [1.0, 1e-140, 1e140, 1e-250, 1e250])
+@pytest.mark.parametrize("make", [_rank_one, _graded, _graded_up, lambda n: _matrix("random", n, np.random.default_rng(n)),
+                                  lambda n: np.eye(n) + 1e-15 * _matrix("random", n, np.random.default_rng(n))],
+                         ids=["rank-one", "graded", "graded-up", "random", "identity"])
+def test_syev_squares_out_of_range(ctx, dev, monkeypatch, make, scale, wait):
+    """Columns whose squares are no numbers: what is left of a column when the
+    rank or the grading has used it up, and whole matrices of such a scale."""
+    if wait is not None:
+        monkeypatch.setenv("ITX_EIG_WAIT", wait)
+    mats = [make(n) * scale for n in (2, 3, 24, 64, 65, 128, 153, 200, 256, 300, 400)]
+    for X, (w, U) in zip(mats, _solve(ctx, dev, mats)):
+        _check(X / scale, w / scale, U)
+
+
+@pytest.mark.parametrize("n", [100, 129, 200, 300])
+def test_syev_infinite_coupling(ctx, dev, n):
+    """No decomposition: an error or the diagonal, and the context keeps working.
+    (An infinite coupling of a merge once gave an eigenvalue that is not a
+    number, whose place in the order was never written.)"""
+    d, e = np.linspace(1.0, 2.0, n), np.zeros(n - 1)
+    e[n // 2 - 1] = np.inf
+    X = np.diag(d) + np.diag(e, 1) + np.diag(e, -1)
+    try:
+        (w, U), = _solve(ctx, dev, [X])
+        assert np.array_equal(w, d[::-1])
+    except ItxError as err:
+        assert "(5)" in str(err)
+    rng = np.random.default_rng(n)
+    Y = _matrix("random", n, rng)
+    (w, U), = _solve(ctx, dev, [Y])
+    _check(Y, w, U)
