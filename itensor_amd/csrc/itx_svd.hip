@@ -155,8 +155,19 @@ __device__ __forceinline__ void gesvd_run(const SvdTask &tk, const double *__res
           sn = cs * t;
         } else {
           if (ga == 0.0 || al == 0.0 || be == 0.0 || fabs(ga) <= tol * sqrt(al) * sqrt(be)) continue;
-          const double zeta = (be - al) / (2.0 * ga);
-          const double t = copysign(1.0, zeta) / (fabs(zeta) + sqrt(fma(zeta, zeta, 1.0)));
+          // What is left of a column that depends on the others shrinks from sweep
+          // to sweep (where rows repeat, by 1e6), and once its square is denormal
+          // no rotation makes it orthogonal to working precision.  Then, or past
+          // the sweeps that independent columns take, it is zero beside a column
+          // more than 1e30 times as long.
+          if ((low < 1e-290 && top > 1e-230) || (sweep >= 20 && low < 1e-60 * top)) {
+            double *x = al < be ? xa : xb;
+            for (int c = g; c < C; c += G) x[c] = 0.0;
+            continue;
+          }
+          const double zeta = (be - al) / (2.0 * ga), z = fabs(zeta);
+          const double t = copysign(1.0, zeta) / (z + (z < 1e150 ? sqrt(fma(z, z, 1.0)) : z));
+          if (t == 0.0) continue;  // past the smallest number
           cs = 1.0 / sqrt(fma(t, t, 1.0));
           sn = cs * t;
         }
